@@ -156,14 +156,11 @@ class _Mlp(nn.Module):
         return self.bn2(self.fc2(torch.relu(self.bn1(self.fc1(x)))))
 
 
-def _compact(model, gen):
-    """Swap the layers of `model` for quantized ones, give them trained ternary weights and pack them."""
-    ctrl = tmq_amd.QuantizationControl(post_scale=False)
-    tmq_amd.quantize_model(model, ctrl)
-    model.to(DEVICE).eval()
+def _train(model, gen, layers=(nn.Linear, nn.Conv2d, nn.ConvTranspose2d)):
+    """Give the `layers` of `model` trained ternary weights and its norms the statistics that go with them."""
     with torch.no_grad():
         for m in model.modules():
-            if isinstance(m, tmq_amd.TMQLayer):
+            if isinstance(m, layers):
                 m.weight.data = _ternary(m.weight.shape, gen)
                 if m.bias is not None:
                     m.bias.data.normal_(generator=gen)
@@ -173,10 +170,19 @@ def _compact(model, gen):
                 m.running_var.uniform_(0.8, 1.25, generator=gen)
                 m.weight.uniform_(0.75, 1.25, generator=gen)
                 m.bias.normal_(0, 0.1, generator=gen)
-        convs = [m for m in model.modules() if isinstance(m, tmq_amd.Conv2d)]
+        convs = [m for m in model.modules() if isinstance(m, layers) and m.weight.dim() == 4]
         norms = [m for m in model.modules() if isinstance(m, nn.BatchNorm2d)]
         for conv, bn in zip(convs, norms):
             bn.running_var.mul_(0.5 * conv.weight[0].numel())
+    return model
+
+
+def _compact(model, gen):
+    """Swap the layers of `model` for quantized ones, give them trained ternary weights and pack them."""
+    ctrl = tmq_amd.QuantizationControl(post_scale=False)
+    tmq_amd.quantize_model(model, ctrl)
+    model.to(DEVICE).eval()
+    _train(model, gen, tmq_amd.TMQLayer)
     tmq_amd.compressed_state_dict(model)
     return model
 
@@ -197,6 +203,13 @@ class _Layers(nn.Module):
         self.layers = nn.ModuleList(made)
 
 
+def _conv_layer(case):
+    C, N, k, s = case["C"], case["N"], case["k"], case["s"]
+    if case["form"] == "transposed":
+        return nn.ConvTranspose2d(C, N, k, s, (k - s) // 2, bias=case["bias"])
+    return nn.Conv2d(C, N, k, s, k // 2, groups=C if case["form"] == "depthwise" else 1, bias=case["bias"])
+
+
 def prepare(case, seed):
     gen = torch.Generator(device=DEVICE).manual_seed(seed)
     kind, st = case["kind"], {"case": case}
@@ -205,13 +218,8 @@ def prepare(case, seed):
         st["layer"] = model[0]
         st["x"] = torch.randn(case["M"], case["K"], generator=gen, device=DEVICE).to(_DTYPE[case["dtype"]])
     elif kind == "conv":
-        C, N, k, s = case["C"], case["N"], case["k"], case["s"]
-        if case["form"] == "transposed":
-            layer = nn.ConvTranspose2d(C, N, k, s, (k - s) // 2, bias=case["bias"])
-        else:
-            layer = nn.Conv2d(C, N, k, s, k // 2, groups=C if case["form"] == "depthwise" else 1, bias=case["bias"])
-        st["layer"] = _compact(nn.Sequential(layer), gen)[0]
-        x = torch.randn(case["B"], C, case["H"], case["W"], generator=gen, device=DEVICE)
+        st["layer"] = _compact(nn.Sequential(_conv_layer(case)), gen)[0]
+        x = torch.randn(case["B"], case["C"], case["H"], case["W"], generator=gen, device=DEVICE)
         st["x"] = x if case["dtype"] == "f32" else x.to(dtype=torch.float16, memory_format=torch.channels_last)
     elif kind == "resnet":
         st["session"] = tmq_amd.optimize_for_inference(_compact(_ResNet18(), gen))
@@ -287,6 +295,113 @@ def run(state):
         streams = [nn.functional.pad(s, (0, layer.weight.numel() // 4 + 64 - s.numel())) for s, layer in zip(streams, model.layers)]
     return streams + \
         [layer.weight.data for layer in other.layers] + [layer.weight.data for layer in model.layers]
+
+
+# ---- the same in 64 bits, plain torch ------------------------------------------------------------------------------
+def _conv64(x, layer):
+    """A convolution layer of torch.nn on a float64 tensor, as columns and one matrix product."""
+    w, k, s, p = layer.weight.double(), layer.kernel_size, layer.stride, layer.padding
+    B, C, H, W = x.shape
+    if isinstance(layer, nn.ConvTranspose2d):
+        size = [(n - 1) * s[i] - 2 * p[i] + k[i] for i, n in enumerate((H, W))]
+        cols = (w.reshape(C, -1).t() @ x.permute(1, 0, 2, 3).reshape(C, -1)).view(-1, B, H * W).permute(1, 0, 2)
+        y = nn.functional.fold(cols, size, k, stride=s, padding=p)
+    else:
+        size = [(n + 2 * p[i] - k[i]) // s[i] + 1 for i, n in enumerate((H, W))]
+        cols = nn.functional.unfold(x, k, padding=p, stride=s)
+        if layer.groups != 1:
+            y = (cols.view(B, C, k[0] * k[1], -1) * w.view(1, C, -1, 1)).sum(2)
+        else:
+            y = (w.reshape(len(w), -1) @ cols.permute(1, 0, 2).reshape(cols.shape[1], -1)).view(len(w), B, -1).permute(1, 0, 2)
+        y = y.reshape(B, -1, *size)
+    return y if layer.bias is None else y + layer.bias.double().view(1, -1, 1, 1)
+
+
+def _norm64(x, bn):
+    v = [t.double().view(1, -1, 1, 1) for t in (bn.running_mean, bn.running_var, bn.weight, bn.bias)]
+    return (x - v[0]) / (v[1] + bn.eps).sqrt() * v[2] + v[3]
+
+
+def _resnet64(net, x):
+    x = nn.functional.max_pool2d(torch.relu(_norm64(_conv64(x, net.conv1), net.bn1)), 3, 2, 1)
+    for stage in (net.layer1, net.layer2, net.layer3, net.layer4):
+        for block in stage:
+            idt = x if block.downsample is None else _norm64(_conv64(x, block.downsample[0]), block.downsample[1])
+            y = torch.relu(_norm64(_conv64(x, block.conv1), block.bn1))
+            x = torch.relu(_norm64(_conv64(y, block.conv2), block.bn2) + idt)
+    return x.mean((2, 3)) @ net.fc.weight.double().t() + net.fc.bias.double()
+
+
+def _staircase64(w, d, order):
+    """The soft staircase of steepness d (order 0), its slope (1) and the slope's derivative (2)."""
+    half = min(3.0, d / 2)
+    c = 2 * half * (half * half + 27) / (27 + 9 * half * half)
+    x = (d * (w - w.floor()) - d / 2).clamp(-3, 3)
+    b = x * x + 3
+    if order == 0:
+        return x * (x * x + 27) / (9 * b) / c + 0.5 + w.floor()
+    return d * (b - 12) ** 2 / (9 * b * b) / c if order == 1 else d * d * 16 * x * (b - 12) / (3 * b ** 3) / c
+
+
+class _Soft64(torch.autograd.Function):
+    """The staircase with the slope the training rule gives it, order 0, or the penalty on it, order 1."""
+
+    @staticmethod
+    def forward(ctx, w, d, order, strength):
+        ctx.save_for_backward(w)
+        ctx.args = d, order, strength
+        return strength * _staircase64(w, d, order)
+
+    @staticmethod
+    def backward(ctx, g):
+        d, order, strength = ctx.args
+        return g * strength * _staircase64(ctx.saved_tensors[0], d, order + 1), None, None, None
+
+
+@torch.enable_grad()
+def exact(case, seed):
+    gen = torch.Generator(device=DEVICE).manual_seed(seed)
+    kind = case["kind"]
+    if kind == "linear":
+        layer = _train(nn.Sequential(nn.Linear(case["K"], case["N"], bias=case["bias"])).to(DEVICE), gen)[0]
+        x = torch.randn(case["M"], case["K"], generator=gen, device=DEVICE).to(_DTYPE[case["dtype"]])
+        y = x.double() @ layer.weight.detach().double().t()
+        return y if layer.bias is None else y + layer.bias.detach().double()
+    if kind == "conv":
+        layer = _train(nn.Sequential(_conv_layer(case)).to(DEVICE), gen)[0].requires_grad_(False)
+        x = torch.randn(case["B"], case["C"], case["H"], case["W"], generator=gen, device=DEVICE)
+        return _conv64(x.to(_DTYPE[case["dtype"]]).double(), layer)
+    if kind == "resnet":
+        net = _train(_ResNet18().to(DEVICE).eval(), gen).requires_grad_(False)
+        x = torch.randn(case["B"], 3, case["size"], case["size"], generator=gen, device=DEVICE).to(_DTYPE[case["dtype"]])
+        return _resnet64(net, x.double())
+    if kind == "mlp":
+        net = _Mlp(case["features"], case["hidden"], case["classes"]).to(DEVICE).double().train()
+        for m in (net.fc1, net.fc2):
+            m.weight.data = (2 * torch.rand(m.weight.shape, generator=gen, device=DEVICE) - 1).double()
+        x = torch.randn(case["batch"], case["features"], generator=gen, device=DEVICE).double()
+        labels = torch.randint(0, case["classes"], (case["batch"],), generator=gen, device=DEVICE)
+        schedule = tmq_amd.QuantizationControl(epoch_knots=tmq_amd.QuantizationScheduleBuilder.default_schedule(150),
+                                               qpenalty_range=(5e-4, 5e-4))
+        for epoch in range(60):
+            schedule.step(epoch)
+        w1, w2 = (_Soft64.apply(m.weight, schedule.digamma, 0, 1.0) for m in (net.fc1, net.fc2))
+        out = net.bn2(torch.relu(net.bn1(x @ w1.t())) @ w2.t())
+        loss = nn.functional.cross_entropy(out, labels)
+        for m in (net.fc1, net.fc2):
+            loss = loss + _Soft64.apply(m.weight, schedule.qpenalty_sharpness, 1, schedule.qpenalty).mean()
+        loss.backward()
+        grads = [p.grad for p in net.parameters()]
+        return [loss.detach(), out.detach()] + grads + [(m.weight.detach() - 1e-4 * m.weight.grad).clamp(-1, 1) for m in (net.fc1, net.fc2)]
+    if kind == "qat":
+        sizes = _spread(case["layers"], case["smallest"], case["largest"])
+        ws = [(2.04 * torch.rand(n, generator=gen, device=DEVICE) - 1.02).double() for n in sizes]
+        gs = [(1e-2 * torch.randn(n, generator=gen, device=DEVICE)).double() for n in sizes]
+        loss = sum(5e-4 * _staircase64(w, 5.0, 1).mean() for w in ws)
+        return [_staircase64(w, 3.0004, 0) for w in ws] + [loss] + \
+            [g * _staircase64(w, 3.0004, 1) + 5e-4 / w.numel() * _staircase64(w, 5.0, 2) for w, g in zip(ws, gs)] + \
+            [w.clamp(-1, 1) for w in ws]
+    return None                                    # bytes, words and whole numbers
 
 
 # ---- what a pass cannot do without ---------------------------------------------------------------------------------
