@@ -379,6 +379,10 @@ int tmq_split_f32(const float *x, void *hi, void *lo, int64_t n, void *stream);
 size_t tmq_f32_to_f16_prescaled_workspace_bytes(int64_t n);
 int tmq_f32_to_f16_prescaled(const float *x, int64_t n, float *prescale, void *hi, const float *scale_in, float *scale_out,
                              int64_t channels, void *workspace, void *stream);
+/* The same for a planar tensor x [B][C][HW], hi in channels-last order [B][HW][C]: conversion and reordering in one
+ * launch behind the scan (workspace: tmq_f32_to_f16_prescaled_workspace_bytes(B C HW) bytes).            */
+int tmq_f32_nchw_to_f16_nhwc_prescaled(const float *x, int64_t B, int64_t C, int64_t HW, float *prescale, void *hi,
+                                       const float *scale_in, float *scale_out, int64_t channels, void *workspace, void *stream);
 
 /* 1 if M fp32 rows against a K x N layer are faster as two fp16 passes over tmq_split_f32's terms than
  * as one tmq_ternary_linear call with x_dtype TMQ_F32 (many rows, or a few rows over a large

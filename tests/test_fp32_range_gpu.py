@@ -221,6 +221,25 @@ def test_one_call_conversion_equals_prescale_then_split(cuda, shape):
         assert torch.equal(hi3.view(torch.int16), want.view(torch.int16)) and torch.equal(adj3, ops.f32_prescale(x, None, 24)[2])
 
 
+@pytest.mark.parametrize("shape", [(2, 64, 56, 56), (3, 5, 9, 11), (1, 70, 13, 4), (2, 100, 3, 7), (5, 17, 16, 16), (1, 130, 1, 65),
+                                   (300, 3, 2, 1), (2, 24, 31, 36)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_planar_input_converts_straight_into_channels_last(cuda, shape, shift):
+    """The converting launch that also reorders: the same bits as the conversion in place followed by a strided copy,
+    at the edges of its tiles (16 / 32 / 64 channels by 256 / 128 / 64 pixels), for odd channel counts and planes, and for
+    a base that is not 16-byte aligned (shift)."""
+    from tmq_amd import ops
+    g = torch.Generator(device=cuda).manual_seed(sum(shape))
+    n = int(np.prod(shape))
+    x = (torch.randn(n + shift, device=cuda, generator=g) * 3e5)[shift:].view(shape)
+    x.view(-1)[n // 2] = float("nan")                             # takes no part in the maximum, stays NaN
+    scale = torch.rand(24, device=cuda, generator=g) + 0.5
+    want, adj = ops.f32_to_f16_prescaled(x, scale, 24)
+    got, adj2 = ops.f32_to_f16_prescaled(x, scale, 24, channels_last=True)
+    assert got.is_contiguous(memory_format=torch.channels_last) and got.shape == x.shape
+    assert torch.equal(got.contiguous().view(torch.int16), want.view(torch.int16)) and torch.equal(adj, adj2)
+
+
 def test_switch_sends_many_rows_against_a_narrow_layer_to_the_one_pass_kernel(cuda):
     """With the prescale switched off (values promised to lie in fp16's range), a thousand fp32 rows or more against at
     most 128 channels skip the row-pair route, whose split pass would move the rows three times: same values to fp32

@@ -592,10 +592,11 @@ def split_f32(x: torch.Tensor, prescale=None, want_lo: bool = True):
     return hi, lo
 
 
-def f32_to_f16_prescaled(x: torch.Tensor, scale, channels: int):
+def f32_to_f16_prescaled(x: torch.Tensor, scale, channels: int, channels_last: bool = False):
     """One fp16 term of an fp32 activation tensor for the convolution kernels: (fp16 tensor of x's shape and
     memory format holding s x, scale / s) with the range prescale s, or (x.half(), scale) when the prescale
-    is switched off."""
+    is switched off. channels_last: a planar [B, C, H, W] tensor comes back in channels_last memory, reordered by
+    the launch that converts it."""
     if not _fp32_prescale or x.numel() == 0:      # nothing to scale in an empty batch
         return x.to(torch.float16), scale
     if not (x.is_contiguous() or x.is_contiguous(memory_format=torch.channels_last)):
@@ -606,9 +607,16 @@ def f32_to_f16_prescaled(x: torch.Tensor, scale, channels: int):
     lib = _lib()
     n = x.numel()
     ps = torch.empty(2, dtype=torch.float32, device=x.device)
-    hi = torch.empty_like(x, dtype=torch.float16)
     adj = torch.empty(channels, dtype=torch.float32, device=x.device) if channels else None
     ws = torch.empty(lib.tmq_f32_to_f16_prescaled_workspace_bytes(n), dtype=torch.uint8, device=x.device)
+    if channels_last and not x.is_contiguous(memory_format=torch.channels_last):
+        B, C, H, W = x.shape
+        hi = torch.empty((B, C, H, W), dtype=torch.float16, device=x.device, memory_format=torch.channels_last)
+        with _capi.on_device(x.device):
+            check(lib.tmq_f32_nchw_to_f16_nhwc_prescaled(ptr(x), B, C, H * W, ptr(ps), ptr(hi), ptr(scale), ptr(adj), channels,
+                                                         ptr(ws), stream_of(x)), "f32_nchw_to_f16_nhwc_prescaled")
+        return hi, (adj if channels else scale)
+    hi = torch.empty_like(x, dtype=torch.float16)
     with _capi.on_device(x.device):
         check(lib.tmq_f32_to_f16_prescaled(ptr(x), n, ptr(ps), ptr(hi), ptr(scale), ptr(adj), channels, ptr(ws), stream_of(x)),
               "f32_to_f16_prescaled")
@@ -727,7 +735,7 @@ def ternary_conv2d(x: torch.Tensor, nw: NativeWeights, stride=1, padding=0, dila
     if x.shape[1] != nw.C:
         raise RuntimeError(f"ternary_conv2d: input has {x.shape[1]} channels, weights expect {nw.C}")
     if x.dtype == torch.float32:
-        x, scale = f32_to_f16_prescaled(x, scale, nw.N)
+        x, scale = f32_to_f16_prescaled(x, scale, nw.N, channels_last=True)
     if x.dtype != torch.float16 or not x.is_contiguous(memory_format=torch.channels_last):
         x = x.to(dtype=torch.float16, memory_format=torch.channels_last)
     B, C, H, W = x.shape
@@ -796,7 +804,7 @@ def ternary_conv2d_relu_maxpool(x: torch.Tensor, nw: NativeWeights, stride=1, pa
     if x.shape[1] != nw.C:
         raise RuntimeError(f"ternary_conv2d_relu_maxpool: input has {x.shape[1]} channels, weights expect {nw.C}")
     if x.dtype == torch.float32:
-        x, scale = f32_to_f16_prescaled(x, scale, nw.N)
+        x, scale = f32_to_f16_prescaled(x, scale, nw.N, channels_last=True)
     if x.dtype != torch.float16 or not x.is_contiguous(memory_format=torch.channels_last):
         x = x.to(dtype=torch.float16, memory_format=torch.channels_last)
     B, C, H, W = x.shape
@@ -884,7 +892,7 @@ def ternary_dwconv2d(x: torch.Tensor, words: torch.Tensor, kernel, stride=1, pad
     if words.dtype != torch.int32 or words.numel() != ky * kx * ((C + 15) // 16):
         raise RuntimeError("ternary_dwconv2d: expected the int32 compact words of a [C, 1, ky, kx] weight tensor")
     if x.dtype == torch.float32:
-        x, scale = f32_to_f16_prescaled(x, scale, C)
+        x, scale = f32_to_f16_prescaled(x, scale, C, channels_last=True)
     if x.dtype != torch.float16 or not x.is_contiguous(memory_format=torch.channels_last):
         x = x.to(dtype=torch.float16, memory_format=torch.channels_last)
     words = words.contiguous()
@@ -943,7 +951,7 @@ def ternary_dwconvtrans2d(x: torch.Tensor, words: torch.Tensor, kernel, stride=1
     if words.dtype != torch.int32 or words.numel() != ky * kx * ((C + 15) // 16):
         raise RuntimeError("ternary_dwconvtrans2d: expected the int32 compact words of a [C, 1, ky, kx] weight tensor")
     if x.dtype == torch.float32:
-        x, scale = f32_to_f16_prescaled(x, scale, C)
+        x, scale = f32_to_f16_prescaled(x, scale, C, channels_last=True)
     if x.dtype != torch.float16 or not x.is_contiguous(memory_format=torch.channels_last):
         x = x.to(dtype=torch.float16, memory_format=torch.channels_last)
     words = words.contiguous()

@@ -1037,7 +1037,7 @@ class ConvTranspose2d(Conv2d):
         scale = self._epilogue_scale(cout, x.device)
         bias = self.bias.data.float() if self.bias is not None else None
         if x.dtype == torch.float32:
-            x, scale = ops.f32_to_f16_prescaled(x, scale, cout)     # once for all phases
+            x, scale = ops.f32_to_f16_prescaled(x, scale, cout, channels_last=True)     # once for all phases
         if x.dtype != torch.float16 or not x.is_contiguous(memory_format=torch.channels_last):
             x = x.to(dtype=torch.float16, memory_format=torch.channels_last)
         y = torch.empty((B, cout, h_out, w_out), dtype=_compact_out, device=x.device, memory_format=torch.channels_last)
