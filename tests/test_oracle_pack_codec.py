@@ -168,6 +168,27 @@ def test_codec_round_trip_and_agreement(oracle, p0, shape):
     assert int.from_bytes(so[8:16].tobytes(), "big") == 8 * (so.size - 26 - 1) and so[-1] == 0
 
 
+def test_decoder_on_crafted_probability_tables(oracle):
+    """Headers no encoder writes: tables that sum to 1, to a power of two, far beyond 16 bits, with empty intervals --
+    the divisions the decoder makes as products with an inverse. What it accepts decodes as the oracle (plain divisions)
+    decodes it; an empty interval or a step of zero is refused."""
+    rng = np.random.default_rng(12)
+    tables = [(0, 1, 0), (1, 0, 0), (0, 0, 1), (1, 1, 1), (1, 1, 0), (2, 1, 1), (65535, 65535, 65535), (65535, 1, 65535), (0, 65535, 0),
+              (16384, 32768, 16383), (1, 65533, 1)] + [tuple(int(v) for v in rng.integers(0, 65536, 3)) for _ in range(40)]
+    rows, cols, accepted = 7, 37, 0
+    for k, pmf in enumerate(tables):
+        for payload in (rng.integers(0, 256, 400), np.zeros(400), np.full(400, 255)):
+            head = (rows * cols).to_bytes(8, "big") + (3200).to_bytes(8, "big") + (426).to_bytes(4, "big") + \
+                b"".join(v.to_bytes(2, "big") for v in pmf)
+            stream = np.concatenate([np.frombuffer(head, np.uint8), payload.astype(np.uint8)])
+            rc, words = _lib_decompress(stream, rows, cols)
+            assert rc in (0, -5), (pmf, rc)
+            if rc == 0:
+                accepted += 1
+                assert np.array_equal(words, oracle.decompress(stream, rows, cols)), pmf
+    assert accepted > 50
+
+
 def test_codec_size_is_near_entropy(oracle):
     rng = np.random.default_rng(0)
     u = rng.random((1024, 1024))

@@ -21,11 +21,20 @@ struct Model {
     uint16_t pmf[3];
     uint32_t cum[3];
     uint32_t total;
+    uint64_t inverse;          // floor(2^64 / total) + 1, 0 for total == 1
     void finish() {
         cum[0] = 0;
         cum[1] = pmf[0];
         cum[2] = cum[1] + pmf[1];
         total = cum[2] + pmf[2];
+        inverse = total > 1 ? ~uint64_t(0) / total + 1 : 0;
+    }
+    // range / total without a division, which stood in the chain from one symbol to the next: inverse * total exceeds 2^64
+    // by at most total < 2^18, so the product's high word exceeds the quotient by less than 2^32 2^18 / (2^64 total)
+    // < 1 / total and has the same floor. A symbol in ns (2.7 GHz Xeon, (1/4, 1/2, 1/4)): encoding 9.3 -> 5.6, decoding,
+    // with the search for the symbol as selects, 14.1 -> 7.2.
+    uint32_t step(uint32_t range) const {
+        return inverse ? (uint32_t)(((unsigned __int128)range * inverse) >> 64) : range;
     }
 };
 
@@ -34,9 +43,9 @@ struct RangeState {
     uint32_t low = 0;
     uint32_t range = 0xFFFFFFFFu;
     void narrow(const Model &m, int sym) {
-        range /= m.total;
-        low += m.cum[sym] * range;
-        range *= m.pmf[sym];
+        const uint32_t step = m.step(range);
+        low += m.cum[sym] * step;
+        range = step * m.pmf[sym];
     }
     bool settle() {
         if (((low ^ (low + range)) >> 24) == 0) return true;   // top byte decided
@@ -69,7 +78,6 @@ T load_be(const uint8_t *p) {
 }
 
 constexpr uint8_t kSymOfCode[4] = {1, 2, 0, 3};   // code 00 (0) -> 1, 01 (+1) -> 2, 10 (-1) -> 0
-constexpr uint8_t kCodeOfSym[3] = {2, 0, 1};
 
 }  // namespace
 
@@ -85,13 +93,18 @@ int tmq_compress_ternary(const uint32_t *words, int64_t rows, int64_t columns, u
                          size_t *out_size) {
     if (!words || !out || !out_size || rows <= 0 || columns <= 0) return TMQ_ERR_INVALID_ARG;
     const int64_t qcols = (columns + 15) / 16;
-    int64_t histo[4] = {0, 0, 0, 0};
+    int64_t histo[3] = {0, 0, 0};
     for (int64_t r = 0; r < rows; r++)
         for (int64_t qc = 0; qc < qcols; qc++) {
-            const uint32_t w = words[r * qcols + qc];
-            for (int i = 0, n = lanes_in_word(columns, qc); i < n; i++) histo[kSymOfCode[(w >> (30 - 2 * i)) & 3u]]++;
+            const int n = lanes_in_word(columns, qc);
+            const uint32_t w = n == 16 ? words[r * qcols + qc] : words[r * qcols + qc] & ~(0xFFFFFFFFu >> (2 * n));
+            const uint32_t minus = (w >> 1) & 0x55555555u, plus = w & 0x55555555u;
+            if (minus & plus) return TMQ_ERR_BAD_DATA;   // code 11 is not a ternary value
+            const int neg = __builtin_popcount(minus), pos = __builtin_popcount(plus);
+            histo[0] += neg;
+            histo[1] += n - neg - pos;
+            histo[2] += pos;
         }
-    if (histo[3] != 0) return TMQ_ERR_BAD_DATA;   // code 11 is not a ternary value
     const int64_t total = histo[0] + histo[1] + histo[2];
     const float scale = 65535.f / (float)total;
     Model m;
@@ -103,20 +116,24 @@ int tmq_compress_ternary(const uint32_t *words, int64_t rows, int64_t columns, u
     }
     m.finish();
 
-    std::vector<uint8_t> payload;
-    payload.reserve((size_t)(total / 4) + 64);
+    std::vector<uint8_t> payload((size_t)(total / 4) + 256);
+    size_t pos = 0;
     RangeState st;
     for (int64_t r = 0; r < rows; r++)
         for (int64_t qc = 0; qc < qcols; qc++) {
-            const uint32_t w = words[r * qcols + qc];
-            for (int i = 0, n = lanes_in_word(columns, qc); i < n; i++) {
-                st.narrow(m, kSymOfCode[(w >> (30 - 2 * i)) & 3u]);
+            const int n = lanes_in_word(columns, qc);
+            uint32_t w = words[r * qcols + qc];
+            // room for the whole word: a symbol moves a few bytes at most (at least one unit of a 32-bit range is left)
+            if (payload.size() - pos < 256) payload.resize(payload.size() * 2);
+            for (int i = 0; i < n; i++, w <<= 2) {
+                st.narrow(m, kSymOfCode[w >> 30]);
                 while (st.settle()) {
-                    payload.push_back((uint8_t)(st.low >> 24));
+                    payload[pos++] = (uint8_t)(st.low >> 24);
                     st.shift();
                 }
             }
         }
+    payload.resize(pos);
     for (int i = 0; i < 4; i++) {
         payload.push_back((uint8_t)(st.low >> 24));
         st.low <<= 8;
@@ -163,20 +180,23 @@ int tmq_decompress_ternary(const uint8_t *in, size_t in_size, uint32_t *words, i
             uint32_t w = 0;
             const int n = lanes_in_word(columns, qc);
             for (int i = 0; i < n; i++) {
-                const uint32_t step = st.range / m.total;
+                const uint32_t step = m.step(st.range);
                 if (step == 0) return TMQ_ERR_BAD_DATA;
-                const uint32_t freq = (window - st.low) / step;
-                // Largest symbol whose cumulative count does not exceed freq; symbols of zero
-                // probability are skipped because their interval is empty.
-                int sym = 0;
-                if (m.cum[1] <= freq) sym = (m.cum[2] <= freq) ? 2 : 1;
-                if (m.pmf[sym] == 0) return TMQ_ERR_BAD_DATA;
-                st.narrow(m, sym);
+                // Largest symbol whose cumulative count does not exceed (window - low) / step, without the division;
+                // symbols of zero probability are skipped because their interval is empty.
+                // (Selected without branches -- which symbol comes next is what nobody can predict. An interval of zero
+                // width is one whose probability is zero, step being at least 1.)
+                const uint32_t at = window - st.low, c1 = m.cum[1] * step, c2 = m.cum[2] * step;
+                const bool up1 = at >= c1, up2 = at >= c2;
+                const uint32_t from = up2 ? c2 : up1 ? c1 : 0u, to = up2 ? m.total * step : up1 ? c2 : c1;
+                if (to == from) return TMQ_ERR_BAD_DATA;
+                st.low += from;
+                st.range = to - from;
                 while (st.settle()) {
                     window = (window << 8) | next();
                     st.shift();
                 }
-                w = (w << 2) | kCodeOfSym[sym];
+                w = (w << 2) | (up2 ? 1u : up1 ? 0u : 2u);           // codes of (-1, 0, +1)
             }
             if (n != 16) w <<= 2 * (16 - n);
             words[r * qcols + qc] = w;

@@ -1166,6 +1166,7 @@ def _swap_layers(module, ctrl, prefix, exact, globs):
 def compressed_state_dict(module: nn.Module, strong=False, remove_prefix=""):
     """State dict with TMQ weights bit-stuffed (2 bit / weight) or, with strong=True, range coded;
     the layers are switched to compact inference as a side effect (tmq/tmq.py:1183-1248)."""
+    words = {}       # compact words of the layers coded here: what decoding their streams would give back
     for _, _, _, layer in _tmq_layers(module):
         if not hasattr(layer, "tensor_type"):
             continue
@@ -1176,7 +1177,11 @@ def compressed_state_dict(module: nn.Module, strong=False, remove_prefix=""):
             layer.tensor_type = TensorType.COMPACT_TERNARY_32BIT
         elif strong and layer.tensor_type != TensorType.COMPRESSED_TERNARY_32BIT:
             from_compact = layer.tensor_type == TensorType.COMPACT_TERNARY_32BIT
-            stream = _b.compress_ternary(layer.weight.data, layer.original_shape, from_compact)
+            if not from_compact and layer.weight.dtype == torch.float32:
+                words[id(layer)] = _b.compactify_ternary(layer.weight.data)
+                stream = _b.compress_ternary(words[id(layer)], layer.original_shape, True)
+            else:
+                stream = _b.compress_ternary(layer.weight.data, layer.original_shape, from_compact)
             layer._stream_device = layer.weight.device
             layer.weight = nn.Parameter(stream, requires_grad=False)
             layer.tensor_type = TensorType.COMPRESSED_TERNARY_32BIT
@@ -1191,8 +1196,10 @@ def compressed_state_dict(module: nn.Module, strong=False, remove_prefix=""):
         if layer.tensor_type == TensorType.COMPRESSED_TERNARY_32BIT:
             # keep the model usable right away: back to the compact form in memory
             dev = getattr(layer, "_stream_device", layer.weight.device)
-            layer.weight = nn.Parameter(_b.decompress_ternary(layer.weight.data.cpu(), layer.original_shape).to(dev),
-                                        requires_grad=False)
+            packed = words.pop(id(layer), None)
+            if packed is None:
+                packed = _b.decompress_ternary(layer.weight.data.cpu(), layer.original_shape).to(dev)
+            layer.weight = nn.Parameter(packed, requires_grad=False)
             layer.tensor_type = TensorType.COMPACT_TERNARY_32BIT
     return state
 
