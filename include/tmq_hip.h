@@ -431,6 +431,19 @@ typedef struct tmq_output_view {
 int tmq_ternary_conv2d_view(const void *x, const tmq_conv_shape *shape, const void *native,
                             const tmq_epilogue *epilogue, void *y, const tmq_output_view *view, void *stream);
 
+/* Several such convolutions of ONE input (same B, C, H, W and N; windows, padding and dilation of their own) written
+ * into one destination: phase q goes to the view that starts `first` pixels into y (and into epilogue->residual).
+ * The phases of a transposed convolution, tmq/tmq.py:1007-1042. Inputs of a multiple of 64 channels take one launch
+ * for up to four phases, others one launch per phase.                                               */
+typedef struct tmq_conv_phase {
+    tmq_conv_shape shape;
+    tmq_output_view view;
+    int64_t first;           /* pixel of y where the view starts */
+    const void *native;      /* the phase's own weights */
+} tmq_conv_phase;
+int tmq_ternary_conv2d_phases(const void *x, const tmq_conv_phase *phases, int count, const tmq_epilogue *epilogue, void *y,
+                              void *stream);
+
 /* Depthwise ternary convolution (groups == channels; shape->N must equal shape->C). x: fp16 NHWC;
  * words: the reference packing of a [C][1][ky][kx] weight tensor, words[ky*kx][ceil(C/16)]
  * (tmq_pack_ternary with N = C, K = ky*kx) -- read directly, no re-tiling; y: NHWC in

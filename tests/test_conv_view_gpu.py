@@ -138,3 +138,48 @@ def test_transposed_layer_one_pass(cuda, cin, cout, k, stride, pad, opad, hw, ba
     assert got.shape == ref.shape
     err = ((got.double() - ref).abs().max() / ref.abs().max()).item()
     assert err <= 2e-5, err
+
+
+@pytest.mark.parametrize("cin,cout,k,stride,pad,hw,batch", [
+    (64, 64, 4, 2, 1, (33, 18), 3),            # one launch of four phases; 64 x 64 tiles, ragged last tile
+    (64, 130, 3, 2, 1, (70, 66), 2),           # 128 x 128 tiles, phases of 2 x 2, 2 x 1, 1 x 2 and 1 x 1 taps, a third column tile
+    (128, 66, 5, 3, 2, (9, 11), 2),            # nine phases: three launches
+    (32, 40, 4, 2, 1, (17, 9), 2), (8, 7, 4, 2, 1, (9, 9), 2),       # the few-channel loader
+    (24, 72, 4, 2, 1, (60, 60), 2), (104, 16, 3, 2, 1, (13, 7), 1),  # register-staged loaders: whole 16-byte chunks,
+    (100, 64, 4, 2, 1, (14, 15), 2), (5, 9, 4, 2, 1, (7, 8), 2),     # halves of 8 bytes, single elements
+    (300, 20, 4, 2, 1, (6, 5), 1)])            # a reduction long enough for the deeper prefetch
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_phases_in_one_launch_equal_one_launch_each(cuda, cin, cout, k, stride, pad, hw, batch, dtype):
+    """ops.ternary_conv2d_into(phases=...): every phase of a transposed convolution written by the shared launch equals the
+    same phase written by a launch of its own (small integers: exact in either summation order), with residual and ReLU."""
+    import copy
+    import tmq_amd as t
+    from tmq_amd import ops
+    torch.manual_seed(cin * 100 + cout)
+    net = torch.nn.Sequential(torch.nn.ConvTranspose2d(cin, cout, k, stride, pad, bias=True))
+    t.quantize_model(net, t.QuantizationControl())
+    net.to(cuda).eval()
+    net[0].weight.data = torch.randint(-1, 2, net[0].weight.shape, device=cuda).float()
+    net[0].bias.data = torch.randint(-4, 5, (cout,), device=cuda).float()
+    t.compressed_state_dict(net)
+    layer = net[0]
+    x = torch.randint(-3, 4, (batch, cin) + hw, device=cuda).half().contiguous(memory_format=torch.channels_last)
+    want = F.conv_transpose2d(x.cpu().float(), ops.expand_ternary(layer.weight.data, layer.original_shape).cpu(),
+                              layer.bias.data.cpu(), stride, pad).to(dtype)
+    prev = t.set_compact_output_dtype(dtype)
+    try:
+        got = net(x)
+        again = copy.deepcopy(net)(x)                       # a copy plans for its own weights
+        net(x[:, :, :5, :4])                                # another shape in between
+        assert torch.equal(got.cpu(), want) and torch.equal(again, got) and torch.equal(net(x), got)
+    finally:
+        t.set_compact_output_dtype(prev)
+    plan = layer._phases[2]
+    res = torch.randint(-9, 10, got.shape, device=cuda).to(dtype).contiguous(memory_format=torch.channels_last)
+    one = ops.ternary_conv2d_into(torch.empty_like(res), x, None, residual=res, relu=True, phases=plan)
+    each = torch.empty_like(res)
+    for nw, padding, dil, first, (o0, p0), (sy, sx), _ in plan.parts:
+        ops.ternary_conv2d_into(each[:, :, o0::sy, p0::sx], x, nw, 1, padding, dil, residual=res[:, :, o0::sy, p0::sx], relu=True, first=first)
+    assert torch.equal(one, each)
+    with pytest.raises(RuntimeError):
+        ops.ternary_conv2d_into(each[:, :, :-1], x, None, phases=plan)

@@ -44,6 +44,11 @@ class OutputView(ctypes.Structure):
                 ("stride_b", ctypes.c_int64), ("stride_h", ctypes.c_int64), ("stride_w", ctypes.c_int64)]
 
 
+class ConvPhase(ctypes.Structure):
+    """tmq_conv_phase of include/tmq_hip.h."""
+    _fields_ = [("shape", ConvShape), ("view", OutputView), ("first", ctypes.c_int64), ("native", ctypes.c_void_p)]
+
+
 class Epilogue(ctypes.Structure):
     """tmq_epilogue of include/tmq_hip.h."""
     _fields_ = [("scale", ctypes.c_void_p), ("bias", ctypes.c_void_p), ("residual", ctypes.c_void_p),
@@ -105,6 +110,7 @@ SIGNATURES = {
     "tmq_avgpool_linear": (_int, [_vp, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _vp]),
     "tmq_ternary_conv2d": (_int, [_vp, ctypes.POINTER(ConvShape), _vp, _vp, _vp, _vp]),
     "tmq_ternary_conv2d_view": (_int, [_vp, ctypes.POINTER(ConvShape), _vp, _vp, _vp, ctypes.POINTER(OutputView), _vp]),
+    "tmq_ternary_conv2d_phases": (_int, [_vp, ctypes.POINTER(ConvPhase), _int, _vp, _vp, _vp]),
     "tmq_ternary_conv2d_relu_maxpool": (_int, [_vp, ctypes.POINTER(ConvShape), _vp, _vp, _vp, _vp, _vp]),
     "tmq_ternary_conv2d_relu_maxpool_planar": (_int, [_vp, ctypes.c_int32, ctypes.POINTER(ConvShape), _vp, _vp, _vp, _vp, _vp]),
     "tmq_ternary_dwconv2d": (_int, [_vp, ctypes.POINTER(ConvShape), _vp, _vp, _vp, _vp]),

@@ -413,21 +413,11 @@ struct ConvLoaderFewC {
 
 // ---- the tile kernel ---------------------------------------------------------------------------------
 template <int WM, int WN, int WGM, int WGN, int D, class Loader, class Ep>
-__global__ __launch_bounds__(64 * WGM * WGN, 2) void tile_kernel(Loader ld, const uint32_t *__restrict__ native,
-                                                              int64_t M, int64_t K, int64_t N, int64_t Kb, int64_t Nb,
-                                                              Ep ep, int tiles_m, int tiles_n) {
-    constexpr int T = 64 * WGM * WGN, BM = 16 * WM * WGM, BN = 16 * WN * WGN, CH = BM * 8 / T;
+__device__ __forceinline__ void tile_body(const Loader &ld, const uint32_t *__restrict__ native, int64_t M, int64_t K, int64_t N,
+                                          int64_t Kb, int64_t Nb, const Ep &ep, int64_t m0, int64_t n0,
+                                          _Float16 (&As)[2][16 * WM * WGM * kPitch]) {
+    constexpr int T = 64 * WGM * WGN, BM = 16 * WM * WGM, CH = BM * 8 / T;
     static_assert(BM * 8 % T == 0, "chunks must divide evenly");
-    // two stages: the next k-tile is written while the current one is multiplied (one barrier per tile)
-    __shared__ __attribute__((aligned(16))) _Float16 As[2][BM * kPitch];
-
-    // XCD-aware tile order: workgroup ids go round-robin over the 8 XCDs; give each XCD a
-    // contiguous run of tiles, n fastest, so its L2 sees the same activation rows.
-    int id = blockIdx.x;
-    const int G = tiles_m * tiles_n;
-    if ((G & 7) == 0) id = (id & 7) * (G >> 3) + (id >> 3);
-    const int tm = id / tiles_n, tn = id % tiles_n;
-    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
 
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int wm = wv / WGN, wn = wv % WGN;
@@ -553,6 +543,22 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void tile_kernel(Loader ld, cons
                        nw0, M, N, ep);
 }
 
+template <int WM, int WN, int WGM, int WGN, int D, class Loader, class Ep>
+__global__ __launch_bounds__(64 * WGM * WGN, 2) void tile_kernel(Loader ld, const uint32_t *__restrict__ native,
+                                                              int64_t M, int64_t K, int64_t N, int64_t Kb, int64_t Nb,
+                                                              Ep ep, int tiles_m, int tiles_n) {
+    constexpr int BM = 16 * WM * WGM, BN = 16 * WN * WGN;
+    // two stages: the next k-tile is written while the current one is multiplied (one barrier per tile)
+    __shared__ __attribute__((aligned(16))) _Float16 As[2][BM * kPitch];
+    // XCD-aware tile order: workgroup ids go round-robin over the 8 XCDs; give each XCD a
+    // contiguous run of tiles, n fastest, so its L2 sees the same activation rows.
+    int id = blockIdx.x;
+    const int G = tiles_m * tiles_n;
+    if ((G & 7) == 0) id = (id & 7) * (G >> 3) + (id >> 3);
+    const int tm = id / tiles_n, tn = id % tiles_n;
+    tile_body<WM, WN, WGM, WGN, D>(ld, native, M, K, N, Kb, Nb, ep, (int64_t)tm * BM, (int64_t)tn * BN, As);
+}
+
 // ---- the tile kernel with direct-to-LDS activation loads ----------------------------------------------
 // Same tiling and arithmetic as tile_kernel; the activation tiles go global -> LDS without passing
 // through registers (global_load_lds_dwordx4). That removes the staging registers and the LDS store
@@ -571,23 +577,18 @@ __device__ __forceinline__ void load_to_lds(const void *src, unsigned char *dst)
 #endif
 }
 
+// Rows of a BM-row tile as loaded: BM rounded up to whole chunk rounds of T threads (a 112-row tile of four wavefronts
+// is loaded as 128 rows: the 16 extra rows are the next tile's, fetched and never read).
+constexpr int rows_loaded(int BM, int T) { return (BM * 8 + T - 1) / T * T / 8; }
+
 template <int WM, int WN, int WGM, int WGN, int P, class Loader, class Ep>
-__global__ __launch_bounds__(64 * WGM * WGN, WGM * WGN > 4 ? 1 : 2) void tile_dma_kernel(Loader ld, const uint32_t *__restrict__ native,
-                                                                  int64_t M, int64_t K, int64_t N, int64_t Kb,
-                                                                  int64_t Nb, Ep ep, int tiles_m, int tiles_n) {
-    // BL: rows per tile as loaded -- BM rounded up to whole chunk rounds of the workgroup (a 112-row tile of four
-    // wavefronts is loaded as 128 rows: the 16 extra rows are the next tile's, fetched and never read)
-    constexpr int T = 64 * WGM * WGN, BM = 16 * WM * WGM, BN = 16 * WN * WGN, BL = (BM * 8 + T - 1) / T * T / 8;
+__device__ __forceinline__ void tile_dma_body(const Loader &ld, const uint32_t *__restrict__ native, int64_t M, int64_t K, int64_t N,
+                                              int64_t Kb, int64_t Nb, const Ep &ep, int64_t m0, int64_t n0,
+                                              _Float16 (&As)[2 * P][rows_loaded(16 * WM * WGM, 64 * WGM * WGN) * kPitch]) {
+    constexpr int T = 64 * WGM * WGN, BL = rows_loaded(16 * WM * WGM, T);
     constexpr int CH = BL * 8 / T, S = 2 * P;
     constexpr int kTileBytes = BL * kPitch * 2;
     static_assert(P >= 1 && P <= 2, "geometry");
-    __shared__ __attribute__((aligned(16))) _Float16 As[S][BL * kPitch];
-
-    int id = blockIdx.x;
-    const int G = tiles_m * tiles_n;
-    if ((G & 7) == 0) id = (id & 7) * (G >> 3) + (id >> 3);
-    const int tm = id / tiles_n, tn = id % tiles_n;
-    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
 
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wv / WGN, wn = wv % WGN;
@@ -706,6 +707,52 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGM * WGN > 4 ? 1 : 2) void tile_dm
     static_assert(WGM * WGN * 16 * kEP * 4 <= S * kTileBytes, "epilogue slab does not fit the LDS buffer");
     write_tile<WM, WN>(reinterpret_cast<float *>(&As[0][0]) + wv * 16 * kEP, acc, cc, lane, m0 + (int64_t)wm * WM * 16,
                        nw0, M, N, ep);
+}
+
+template <int WM, int WN, int WGM, int WGN, int P, class Loader, class Ep>
+__global__ __launch_bounds__(64 * WGM * WGN, WGM * WGN > 4 ? 1 : 2) void tile_dma_kernel(Loader ld, const uint32_t *__restrict__ native,
+                                                                  int64_t M, int64_t K, int64_t N, int64_t Kb,
+                                                                  int64_t Nb, Ep ep, int tiles_m, int tiles_n) {
+    constexpr int BM = 16 * WM * WGM, BN = 16 * WN * WGN;
+    __shared__ __attribute__((aligned(16))) _Float16 As[2 * P][rows_loaded(BM, 64 * WGM * WGN) * kPitch];
+    int id = blockIdx.x;
+    const int G = tiles_m * tiles_n;
+    if ((G & 7) == 0) id = (id & 7) * (G >> 3) + (id >> 3);
+    const int tm = id / tiles_n, tn = id % tiles_n;
+    tile_dma_body<WM, WN, WGM, WGN, P>(ld, native, M, K, N, Kb, Nb, ep, (int64_t)tm * BM, (int64_t)tn * BN, As);
+}
+
+// Up to kPhases convolutions of the same input in one launch (the phases of a transposed convolution): the phases of one
+// tile position are neighbours in an XCD's run of workgroups, so the input they share is fetched into that L2 once, and
+// four short launches with a ramp and a tail each become one. A phase with fewer tiles than the largest leaves the rest out.
+constexpr int kPhases = 4;
+template <class Loader, class Ep>
+struct PhaseSet {
+    struct Phase {
+        Loader ld;
+        const uint32_t *native;
+        int64_t M, K, Kb;
+        Ep ep;
+    } phase[kPhases];
+    int64_t N, Nb;
+    int32_t count, tiles_m, tiles_n;
+};
+
+// P: tiles per pass (direct loaders) or register prefetch depth (register loaders).
+template <int WM, int WN, int WGM, int WGN, int P, class Loader, class Ep>
+__global__ __launch_bounds__(64 * WGM * WGN, 2) void tile_phases_kernel(PhaseSet<Loader, Ep> set) {
+    constexpr int BM = 16 * WM * WGM, BN = 16 * WN * WGN;
+    constexpr int kStages = Loader::kDirect ? 2 * P : 2, kRows = Loader::kDirect ? rows_loaded(BM, 64 * WGM * WGN) : BM;
+    __shared__ __attribute__((aligned(16))) _Float16 As[kStages][kRows * kPitch];
+    const int id = xcd_contiguous(blockIdx.x, set.count * set.tiles_m * set.tiles_n);
+    const int tn = id % set.tiles_n, t = id / set.tiles_n, q = t % set.count;
+    const int64_t m0 = (int64_t)(t / set.count) * BM;
+    const auto ph = set.phase[q];
+    if (m0 >= ph.M) return;                                        // the whole workgroup
+    if constexpr (Loader::kDirect)
+        tile_dma_body<WM, WN, WGM, WGN, P>(ph.ld, ph.native, ph.M, ph.K, set.N, ph.Kb, set.Nb, ph.ep, m0, (int64_t)tn * BN, As);
+    else
+        tile_body<WM, WN, WGM, WGN, P>(ph.ld, ph.native, ph.M, ph.K, set.N, ph.Kb, set.Nb, ph.ep, m0, (int64_t)tn * BN, As);
 }
 
 // ---- one workgroup per CU: everything a wavefront does besides MFMAs goes between its MFMAs -----------------
@@ -968,6 +1015,20 @@ int launch_tile(const Loader &ld, const void *native, int64_t M, int64_t K, int6
     return check_launch();
 }
 
+template <int WM, int WN, int WGM, int WGN, int P, class Loader, class Ep>
+int launch_phases(PhaseSet<Loader, Ep> &set, void *stream) {
+    constexpr int BM = 16 * WM * WGM, BN = 16 * WN * WGN;
+    int64_t tm = 0, tn = (set.N + BN - 1) / BN;
+    for (int q = 0; q < set.count; q++)
+        if ((set.phase[q].M + BM - 1) / BM > tm) tm = (set.phase[q].M + BM - 1) / BM;
+    if (tm * tn * set.count > 0x7FFFFFFF) return TMQ_ERR_TOO_LARGE;
+    set.tiles_m = (int32_t)tm;
+    set.tiles_n = (int32_t)tn;
+    hipLaunchKernelGGL((tile_phases_kernel<WM, WN, WGM, WGN, P, Loader, Ep>), dim3((uint32_t)(set.count * tm * tn)),
+                       dim3(64 * WGM * WGN), 0, as_stream(stream), set);
+    return check_launch();
+}
+
 // Tile choice, from a sweep over M x K x N (4096^2 weights at M = 768 .. 4096 and the ResNet-18 layer
 // shapes): 128 x 256 once it gives 1.5 workgroups per CU, 128 x 128 down to one per CU, else
 // 64 x 64. Larger tiles (256 x 256, 256 x 128) and 128 x 64 never won.
@@ -1194,6 +1255,77 @@ inline size_t pair_rows_bytes(int64_t M, int64_t K, int64_t N) {
 namespace tmq {
 namespace {
 
+// Checks a convolution's shape and the view its rows go to; ho, wo: the computed grid, map: set when there is a view.
+int conv_plan(const tmq_conv_shape *s, const tmq_output_view *view, int32_t &ho, int32_t &wo, RowMap &map) {
+    const int rc = tmq_conv2d_out_hw(s, &ho, &wo);
+    if (rc != TMQ_OK) return rc;
+    if (s->B < 0 || s->C <= 0 || s->H <= 0 || s->W <= 0 || s->N <= 0 || s->py < 0 || s->px < 0) return TMQ_ERR_INVALID_ARG;
+    if (ho <= 0 || wo <= 0) return TMQ_ERR_INVALID_ARG;
+    const int64_t M = (int64_t)s->B * ho * wo;
+    if (M == 0 || !view) return TMQ_OK;
+    // the kept part of the computed grid must lie inside it; rows are decomposed with 32-bit arithmetic
+    if (view->h0 < 0 || view->w0 < 0 || view->h_cnt < 0 || view->w_cnt < 0 || view->h0 + (int64_t)view->h_cnt > ho ||
+        view->w0 + (int64_t)view->w_cnt > wo || view->stride_b < 0 || view->stride_h < 0 || view->stride_w < 0)
+        return TMQ_ERR_INVALID_ARG;
+    if (M >= (int64_t)0x7FFFFFFF) return TMQ_ERR_TOO_LARGE;
+    map.hw = FastDiv((uint32_t)ho * (uint32_t)wo);
+    map.w = FastDiv((uint32_t)wo);
+    map.h0 = view->h0; map.w0 = view->w0; map.h_cnt = view->h_cnt; map.w_cnt = view->w_cnt;
+    map.sb = view->stride_b; map.sh = view->stride_h; map.sw = view->stride_w;
+    return TMQ_OK;
+}
+
+// The convolutions of tmq_ternary_conv2d_phases, kPhases to a launch. 64 x 64 tiles up to 64 channels, 128 x 128 (register
+// loaders: of 64 x 64 per wavefront) beyond where that gives every CU one, all phases counted together. Against one launch
+// per phase, which few tiles sent to the split-reduction kernel -- 4 x 4 / 2 in fp16, one image or a batch: 128 -> 64
+// channels on 56 x 56, batch 32 61.7 -> 44.3 us; 256 -> 128 on 28 x 28, batch 16 41.9 -> 21.4; 64 -> 64 on 32 x 32, batch 8
+// 21.2 -> 7.9; 100 -> 64 on 28 x 28, batch 8 50.4 -> 16.6; 32 -> 32 on 56 x 56, batch 8 23.9 -> 9.6; 128 -> 64 on one 14 x 14
+// image 13.1 -> 7.7; and 512 -> 256 on one 7 x 7 image, where the split reduction is at its best, 16.5 -> 16.7.
+template <class Loader>
+int conv_phases(const _Float16 *x, const tmq_conv_phase *phases, int count, const tmq_epilogue &e, void *y, void *stream) {
+    const int64_t N = phases[0].shape.N, elt = e.y_dtype == TMQ_F16 ? 2 : 4;
+    for (int first = 0; first < count; first += kPhases) {
+        PhaseSet<Loader, ViewEpilogue> set{};
+        set.N = N;
+        set.Nb = native_blocks_n(N);
+        int64_t wide = 0, longest = 0;
+        for (int q = first; q < count && q < first + kPhases; q++) {
+            const tmq_conv_phase &p = phases[q];
+            const tmq_conv_shape &s = p.shape;
+            int32_t ho, wo;
+            RowMap map;
+            if (int rc = conv_plan(&s, &p.view, ho, wo, map)) return rc;
+            const int64_t M = (int64_t)s.B * ho * wo, K = (int64_t)s.C * s.ky * s.kx;
+            if (M == 0 || p.view.h_cnt == 0 || p.view.w_cnt == 0) continue;
+            auto &ph = set.phase[set.count++];
+            ph.ld = Loader{x, M, K, s.B, s.C, s.H, s.W, ho, wo, s.ky, s.kx, s.sy, s.sx, s.py, s.px, s.dy, s.dx};
+            if constexpr (Loader::kDirect) ph.ld = with_divisors(ph.ld);
+            if constexpr (std::is_same<Loader, ConvLoader<false>>::value)
+                ph.ld.quads = s.C % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 7u) == 0 ? 1 : 0;
+            ph.native = static_cast<const uint32_t *>(p.native);
+            ph.M = M;
+            ph.K = K;
+            ph.Kb = native_blocks_k(K);
+            const unsigned char *res = e.residual ? static_cast<const unsigned char *>(e.residual) + p.first * N * elt : nullptr;
+            ph.ep = ViewEpilogue{e.scale, e.bias, res, static_cast<unsigned char *>(y) + p.first * N * elt, e.relu,
+                                 e.y_dtype == TMQ_F16 ? 1 : 0, map};
+            wide += ((M + 127) / 128) * ((N + 127) / 128);
+            if (K > longest) longest = K;
+        }
+        if (set.count == 0) continue;
+        int rc;
+        if constexpr (Loader::kDirect) {
+            rc = N > 64 && wide >= 256 ? launch_phases<8, 2, 1, 4, 1>(set, stream) : launch_phases<4, 2, 1, 2, 1>(set, stream);
+        } else {
+            const bool deep = longest >= 16 * kBK;                 // prefetch depth as in dispatch_tile
+            if (N > 64 && wide >= 256) rc = deep ? launch_phases<4, 4, 2, 2, 2>(set, stream) : launch_phases<4, 4, 2, 2, 1>(set, stream);
+            else rc = deep ? launch_phases<4, 2, 1, 2, 2>(set, stream) : launch_phases<4, 2, 1, 2, 1>(set, stream);
+        }
+        if (rc) return rc;
+    }
+    return TMQ_OK;
+}
+
 // The tile kernels behind tmq_ternary_conv2d for an epilogue with consecutive rows (Epilogue) or rows scattered into a
 // strided destination (ViewEpilogue).
 template <class Ep>
@@ -1338,31 +1470,43 @@ int tmq_ternary_conv2d_view(const void *x, const tmq_conv_shape *s, const void *
     const int relu = e.relu, y_dtype = e.y_dtype;
     if (y_dtype != TMQ_F16 && y_dtype != TMQ_F32) return TMQ_ERR_UNSUPPORTED;
     int32_t ho, wo;
-    int rc = tmq_conv2d_out_hw(s, &ho, &wo);
-    if (rc != TMQ_OK) return rc;
-    if (s->B < 0 || s->C <= 0 || s->H <= 0 || s->W <= 0 || s->N <= 0 || s->py < 0 || s->px < 0) return TMQ_ERR_INVALID_ARG;
-    if (ho <= 0 || wo <= 0) return TMQ_ERR_INVALID_ARG;
-    const int64_t M = (int64_t)s->B * ho * wo, K = (int64_t)s->C * s->ky * s->kx;
-    if (M == 0) return TMQ_OK;
     RowMap map;
-    if (view) {
-        // the kept part of the computed grid must lie inside it; rows are decomposed with 32-bit arithmetic
-        if (view->h0 < 0 || view->w0 < 0 || view->h_cnt < 0 || view->w_cnt < 0 || view->h0 + (int64_t)view->h_cnt > ho ||
-            view->w0 + (int64_t)view->w_cnt > wo || view->stride_b < 0 || view->stride_h < 0 || view->stride_w < 0)
-            return TMQ_ERR_INVALID_ARG;
-        if (M >= (int64_t)0x7FFFFFFF) return TMQ_ERR_TOO_LARGE;
-        if (view->h_cnt == 0 || view->w_cnt == 0) return TMQ_OK;
-        map.hw = FastDiv((uint32_t)ho * (uint32_t)wo);
-        map.w = FastDiv((uint32_t)wo);
-        map.h0 = view->h0; map.w0 = view->w0; map.h_cnt = view->h_cnt; map.w_cnt = view->w_cnt;
-        map.sb = view->stride_b; map.sh = view->stride_h; map.sw = view->stride_w;
-    }
+    const int rc = conv_plan(s, view, ho, wo, map);
+    if (rc != TMQ_OK) return rc;
+    const int64_t M = (int64_t)s->B * ho * wo, K = (int64_t)s->C * s->ky * s->kx;
+    if (M == 0 || (view && (view->h_cnt == 0 || view->w_cnt == 0))) return TMQ_OK;
     const int y_f16 = y_dtype == TMQ_F16 ? 1 : 0;
     // few output tiles: split the reduction inside the workgroup (mid.hip)
     if (mid_conv_ok(x, s) && split_reduction_pays(M, K, s->N))
         return launch_mid_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, view ? &map : nullptr, stream);
     if (view) return conv_tiles(x, s, ho, wo, native, ViewEpilogue{scale, bias, residual, y, relu, y_f16, map}, stream);
     return conv_tiles(x, s, ho, wo, native, Epilogue{scale, bias, residual, y, relu, y_f16, {}}, stream);
+}
+
+int tmq_ternary_conv2d_phases(const void *x, const tmq_conv_phase *phases, int count, const tmq_epilogue *epilogue, void *y,
+                              void *stream) {
+    if (!x || !phases || count <= 0 || !y) return TMQ_ERR_INVALID_ARG;
+    tmq_epilogue e = {nullptr, nullptr, nullptr, 0, TMQ_F32};
+    if (epilogue) e = *epilogue;
+    if (e.y_dtype != TMQ_F16 && e.y_dtype != TMQ_F32) return TMQ_ERR_UNSUPPORTED;
+    const tmq_conv_shape &s0 = phases[0].shape;
+    int taps = 1;
+    for (int q = 0; q < count; q++) {                              // everything is checked before anything is launched
+        const tmq_conv_phase &p = phases[q];
+        int32_t ho, wo;
+        RowMap map;
+        if (!p.native || !aligned16(p.native) || p.first < 0) return TMQ_ERR_INVALID_ARG;
+        if (p.shape.B != s0.B || p.shape.C != s0.C || p.shape.H != s0.H || p.shape.W != s0.W || p.shape.N != s0.N) return TMQ_ERR_INVALID_ARG;
+        if (int rc = conv_plan(&p.shape, &p.view, ho, wo, map)) return rc;
+        if (p.shape.ky > taps) taps = p.shape.ky;
+        if (p.shape.kx > taps) taps = p.shape.kx;
+    }
+    const _Float16 *xp = static_cast<const _Float16 *>(x);
+    const bool small = (int64_t)s0.B * s0.H * s0.W * s0.C < (int64_t)0x7FFFFFF0;
+    if (s0.C % kBK == 0 && taps <= 15 && aligned16(x) && small) return conv_phases<ConvLoader64>(xp, phases, count, e, y, stream);
+    if ((s0.C == 8 || s0.C == 16 || s0.C == 32) && aligned16(x) && small) return conv_phases<ConvLoaderFewC>(xp, phases, count, e, y, stream);
+    if (s0.C % 8 == 0 && aligned16(x)) return conv_phases<ConvLoader<true>>(xp, phases, count, e, y, stream);
+    return conv_phases<ConvLoader<false>>(xp, phases, count, e, y, stream);
 }
 
 }  // extern "C"

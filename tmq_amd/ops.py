@@ -757,11 +757,15 @@ def ternary_conv2d(x: torch.Tensor, nw: NativeWeights, stride=1, padding=0, dila
 
 
 def ternary_conv2d_into(out: torch.Tensor, x: torch.Tensor, nw: NativeWeights, stride=1, padding=0, dilation=1, scale=None,
-                        bias=None, residual=None, relu=False, first=(0, 0)) -> torch.Tensor:
+                        bias=None, residual=None, relu=False, first=(0, 0), phases=None) -> torch.Tensor:
     """ternary_conv2d written straight into `out`, a strided view [B, N, h, w] of a channels_last tensor (fp16 or
     fp32, e.g. big[:, :, 1::2, 0::2]): output position (first[0] + i, first[1] + j) of the convolution goes to
     out[:, :, i, j]; positions of the convolution outside that h x w window are dropped. `residual`, when given, is a
-    view with out's shape and strides. One launch, no temporary. x must already be fp16."""
+    view with out's shape and strides. One launch, no temporary. x must already be fp16.
+    phases (then nw is None and `out` the whole dense channels_last tensor): several convolutions of x, each with weights,
+    padding and a share of `out` of its own, as a ConvPhases."""
+    if phases is not None:
+        return phases.run(out, x, scale, bias, residual, relu)
     pair = lambda v: tuple(v) if isinstance(v, (tuple, list)) else (v, v)
     (sy, sx), (py, px), (dy, dx) = pair(stride), pair(padding), pair(dilation)
     (py, py_end), (px, px_end) = pair(py), pair(px)
@@ -787,6 +791,50 @@ def ternary_conv2d_into(out: torch.Tensor, x: torch.Tensor, nw: NativeWeights, s
         check(_lib().tmq_ternary_conv2d_view(ptr(x), ctypes.byref(shp), ptr(nw.buf), ctypes.byref(ep), ptr(out),
                                              ctypes.byref(view), stream_of(x)), "ternary_conv2d_view")
     return out
+
+
+class ConvPhases:
+    """Convolutions of one [B, C, H, W] input whose results interleave in one [B, N, Ho, Wo] channels_last tensor: what
+    ternary_conv2d_into(phases=...) launches together (up to four per launch). parts: (NativeWeights, padding as
+    ((top, bottom), (left, right)), dilation, first position of the convolution that is kept, first position in the
+    output, steps in the output, kept extents), all pairs. Holds the shapes and the weights, no activations."""
+
+    def __init__(self, x_shape, out_shape, parts):
+        (B, C, H, W), (_, N, ho, wo) = self.x_shape, self.out_shape = tuple(x_shape), tuple(out_shape)
+        self.parts, self._table = list(parts), None
+        if self.out_shape[0] != B:
+            raise RuntimeError("ConvPhases: input and output differ in batch")
+        for nw, _, _, _, (o0, p0), (sy, sx), (cnt_h, cnt_w) in self.parts:
+            if nw.C != C or nw.N != N or o0 < 0 or p0 < 0 or o0 + sy * (cnt_h - 1) >= ho or p0 + sx * (cnt_w - 1) >= wo:
+                raise RuntimeError("ConvPhases: a phase does not match the input or lies outside the output")
+
+    def __getstate__(self):
+        return {**self.__dict__, "_table": None}     # (addresses of this object's weights: a copy makes its own)
+
+    def table(self):
+        if self._table is None:
+            (B, C, H, W), (_, N, ho, wo) = self.x_shape, self.out_shape
+            table = (_capi.ConvPhase * len(self.parts))()
+            for e, (nw, ((pt, pb), (pl, pr)), (dy, dx), (h0, w0), (o0, p0), (sy, sx), (cnt_h, cnt_w)) in zip(table, self.parts):
+                e.shape = _capi.ConvShape(B, C, H, W, N, nw.ky, nw.kx, 1, 1, pt, pl, dy, dx, pb, pr)
+                e.view = _capi.OutputView(h0, w0, cnt_h, cnt_w, ho * wo, sy * wo, sx)
+                e.first, e.native = o0 * wo + p0, nw.buf.data_ptr()
+            self._table = table
+        return self._table
+
+    def run(self, out, x, scale, bias, residual, relu):
+        if not x.is_cuda or x.dtype != torch.float16 or tuple(x.shape) != self.x_shape or out.device != x.device or \
+                tuple(out.shape) != self.out_shape or not out.is_contiguous(memory_format=torch.channels_last):
+            raise RuntimeError("ternary_conv2d_into: input or output does not match the phases")
+        if not x.is_contiguous(memory_format=torch.channels_last):
+            x = x.contiguous(memory_format=torch.channels_last)
+        if out.numel() == 0 or not self.parts:
+            return out
+        ep = _epilogue(self.parts[0][0], scale, bias, residual, relu, out.dtype, out)
+        with _capi.on_device(x.device):
+            check(_lib().tmq_ternary_conv2d_phases(ptr(x), self.table(), len(self.parts), ctypes.byref(ep), ptr(out), stream_of(x)),
+                  "ternary_conv2d_phases")
+        return out
 
 
 def ternary_conv2d_relu_maxpool(x: torch.Tensor, nw: NativeWeights, stride=1, padding=0, dilation=1, scale=None,

@@ -981,6 +981,8 @@ class ConvTranspose2d(Conv2d):
 
     _transposed = True
 
+    _phases = None      # (phase weights, shapes, plan, empty phases) for the shapes last seen, see _phase_plan
+
     def __init__(self, in_channels, out_channels, kernel, stride=1, padding=0, output_padding=0, groups=1, bias=True,
                  dilation=1, device=None, ctrl=None, quant_mode=QuantMode.NONE, post_scale=False):
         super().__init__(in_channels, out_channels, kernel, stride, padding, groups, dilation, bias, device, ctrl,
@@ -1041,21 +1043,36 @@ class ConvTranspose2d(Conv2d):
         if x.dtype != torch.float16 or not x.is_contiguous(memory_format=torch.channels_last):
             x = x.to(dtype=torch.float16, memory_format=torch.channels_last)
         y = torch.empty((B, cout, h_out, w_out), dtype=_compact_out, device=x.device, memory_format=torch.channels_last)
+        plan, empty = self._phase_plan(tuple(x.shape), tuple(y.shape), phases, (sy, sx), (py, px))
+        for o0, p0 in empty:                                         # no tap reaches this phase: bias only
+            target = y[:, :, o0::sy, p0::sx]
+            target.zero_()
+            if bias is not None:
+                target += bias.to(y.dtype).view(1, -1, 1, 1)
+        # every phase written in place: the kernel's epilogue scatters its rows into the phase's pixels
+        return ops.ternary_conv2d_into(y, x, None, scale=scale, bias=bias, phases=plan)
+
+    def _phase_plan(self, x_shape, y_shape, phases, stride, padding):
+        """The phases of _phase_weights as convolutions of an x_shape input into a y_shape output (ops.ConvPhases), and the
+        first positions of the phases no tap reaches. The last shape's plan is kept; it holds shapes and weights only."""
+        key, last = (x_shape, y_shape), self._phases
+        if last is not None and last[0] is phases and last[1] == key:
+            return last[2], last[3]
+        (sy, sx), (py, px) = stride, padding
+        parts, empty = [], []
         for (rh, rw), (nw, geo_h, geo_w) in phases.items():
-            rows, cols = _phase_extent(rh, sy, py, h_out, H, geo_h), _phase_extent(rw, sx, px, w_out, W, geo_w)
+            rows = _phase_extent(rh, sy, py, y_shape[2], x_shape[2], geo_h)
+            cols = _phase_extent(rw, sx, px, y_shape[3], x_shape[3], geo_w)
             if rows is None or cols is None:
                 continue                                             # no output position in this phase
             (o0, cnt_h, pt, pb, skip_h), (p0, cnt_w, pl, pr, skip_w) = rows, cols
-            target = y[:, :, o0::sy, p0::sx]
-            if nw is None:                                           # no tap reaches this phase: bias only
-                target.zero_()
-                if bias is not None:
-                    target += bias.to(y.dtype).view(1, -1, 1, 1)
-                continue
-            # one launch per phase, written in place: the kernel's epilogue scatters its rows into the phase's pixels
-            ops.ternary_conv2d_into(target, x, nw, (1, 1), ((pt, pb), (pl, pr)), (geo_h[2], geo_w[2]), scale=scale, bias=bias,
-                                    first=(skip_h, skip_w))
-        return y
+            if nw is None:
+                empty.append((o0, p0))
+            else:
+                parts.append((nw, ((pt, pb), (pl, pr)), (geo_h[2], geo_w[2]), (skip_h, skip_w), (o0, p0), (sy, sx), (cnt_h, cnt_w)))
+        plan = ops.ConvPhases(x_shape, y_shape, parts)
+        self._phases = (phases, key, plan, empty)
+        return plan, empty
 
     def _phase_weights(self, cin, cout, ky, kx, sy, sx, dy, dx):
         """The transposed convolution as sy * sx ordinary stride-1 convolutions, one per phase
