@@ -10,6 +10,8 @@
 #include <ATen/hip/HIPContext.h>
 #include <c10/core/DeviceGuard.h>
 
+#include <algorithm>
+#include <array>
 #include <list>
 #include <map>
 #include <mutex>
@@ -83,19 +85,24 @@ struct Carved {
     std::vector<torch::Tensor> parts;
 };
 
+// A tensor of its own on `flat`'s storage, built without a trip through the dispatcher (two of those per tensor were
+// most of what a 21-layer step spent on the host).
+torch::Tensor on_storage(const torch::Tensor &flat, int64_t offset, at::IntArrayRef sizes, at::IntArrayRef strides) {
+    auto part = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(flat.storage()), flat.key_set(), flat.dtype());
+    part.unsafeGetTensorImpl()->set_sizes_and_strides(sizes, strides, offset);
+    return part;
+}
+
 Carved carve(const std::vector<torch::Tensor> &like) {
     int64_t total = 0;
-    std::vector<int64_t> offs;
-    for (const auto &t : like) {
-        offs.push_back(total);
-        total += (t.numel() + 63) / 64 * 64;
-    }
+    for (const auto &t : like) total += (t.numel() + 63) / 64 * 64;
     Carved c;
     c.flat = torch::empty({total}, like[0].options());
-    for (size_t i = 0; i < like.size(); i++) {
-        auto part = torch::empty({0}, like[0].options());
-        part.set_(c.flat.storage(), offs[i], like[i].sizes(), like[i].strides());
-        c.parts.push_back(part);
+    c.parts.reserve(like.size());
+    int64_t at = 0;
+    for (const auto &t : like) {
+        c.parts.push_back(on_storage(c.flat, at, t.sizes(), t.strides()));
+        at += (t.numel() + 63) / 64 * 64;
     }
     return c;
 }
@@ -464,6 +471,150 @@ torch::Tensor compress_ternary(torch::Tensor input, std::vector<int64_t> orig_sh
     return buf.narrow(0, 0, (int64_t)size).clone();
 }
 
+// ---- the plain calls of tmq_amd/ops.py ----------------------------------------------------------------------------
+// One fp32 or fp16 tensor in, one tensor out: the argument checks, output and workspace allocations and the launch of
+// ops.ternary_linear, ternary_conv2d, ternary_dwconv2d, softstep_fwd_all and softstep_bwd_all in one native call -- through
+// ctypes they cost 10 to 30 us (a 4096 x 4096 layer's row takes 3.4 us on the GPU). What is not the plain case (another
+// dtype, device, layout or shape, a route with launches in between, a failing status) gives None: the Python function
+// then does what it always did, its errors included.
+typedef c10::optional<torch::Tensor> Maybe;
+
+bool plain(const Maybe &t, const torch::Tensor &x, int64_t n) {    // a per-channel vector
+    return !t.has_value() || (t->device() == x.device() && t->scalar_type() == torch::kFloat32 && t->numel() == n && t->is_contiguous());
+}
+
+bool residual_ok(const Maybe &r, const torch::Tensor &y) {
+    if (!r.has_value()) return true;
+    if (r->device() != y.device() || r->scalar_type() != y.scalar_type() || r->sizes() != y.sizes()) return false;
+    for (int64_t d = 0; d < y.dim(); d++)
+        if (y.size(d) > 1 && r->stride(d) != y.stride(d)) return false;
+    return true;
+}
+
+tmq_epilogue epilogue_of(const Maybe &scale, const Maybe &bias, const Maybe &residual, bool relu, const torch::Tensor &y) {
+    return tmq_epilogue{scale.has_value() ? scale->data_ptr<float>() : nullptr, bias.has_value() ? bias->data_ptr<float>() : nullptr,
+                        residual.has_value() ? residual->data_ptr() : nullptr, relu ? 1 : 0,
+                        y.scalar_type() == torch::kFloat16 ? TMQ_F16 : TMQ_F32};
+}
+
+Maybe plain_linear(const torch::Tensor &x, const torch::Tensor &native, int64_t K, int64_t N, const Maybe &scale, const Maybe &bias,
+                   const Maybe &residual, bool relu, bool out_f16, bool prescale) {
+    const bool f32 = x.scalar_type() == torch::kFloat32;
+    if (!x.device().is_cuda() || native.device() != x.device() || !(f32 || x.scalar_type() == torch::kFloat16) || !x.is_contiguous() ||
+        x.dim() < 1 || K <= 0 || x.size(-1) != K || x.numel() == 0 || !plain(scale, x, N) || !plain(bias, x, N))
+        return c10::nullopt;
+    const int64_t M = x.numel() / K;
+    const c10::DeviceGuard guard(x.device());
+    size_t bytes = 0;
+    if (!f32) {
+        bytes = M > 16 && (M <= 32 || K % 64) ? tmq_ternary_linear_workspace_bytes(TMQ_F16, M, K, N) : 0;
+    } else if (!(M <= 2 && tmq_fp32_rows_self_scaled_for(x.data_ptr(), M, K, N))) {
+        if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 || (!prescale && M >= 1024 && N <= 128)) return c10::nullopt;
+        bytes = tmq_ternary_linear_workspace_bytes(TMQ_F32, M, K, N);
+        if (!bytes) return c10::nullopt;
+    }
+    auto sizes = x.sizes().vec();
+    sizes.back() = N;
+    auto y = at::empty(sizes, x.options().dtype(out_f16 ? torch::kFloat16 : torch::kFloat32));
+    if (!residual_ok(residual, y)) return c10::nullopt;
+    const tmq_epilogue ep = epilogue_of(scale, bias, residual, relu, y);
+    torch::Tensor ws;
+    if (bytes) ws = at::empty({(int64_t)bytes}, x.options().dtype(torch::kUInt8));
+    const int status = tmq_ternary_linear_ws(x.data_ptr(), f32 ? TMQ_F32 : TMQ_F16, M, K, native.data_ptr(), N, &ep, y.data_ptr(),
+                                             bytes ? ws.data_ptr() : nullptr, bytes, stream_of(x));
+    if (status != TMQ_OK) return c10::nullopt;
+    return y;
+}
+
+// words: the native weights of a dense convolution, the compact words of a depthwise one. geometry: stride, padding in
+// front, padding behind, dilation, each (y, x).
+Maybe plain_conv(const torch::Tensor &input, const torch::Tensor &words, bool depthwise, int64_t C, int64_t N, int64_t ky, int64_t kx,
+                 const std::array<int32_t, 8> &geometry, Maybe scale, const Maybe &bias, const Maybe &residual, bool relu, bool out_f16,
+                 bool prescale) {
+    torch::Tensor x = input;
+    const auto last = at::MemoryFormat::ChannelsLast;
+    const bool f32 = x.scalar_type() == torch::kFloat32;
+    if (!x.device().is_cuda() || words.device() != x.device() || !words.is_contiguous() || x.dim() != 4 || x.size(1) != C || x.numel() == 0 ||
+        !plain(scale, x, N) || !plain(bias, x, N))
+        return c10::nullopt;
+    if (depthwise && (words.scalar_type() != torch::kInt32 || words.numel() != ky * kx * ((C + 15) / 16))) return c10::nullopt;
+    const bool nhwc = x.is_contiguous(last);
+    if (f32 ? !(prescale && (nhwc || x.is_contiguous())) : !(x.scalar_type() == torch::kFloat16 && nhwc)) return c10::nullopt;
+    const int64_t B = x.size(0), H = x.size(2), W = x.size(3);
+    if (std::max({B, C, N, H, W, ky, kx}) > INT32_MAX) return c10::nullopt;
+    const auto &g = geometry;
+    const tmq_conv_shape shape = {(int32_t)B, (int32_t)C, (int32_t)H, (int32_t)W, (int32_t)N, (int32_t)ky, (int32_t)kx,
+                                  g[0], g[1], g[2], g[3], g[6], g[7], g[4], g[5]};
+    int32_t ho = 0, wo = 0;
+    if (tmq_conv2d_out_hw(&shape, &ho, &wo) != TMQ_OK || ho <= 0 || wo <= 0) return c10::nullopt;
+    const c10::DeviceGuard guard(x.device());
+    auto y = at::empty({B, N, ho, wo}, x.options().dtype(out_f16 ? torch::kFloat16 : torch::kFloat32).memory_format(last));
+    if (!residual_ok(residual, y)) return c10::nullopt;
+    torch::Tensor scratch;
+    if (f32) {
+        // one fp16 term of the activations, channels-last; the scan's partial maxima, the prescale and scale / s share a buffer
+        const int64_t n = x.numel(), part = (int64_t)tmq_f32_to_f16_prescaled_workspace_bytes(n) / 4;
+        scratch = at::empty({part + 4 + N}, x.options());
+        float *ws = scratch.data_ptr<float>();
+        auto hi = at::empty({B, C, H, W}, x.options().dtype(torch::kFloat16).memory_format(last));
+        const float *per = scale.has_value() ? scale->data_ptr<float>() : nullptr;
+        const int status = nhwc ? tmq_f32_to_f16_prescaled(x.data_ptr<float>(), n, ws + part, hi.data_ptr(), per, ws + part + 4, N, ws, stream_of(x))
+                                : tmq_f32_nchw_to_f16_nhwc_prescaled(x.data_ptr<float>(), B, C, H * W, ws + part, hi.data_ptr(), per,
+                                                                     ws + part + 4, N, ws, stream_of(x));
+        if (status != TMQ_OK) return c10::nullopt;
+        scale = scratch.narrow(0, part + 4, N);
+        x = hi;
+    }
+    const tmq_epilogue ep = epilogue_of(scale, bias, residual, relu, y);
+    const int status = depthwise ? tmq_ternary_dwconv2d(x.data_ptr(), &shape, reinterpret_cast<const uint32_t *>(words.data_ptr<int32_t>()), &ep, y.data_ptr(), stream_of(x))
+                                 : tmq_ternary_conv2d(x.data_ptr(), &shape, words.data_ptr(), &ep, y.data_ptr(), stream_of(x));
+    if (status != TMQ_OK) return c10::nullopt;
+    return y;
+}
+
+bool plain_weights(const std::vector<torch::Tensor> &ws) {
+    for (const auto &w : ws)
+        if (!w.device().is_cuda() || w.device() != ws[0].device() || w.scalar_type() != torch::kFloat32 || !w.is_contiguous()) return false;
+    return !ws.empty();
+}
+
+c10::optional<std::pair<std::vector<torch::Tensor>, Maybe>> plain_softstep_fwd(const std::vector<torch::Tensor> &ws, double digamma,
+                                                                               bool want_loss, double sharpness, double strength) {
+    if (!plain_weights(ws)) return c10::nullopt;
+    const c10::DeviceGuard guard(ws[0].device());
+    Carved ys = carve(ws);
+    std::vector<tmq_step_tensor> table(ws.size());
+    for (size_t i = 0; i < ws.size(); i++)
+        table[i] = tmq_step_tensor{ws[i].data_ptr<float>(), nullptr, ys.parts[i].data_ptr<float>(), (uint64_t)ws[i].numel()};
+    Maybe loss;
+    if (want_loss) loss = torch::empty({}, ws[0].options());
+    const int status = want_loss ? tmq_softstep_fwd_multi_inlaunch(table.data(), (int)table.size(), digamma, sharpness, strength, nullptr,
+                                                                   loss->data_ptr<float>(), loss_state(ws[0]).data_ptr(), stream_of(ws[0]))
+                                 : tmq_softstep_fwd_multi(table.data(), (int)table.size(), digamma, sharpness, strength, nullptr, nullptr,
+                                                          nullptr, stream_of(ws[0]));
+    if (status != TMQ_OK) return c10::nullopt;
+    return std::make_pair(std::move(ys.parts), loss);
+}
+
+c10::optional<std::vector<torch::Tensor>> plain_softstep_bwd(const std::vector<torch::Tensor> &ws, const std::vector<torch::Tensor> &gs,
+                                                             const Maybe &upstream, double digamma, double sharpness, double strength) {
+    if (!plain_weights(ws) || gs.size() != ws.size()) return c10::nullopt;
+    for (size_t i = 0; i < gs.size(); i++)
+        if (gs[i].device() != ws[0].device() || gs[i].scalar_type() != torch::kFloat32 || gs[i].numel() != ws[i].numel() || !gs[i].is_contiguous())
+            return c10::nullopt;
+    if (upstream.has_value() && (upstream->device() != ws[0].device() || upstream->scalar_type() != torch::kFloat32 || upstream->numel() != 1))
+        return c10::nullopt;
+    const c10::DeviceGuard guard(ws[0].device());
+    Carved dws = carve(ws);
+    std::vector<tmq_step_tensor> table(ws.size());
+    for (size_t i = 0; i < ws.size(); i++)
+        table[i] = tmq_step_tensor{ws[i].data_ptr<float>(), gs[i].data_ptr<float>(), dws.parts[i].data_ptr<float>(), (uint64_t)ws[i].numel()};
+    if (tmq_softstep_bwd_multi(table.data(), (int)table.size(), digamma, sharpness, strength,
+                               upstream.has_value() ? upstream->data_ptr<float>() : nullptr, stream_of(ws[0])) != TMQ_OK)
+        return c10::nullopt;
+    return std::move(dws.parts);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -480,6 +631,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     // additive: all layers of a training step in one launch
     m.def("softstep_fwd_all", &softstep_fwd_all);
     m.def("softstep_bwd_all", &softstep_bwd_all);
+    // additive: the plain calls of tmq_amd/ops.py
+    m.def("plain_linear", &plain_linear);
+    m.def("plain_conv", &plain_conv);
+    m.def("plain_softstep_fwd", &plain_softstep_fwd);
+    m.def("plain_softstep_bwd", &plain_softstep_bwd);
     // tmq_native (tmq/tmq_native.cpp:550-555)
     m.def("compactify_ternary", &compactify_ternary);
     m.def("compress_ternary", &compress_ternary);

@@ -266,6 +266,10 @@ def softstep_fwd_all(weights, digamma: float, want_loss: bool = False, sharpness
     layer of a model, tmq/tmq.py:404-419) and, with want_loss, the total quantization loss
     sum_l mean(q(w_l; sharpness, strength)) (tmq/tmq.py:298-310) from the same pass over the weights.
     Returns (list of y, 0-dim fp32 loss or None)."""
+    if ext is not None:
+        out = ext.plain_softstep_fwd(weights, digamma, want_loss, sharpness, strength)
+        if out is not None:
+            return out
     ws, dev = _step_weights(weights, "softstep_fwd_all")
     offs, total = _flat_offsets(ws)
     flat = torch.empty(total, dtype=torch.float32, device=dev)
@@ -297,6 +301,10 @@ def softstep_bwd_all(weights, grads, loss_upstream, digamma: float, sharpness: f
     the two). grads[l] may be None (no gradient reached y_l), loss_upstream (one fp32 GPU value u, the
     gradient arriving at the total quantization loss) may be None; a tensor that gets neither term
     yields None."""
+    if ext is not None and all(g is not None for g in grads):
+        out = ext.plain_softstep_bwd(weights, grads, loss_upstream, digamma, sharpness, strength)
+        if out is not None:
+            return out
     ws, dev = _step_weights(weights, "softstep_bwd_all")
     if len(grads) != len(ws):
         raise ValueError("softstep_bwd_all: one gradient (or None) per tensor")
@@ -541,6 +549,7 @@ def _epilogue(nw, scale, bias, residual, relu, out_dtype, y):
     return ep
 
 
+_OUT_DTYPES = (torch.float32, torch.float16)
 _fp32_prescale = True
 
 
@@ -626,6 +635,10 @@ def f32_to_f16_prescaled(x: torch.Tensor, scale, channels: int, channels_last: b
 def ternary_linear(x: torch.Tensor, nw: NativeWeights, scale=None, bias=None, residual=None, relu=False,
                    out_dtype=torch.float32) -> torch.Tensor:
     """y[..., n] = relu?(scale[n] * sum_k x[..., k] T[k][n] + bias[n] + residual); x fp16 or fp32."""
+    if ext is not None and out_dtype in _OUT_DTYPES:
+        y = ext.plain_linear(x, nw.buf, nw.K, nw.N, scale, bias, residual, bool(relu), out_dtype == torch.float16, _fp32_prescale)
+        if y is not None:
+            return y
     _capi.require_gpu(x, "activations")
     if x.dtype not in (torch.float16, torch.float32):
         raise RuntimeError("ternary_linear: activations must be fp16 or fp32")
@@ -730,6 +743,11 @@ def ternary_conv2d(x: torch.Tensor, nw: NativeWeights, stride=1, padding=0, dila
     (sy, sx), (py, px), (dy, dx) = pair(stride), pair(padding), pair(dilation)
     # padding may also be ((top, bottom), (left, right))
     (py, py_end), (px, px_end) = pair(py), pair(px)
+    if ext is not None and out_dtype in _OUT_DTYPES:
+        y = ext.plain_conv(x, nw.buf, False, nw.C, nw.N, nw.ky, nw.kx, (sy, sx, py, px, py_end, px_end, dy, dx), scale, bias, residual,
+                           bool(relu), out_dtype == torch.float16, _fp32_prescale)
+        if y is not None:
+            return y
     if not x.is_cuda or x.dim() != 4:
         raise RuntimeError("ternary_conv2d: expected a 4-D GPU tensor")
     if x.shape[1] != nw.C:
@@ -936,6 +954,11 @@ def ternary_dwconv2d(x: torch.Tensor, words: torch.Tensor, kernel, stride=1, pad
     if not x.is_cuda or x.dim() != 4:
         raise RuntimeError("ternary_dwconv2d: expected a 4-D GPU tensor")
     B, C, H, W = x.shape
+    if ext is not None and out_dtype in _OUT_DTYPES:
+        y = ext.plain_conv(x, words, True, C, C, ky, kx, (sy, sx, py, px, py_end, px_end, dy, dx), scale, bias, residual, bool(relu),
+                           out_dtype == torch.float16, _fp32_prescale)
+        if y is not None:
+            return y
     _capi.require_gpu(words, "words")
     if words.dtype != torch.int32 or words.numel() != ky * kx * ((C + 15) // 16):
         raise RuntimeError("ternary_dwconv2d: expected the int32 compact words of a [C, 1, ky, kx] weight tensor")

@@ -586,7 +586,9 @@ class TMQLayer:
         the layer's bias, then the affine map of a folded BatchNorm (fold_batchnorm) on top:
         bn(ps * acc + b) = (g * ps) * acc + (g * b + h)."""
         scale = self._epilogue_scale(n, device)
-        bias = self.bias.data.float() if getattr(self, "bias", None) is not None else None
+        bias = getattr(self, "bias", None)
+        if bias is not None:
+            bias = bias.data if bias.dtype == torch.float32 else bias.data.float()
         if self._fold is None:
             return scale, bias
         g, h = self._fold
@@ -673,7 +675,6 @@ class Linear(nn.Module, TMQLayer):
 
     forward_wrap = forward
 
-    @torch.no_grad()
     def compact_forward(self, x, residual=None, relu=False):
         """Inference straight from the 2-bit packed weights (tmq/tmq.py:662-688), any batch shape.
         residual / relu: added / applied in the kernel's epilogue (fuse_epilogues)."""
@@ -682,15 +683,21 @@ class Linear(nn.Module, TMQLayer):
         self._update_scale()
         if x.dim() == 4:
             assert x.shape[1] == 1, "Illegal shape supplied"
-        nw = self._native_weights()
-        xin = x if x.is_contiguous() else x.contiguous()
-        scale, bias = self._epilogue(nw.N, x.device)
         if (residual is not None or relu) and self.bn is not None:
             raise RuntimeError("compact_forward: the layer's own BatchNorm comes between the product and the fused epilogue")
-        if residual is not None:
-            residual = residual.to(_compact_out).contiguous()
-        out = ops.ternary_linear(xin, nw, scale=scale, bias=bias, residual=residual, relu=relu, out_dtype=_compact_out)
-        return self.bn(out) if self.bn is not None else out
+        # (nothing below records for autograd but the layer's own BatchNorm and the folded one: a kernel's output has no history)
+        if self.bn is None and self._fold is None and residual is None and x.is_contiguous():
+            return self._compact_product(x, None, relu)
+        with torch.no_grad():
+            if residual is not None:
+                residual = residual.to(_compact_out).contiguous()
+            out = self._compact_product(x if x.is_contiguous() else x.contiguous(), residual, relu)
+            return self.bn(out) if self.bn is not None else out
+
+    def _compact_product(self, x, residual, relu):
+        nw = self._native_weights()
+        scale, bias = self._epilogue(nw.N, x.device)
+        return ops.ternary_linear(x, nw, scale=scale, bias=bias, residual=residual, relu=relu, out_dtype=_compact_out)
 
     @classmethod
     def from_linear(cls, source: nn.Linear, name: str, ctrl: QuantizationControl):
