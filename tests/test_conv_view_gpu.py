@@ -183,3 +183,32 @@ def test_phases_in_one_launch_equal_one_launch_each(cuda, cin, cout, k, stride, 
     assert torch.equal(one, each)
     with pytest.raises(RuntimeError):
         ops.ternary_conv2d_into(each[:, :, :-1], x, None, phases=plan)
+
+
+@pytest.mark.parametrize("B,C,hw,N,k", [
+    (1, 64, (41, 50), 70, 1),          # short reduction: 64 x 128 tiles, a ragged last tile in rows and columns
+    (1, 64, (116, 127), 200, 1),       # 460 of them in whole 256 columns: 64 x 256
+    (1, 128, (190, 100), 300, 1),      # an odd number of 128s
+    (1, 64, (86, 96), 128, 3),         # 129 tiles at K = 576, where the split reduction ends: 64 x 128 solo
+    (1, 64, (129, 128), 100, 3),       # 258 tiles, N <= 128: dma at K = 576 ...
+    (1, 128, (129, 128), 128, 3),      # ... solo at K = 1152
+    (1, 128, (96, 121), 130, 3),       # 129 .. 256 columns, 364 tiles: 64 x 128 solo
+    (1, 64, (82, 81), 300, 3),         # three 128s: solo up to 512 tiles ...
+    (1, 64, (107, 109), 300, 3),       # ... dma beyond
+    (1, 64, (71, 73), 400, 3)])        # four 128s: 64 x 256
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_wide_tiles_at_their_edges(cuda, B, C, hw, N, k, dtype):
+    """Convolutions with more than 64 outputs on the tiles of 64 x 128 and 64 x 256, each rule of their choice once,
+    against F.conv2d: small integers, so every sum is exact (fp16 results: below 2^11)."""
+    from tmq_amd import ops
+    g = torch.Generator(device=cuda).manual_seed(C + N + k)
+    Wt = torch.randint(-1, 2, (N, C, k, k), device=cuda, generator=g).float()
+    nw = ops.NativeWeights(ops.compactify_ternary(Wt), N, conv_kernel=(k, k))
+    x = torch.randint(-2, 3, (B, C) + hw, device=cuda, generator=g).half().contiguous(memory_format=torch.channels_last)
+    bias = torch.randint(-4, 5, (N,), device=cuda, generator=g).float()
+    res = torch.randint(-9, 10, (B, N) + hw, device=cuda, generator=g).to(dtype).contiguous(memory_format=torch.channels_last)
+    want = F.conv2d(x.cpu().float(), Wt.cpu(), bias.cpu(), 1, k // 2)
+    assert want.abs().max() < 2000
+    assert torch.equal(ops.ternary_conv2d(x, nw, 1, k // 2, 1, bias=bias, out_dtype=dtype).cpu().float(), want)
+    got = ops.ternary_conv2d(x, nw, 1, k // 2, 1, bias=bias, residual=res, relu=True, out_dtype=dtype)
+    assert torch.equal(got.cpu().float(), torch.relu(want + res.cpu().float()))

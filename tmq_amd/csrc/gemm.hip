@@ -1275,8 +1275,9 @@ int conv_plan(const tmq_conv_shape *s, const tmq_output_view *view, int32_t &ho,
     return TMQ_OK;
 }
 
-// The convolutions of tmq_ternary_conv2d_phases, kPhases to a launch. 64 x 64 tiles up to 64 channels, 128 x 128 (register
-// loaders: of 64 x 64 per wavefront) beyond where that gives every CU one, all phases counted together. Against one launch
+// The convolutions of tmq_ternary_conv2d_phases, kPhases to a launch. 64 x 64 tiles up to 64 channels, 64 x 128 beyond
+// (512 -> 256 on 14 x 14, batch 8: 17.8 us against 20.8 on 128 x 128 tiles); register loaders 128 x 128 beyond, where that
+// gives every CU one, all phases counted together. Against one launch
 // per phase, which few tiles sent to the split-reduction kernel -- 4 x 4 / 2 in fp16, one image or a batch: 128 -> 64
 // channels on 56 x 56, batch 32 61.7 -> 44.3 us; 256 -> 128 on 28 x 28, batch 16 41.9 -> 21.4; 64 -> 64 on 32 x 32, batch 8
 // 21.2 -> 7.9; 100 -> 64 on 28 x 28, batch 8 50.4 -> 16.6; 32 -> 32 on 56 x 56, batch 8 23.9 -> 9.6; 128 -> 64 on one 14 x 14
@@ -1288,7 +1289,7 @@ int conv_phases(const _Float16 *x, const tmq_conv_phase *phases, int count, cons
         PhaseSet<Loader, ViewEpilogue> set{};
         set.N = N;
         set.Nb = native_blocks_n(N);
-        int64_t wide = 0, longest = 0;
+        [[maybe_unused]] int64_t squares = 0, longest = 0;          // 128 x 128 tiles; the longest reduction
         for (int q = first; q < count && q < first + kPhases; q++) {
             const tmq_conv_phase &p = phases[q];
             const tmq_conv_shape &s = p.shape;
@@ -1309,21 +1310,58 @@ int conv_phases(const _Float16 *x, const tmq_conv_phase *phases, int count, cons
             const unsigned char *res = e.residual ? static_cast<const unsigned char *>(e.residual) + p.first * N * elt : nullptr;
             ph.ep = ViewEpilogue{e.scale, e.bias, res, static_cast<unsigned char *>(y) + p.first * N * elt, e.relu,
                                  e.y_dtype == TMQ_F16 ? 1 : 0, map};
-            wide += ((M + 127) / 128) * ((N + 127) / 128);
+            squares += ((M + 127) / 128) * ((N + 127) / 128);
             if (K > longest) longest = K;
         }
         if (set.count == 0) continue;
         int rc;
         if constexpr (Loader::kDirect) {
-            rc = N > 64 && wide >= 256 ? launch_phases<8, 2, 1, 4, 1>(set, stream) : launch_phases<4, 2, 1, 2, 1>(set, stream);
+            rc = N > 64 ? launch_phases<4, 2, 1, 4, 1>(set, stream) : launch_phases<4, 2, 1, 2, 1>(set, stream);
         } else {
             const bool deep = longest >= 16 * kBK;                 // prefetch depth as in dispatch_tile
-            if (N > 64 && wide >= 256) rc = deep ? launch_phases<4, 4, 2, 2, 2>(set, stream) : launch_phases<4, 4, 2, 2, 1>(set, stream);
+            if (N > 64 && squares >= 256) rc = deep ? launch_phases<4, 4, 2, 2, 2>(set, stream) : launch_phases<4, 4, 2, 2, 1>(set, stream);
             else rc = deep ? launch_phases<4, 2, 1, 2, 2>(set, stream) : launch_phases<4, 2, 1, 2, 1>(set, stream);
         }
         if (rc) return rc;
     }
     return TMQ_OK;
+}
+
+// Tiles of 64 rows x 128 or 256 columns for convolutions over a multiple of 64 channels with more than 64 outputs: an
+// im2col tile is fetched once per 128 (256) columns instead of once per 64, and half as many rows per workgroup as in a
+// 128 x 128 tile leave fewer CUs idle in the last wave. Where the line lies, from a sweep over N = 96 .. 512, 64 .. 512
+// channels, 1 x 1 and 3 x 3, 4096 .. 65536 rows (fp16 out, residual and ReLU; what took the shape before = 1):
+//   reductions below 512                            64 x 128 dma   0.76 .. 0.98
+//     ... in whole 256 columns, 448 .. 1100 tiles   64 x 256 solo  0.77 .. 0.93 (64 x 128: 0.80 .. 0.97)
+//     ... in whole 256 columns, more tiles          the old choice (64 x 128: 0.92 .. 0.98, but up to 1.19 into fp32)
+//   up to 512 tiles of 64 x 64 (split reduction)    64 x 128 solo  0.83 .. 0.89 from 192 tiles on up to K = 1536 (K = 4608: 0.97 .. 1.03;
+//                                                   128 tiles: 0.89 .. 0.95 at K <= 640, 1.05 at 1152, 1.2 at 2304)
+//   more of them: N <= 128, up to 512 tiles         0.82 .. 0.89 (dma to K = 768, then solo; 1024 tiles: 0.96 .. 1.04)
+//   129 .. 256                                      64 x 128 solo 0.94 below 448 tiles from K = 1024 on (K = 512: 1.07), else
+//                                                   64 x 256 solo as before
+//   an odd number of 128s (256-wide tiles waste)    solo 0.86 .. 0.94 up to 512 tiles, dma 0.79 .. 0.93 beyond
+//   other widths, up to 1100 tiles                  64 x 256 solo 0.79 .. 1.00
+// 128 -> 128, 3 x 3 on 28 x 28, batch 32: 14.7 -> 13.7 us; 320 -> 76, 1 x 1 on 54 x 54, batch 34: 23.9 -> 18.4.
+enum class WideTile { kNone, kDma128, kSolo128, kSolo256 };
+WideTile wide_tile(int64_t M, int64_t K, int64_t N) {
+    if (N <= 64) return WideTile::kNone;
+    const int64_t tm = (M + 63) / 64, t64 = tm * ((N + 63) / 64), n128 = (N + 127) / 128, t = tm * n128;
+    const bool whole256 = n128 % 2 == 0;
+    if (K < 512) {
+        if (t64 <= K / 2) return WideTile::kNone;                  // the split reduction's
+        return !whole256 || t < 448 ? WideTile::kDma128 : t <= 1100 ? WideTile::kSolo256 : WideTile::kNone;
+    }
+    if (t64 <= 512)
+        return (t >= 192 && K <= 1536) || (t >= 128 && t64 >= 256 && K <= 640) ? WideTile::kSolo128 : WideTile::kNone;
+    if (n128 == 1) return t > 512 ? WideTile::kNone : K <= 768 ? WideTile::kDma128 : WideTile::kSolo128;
+    if (n128 == 2) return t < 448 && K >= 1024 ? WideTile::kSolo128 : WideTile::kSolo256;
+    if (!whole256) return t <= 512 ? WideTile::kSolo128 : WideTile::kDma128;
+    return t <= 1100 ? WideTile::kSolo256 : WideTile::kNone;
+}
+// What those tiles' loader takes.
+bool wide_conv_ok(const void *x, const tmq_conv_shape *s, int64_t M) {
+    return s->C % kBK == 0 && s->ky <= 15 && s->kx <= 15 && aligned16(x) && (int64_t)s->B * s->H * s->W * s->C < (int64_t)0x7FFFFFF0 &&
+           M < (int64_t)0x7FFFFFFF;
 }
 
 // The tile kernels behind tmq_ternary_conv2d for an epilogue with consecutive rows (Epilogue) or rows scattered into a
@@ -1333,17 +1371,16 @@ int conv_tiles(const void *x, const tmq_conv_shape *s, int ho, int wo, const voi
     const int64_t M = (int64_t)s->B * ho * wo, K = (int64_t)s->C * s->ky * s->kx;
     const _Float16 *xp = static_cast<const _Float16 *>(x);
     const bool small = (int64_t)s->B * s->H * s->W * s->C < (int64_t)0x7FFFFFF0 && M < (int64_t)0x7FFFFFFF;   // 32-bit offsets and rows
-    // 129 .. 256 output channels over at least 128 tiles of 64 rows: one 64 x 256 tile per workgroup, eight
-    // wavefronts of 64 rows x 32 channels -- an im2col tile is then fetched once instead of once per 64 channels
-    // (the four such 3 x 3 convolutions of ResNet-18 at batch 64: 18.9 / 25.8 / 23.3 / 23.2 -> 14.4 / 21.4 / 21.3 / 22.0 us;
-    // the 1 x 1 downsample beside them, two k-tiles, is faster on the small tiles: 5.4 against 7.9 us)
-    if ((s->C % kBK == 0) && s->ky <= 15 && s->kx <= 15 && aligned16(x) && small && s->N > 128 && s->N <= 256 && M >= 128 * 64 && K >= 8 * kBK)
-        return launch_tile_solo<4, 2, 1, 8, 1>(with_divisors(ConvLoader64{xp, M, K, s->B, s->C, s->H, s->W, ho, wo, s->ky, s->kx,
-                                                                          s->sy, s->sx, s->py, s->px, s->dy, s->dx, {}, {}}),
-                                               native, M, K, s->N, ep, stream);
-    if ((s->C % kBK == 0) && s->ky <= 15 && s->kx <= 15 && aligned16(x) && small)
-        return dispatch_tile(with_divisors(ConvLoader64{xp, M, K, s->B, s->C, s->H, s->W, ho, wo, s->ky, s->kx, s->sy,
-                                                        s->sx, s->py, s->px, s->dy, s->dx, {}, {}}), native, M, K, s->N, ep, stream);
+    if (wide_conv_ok(x, s, M)) {
+        const auto ld = with_divisors(ConvLoader64{xp, M, K, s->B, s->C, s->H, s->W, ho, wo, s->ky, s->kx, s->sy, s->sx, s->py, s->px,
+                                                   s->dy, s->dx, {}, {}});
+        switch (wide_tile(M, K, s->N)) {
+            case WideTile::kDma128: return launch_tile_dma<4, 2, 1, 4, 1>(ld, native, M, K, s->N, ep, stream);
+            case WideTile::kSolo128: return launch_tile_solo<4, 2, 1, 4, 2>(ld, native, M, K, s->N, ep, stream);
+            case WideTile::kSolo256: return launch_tile_solo<4, 2, 1, 8, 1>(ld, native, M, K, s->N, ep, stream);
+            case WideTile::kNone: return dispatch_tile(ld, native, M, K, s->N, ep, stream);
+        }
+    }
     if ((s->C == 8 || s->C == 16 || s->C == 32) && aligned16(x) && small)
         return dispatch_tile(with_divisors(ConvLoaderFewC{xp, M, K, s->B, s->C, s->H, s->W, ho, wo, s->ky, s->kx, s->sy,
                                                           s->sx, s->py, s->px, s->dy, s->dx, {}, {}}), native, M, K, s->N, ep, stream);
@@ -1477,7 +1514,8 @@ int tmq_ternary_conv2d_view(const void *x, const tmq_conv_shape *s, const void *
     if (M == 0 || (view && (view->h_cnt == 0 || view->w_cnt == 0))) return TMQ_OK;
     const int y_f16 = y_dtype == TMQ_F16 ? 1 : 0;
     // few output tiles: split the reduction inside the workgroup (mid.hip)
-    if (mid_conv_ok(x, s) && split_reduction_pays(M, K, s->N))
+    if (mid_conv_ok(x, s) && split_reduction_pays(M, K, s->N) &&
+        !(wide_conv_ok(x, s, M) && wide_tile(M, K, s->N) != WideTile::kNone))
         return launch_mid_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, view ? &map : nullptr, stream);
     if (view) return conv_tiles(x, s, ho, wo, native, ViewEpilogue{scale, bias, residual, y, relu, y_f16, map}, stream);
     return conv_tiles(x, s, ho, wo, native, Epilogue{scale, bias, residual, y, relu, y_f16, {}}, stream);
