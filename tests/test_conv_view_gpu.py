@@ -195,7 +195,10 @@ def test_phases_in_one_launch_equal_one_launch_each(cuda, cin, cout, k, stride, 
     (1, 128, (96, 121), 130, 3),       # 129 .. 256 columns, 364 tiles: 64 x 128 solo
     (1, 64, (82, 81), 300, 3),         # three 128s: solo up to 512 tiles ...
     (1, 64, (107, 109), 300, 3),       # ... dma beyond
-    (1, 64, (71, 73), 400, 3)])        # four 128s: 64 x 256
+    (1, 64, (71, 73), 400, 3),         # four 128s: 64 x 256
+    (2, 64, (97, 95), 32, 3),          # at most 32 columns: 128 x 32 tiles, a ragged last one, direct loads ...
+    (3, 16, (31, 33), 17, 5), (1, 104, (40, 41), 24, 3),     # ... of few channels, through registers
+    (1, 136, (19, 21), 30, 3), (2, 17, (15, 16), 5, 3)])     # (reduction of 1224: deeper prefetch; single elements)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_wide_tiles_at_their_edges(cuda, B, C, hw, N, k, dtype):
     """Convolutions with more than 64 outputs on the tiles of 64 x 128 and 64 x 256, each rule of their choice once,

@@ -1050,6 +1050,14 @@ template <class Loader, class Ep>
 int dispatch_tile(const Loader &ld, const void *native, int64_t M, int64_t K, int64_t N, const Ep &ep,
                   void *stream) {
     auto wgs = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    // At most 32 columns: 128 x 32 tiles, four wavefronts of 32 rows each, where a 64 x 64 tile's second wavefront would
+    // multiply columns that don't exist. Convolutions into 16, 24 and 32 channels against 64 x 64 tiles (rows 784 .. 50176):
+    // 64 -> 32, 3 x 3 on 56 x 56, batch 16 10.1 -> 8.6 us; 16 -> 16, 5 x 5 9.1 -> 7.9; 104 -> 24, 3 x 3 18.3 -> 16.3; 256 -> 16,
+    // 1 x 1 on 28 x 28, batch 16 5.8 -> 5.1; 0.85 .. 0.98 throughout, 17 -> 32 (single elements) 0.95 .. 1.02.
+    if (N <= 32) {
+        if constexpr (Loader::kDirect) return launch_tile_dma<2, 2, 4, 1, 1>(ld, native, M, K, N, ep, stream);
+        else return K >= 16 * kBK ? launch_tile<2, 2, 4, 1, 2>(ld, native, M, K, N, ep, stream) : launch_tile<2, 2, 4, 1, 1>(ld, native, M, K, N, ep, stream);
+    }
     if constexpr (Loader::kDirect) {
         // Tiles per pass: two (half the barriers, a whole extra tile of time for the loads to land) pay
         // on long reductions when the doubled ring does not cost residency -- the 128 x 256 tile, which
@@ -1316,10 +1324,12 @@ int conv_phases(const _Float16 *x, const tmq_conv_phase *phases, int count, cons
         if (set.count == 0) continue;
         int rc;
         if constexpr (Loader::kDirect) {
-            rc = N > 64 ? launch_phases<4, 2, 1, 4, 1>(set, stream) : launch_phases<4, 2, 1, 2, 1>(set, stream);
+            rc = N > 64 ? launch_phases<4, 2, 1, 4, 1>(set, stream) : N > 32 ? launch_phases<4, 2, 1, 2, 1>(set, stream)
+                                                                             : launch_phases<2, 2, 4, 1, 1>(set, stream);
         } else {
             const bool deep = longest >= 16 * kBK;                 // prefetch depth as in dispatch_tile
-            if (N > 64 && squares >= 256) rc = deep ? launch_phases<4, 4, 2, 2, 2>(set, stream) : launch_phases<4, 4, 2, 2, 1>(set, stream);
+            if (N <= 32) rc = deep ? launch_phases<2, 2, 4, 1, 2>(set, stream) : launch_phases<2, 2, 4, 1, 1>(set, stream);
+            else if (N > 64 && squares >= 256) rc = deep ? launch_phases<4, 4, 2, 2, 2>(set, stream) : launch_phases<4, 4, 2, 2, 1>(set, stream);
             else rc = deep ? launch_phases<4, 2, 1, 2, 2>(set, stream) : launch_phases<4, 2, 1, 2, 1>(set, stream);
         }
         if (rc) return rc;
