@@ -145,3 +145,36 @@ def test_missing_library_fails_loudly(tmp_path, monkeypatch):
     monkeypatch.setattr(_capi, "LIB_PATH", str(tmp_path / "nope.so"))
     with pytest.raises(ImportError, match="no CPU or PyTorch fallback"):
         _capi.load()
+
+
+def _phase_parts(layer, hw):
+    """The parts of the plan that layer makes for a [1, 2, hw, hw] input, its sub-kernels stood in for by their shapes."""
+    from types import SimpleNamespace
+    ky, kx = layer.kernel
+    (s, _), (p, _), o = layer.stride, layer.padding, layer.output_padding
+    weights = layer.__dict__.setdefault("_test_phases", {})
+    if not weights:
+        for rh in range(s):
+            for rw in range(s):
+                th, tw = len(range(rh, ky, s)), len(range(rw, kx, s))
+                nw = SimpleNamespace(C=2, N=3, ky=th, kx=tw) if th and tw else None
+                weights[(rh, rw)] = (nw, (th, max(th - 1, 0), 1), (tw, max(tw - 1, 0), 1))
+    out = (hw - 1) * s - 2 * p + ky + o[0]
+    plan, empty = layer._phase_plan((1, 2, hw, hw), (1, 3, out, out), weights, layer.stride, layer.padding)
+    return out, plan.parts, empty
+
+
+def test_phase_plan_follows_the_padding():
+    """A transposed layer whose padding changes while the output keeps its size (3 x 3 / 3 on 8 x 8, padding and output
+    padding from 0, 0 to 1, 2) plans its phases anew: the plan a fresh layer makes, with other first positions."""
+    t = _tmq()
+    make = lambda p, o: t.ConvTranspose2d(2, 3, (3, 3), (3, 3), (p, p), (o, o), bias=False, ctrl=t.QuantizationControl())
+    layer, fresh = make(0, 0), make(1, 2)
+    before = _phase_parts(layer, 8)
+    again = _phase_parts(layer, 8)
+    assert again[1] is before[1]                              # kept for the shape and padding last seen
+    layer.padding, layer.output_padding = (1, 1), (2, 2)
+    fresh._test_phases = layer._test_phases
+    after, want = _phase_parts(layer, 8), _phase_parts(fresh, 8)
+    assert before[0] == after[0] == 24
+    assert after[1] == want[1] and after[2] == want[2] and after[1] != before[1]

@@ -215,3 +215,19 @@ def test_wide_tiles_at_their_edges(cuda, B, C, hw, N, k, dtype):
     assert torch.equal(ops.ternary_conv2d(x, nw, 1, k // 2, 1, bias=bias, out_dtype=dtype).cpu().float(), want)
     got = ops.ternary_conv2d(x, nw, 1, k // 2, 1, bias=bias, residual=res, relu=True, out_dtype=dtype)
     assert torch.equal(got.cpu().float(), torch.relu(want + res.cpu().float()))
+
+
+def test_transposed_layer_follows_a_change_of_padding(cuda):
+    """Padding and output padding set anew on a layer that has planned its phases, the output keeping its size."""
+    import tmq_amd as t
+    torch.manual_seed(5)
+    net = torch.nn.Sequential(torch.nn.ConvTranspose2d(8, 7, 3, 3, 0, bias=False))
+    t.quantize_model(net, t.QuantizationControl())
+    net.to(cuda).eval()
+    w = torch.randint(-1, 2, net[0].weight.shape, device=cuda).float()
+    net[0].weight.data = w
+    t.compressed_state_dict(net)
+    x = torch.randint(-3, 4, (2, 8, 8, 8), device=cuda).half()
+    for pad, opad in ((0, 0), (1, 2), (0, 0)):
+        net[0].padding, net[0].output_padding = (pad, pad), (opad, opad)
+        assert torch.equal(net(x).cpu(), F.conv_transpose2d(x.cpu().float(), w.cpu(), None, 3, pad, opad))

@@ -988,7 +988,7 @@ class ConvTranspose2d(Conv2d):
 
     _transposed = True
 
-    _phases = None      # (phase weights, shapes, plan, empty phases) for the shapes last seen, see _phase_plan
+    _phases = None      # (phase weights, shapes and geometry, plan, empty phases) of the last call, see _phase_plan
 
     def __init__(self, in_channels, out_channels, kernel, stride=1, padding=0, output_padding=0, groups=1, bias=True,
                  dilation=1, device=None, ctrl=None, quant_mode=QuantMode.NONE, post_scale=False):
@@ -1061,8 +1061,9 @@ class ConvTranspose2d(Conv2d):
 
     def _phase_plan(self, x_shape, y_shape, phases, stride, padding):
         """The phases of _phase_weights as convolutions of an x_shape input into a y_shape output (ops.ConvPhases), and the
-        first positions of the phases no tap reaches. The last shape's plan is kept; it holds shapes and weights only."""
-        key, last = (x_shape, y_shape), self._phases
+        first positions of the phases no tap reaches. The last plan is kept, for these shapes, stride and padding (attributes
+        a caller may change between calls); it holds shapes and weights only."""
+        key, last = (x_shape, y_shape, stride, padding), self._phases
         if last is not None and last[0] is phases and last[1] == key:
             return last[2], last[3]
         (sy, sx), (py, px) = stride, padding
