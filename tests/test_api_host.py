@@ -178,3 +178,19 @@ def test_phase_plan_follows_the_padding():
     after, want = _phase_parts(layer, 8), _phase_parts(fresh, 8)
     assert before[0] == after[0] == 24
     assert after[1] == want[1] and after[2] == want[2] and after[1] != before[1]
+
+
+def test_phase_plan_goes_with_the_native_weights():
+    """invalidate_native() and loading a state let go of the phase plan too, and with it of the sub-kernels it holds."""
+    import weakref
+    t = _tmq()
+    layer = t.ConvTranspose2d(2, 3, (3, 3), (3, 3), (0, 0), (0, 0), bias=False, ctrl=t.QuantizationControl())
+    for drop in (layer.invalidate_native,
+                 lambda: layer._adopt_stored_weight({}, "", {"tmq.quant": layer.quantization.value, "tmq.tensor_type": layer.tensor_type.value,
+                                                             "tmq.shape": layer.original_shape})):
+        layer.__dict__.pop("_test_phases", None)
+        _phase_parts(layer, 8)
+        held = weakref.ref(layer._phases[2])
+        layer._native = ("key", layer.__dict__.pop("_test_phases"))
+        drop()
+        assert layer._native is None and layer._phases is None and held() is None

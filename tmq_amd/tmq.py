@@ -619,7 +619,7 @@ class TMQLayer:
                 self.compact = False
             self.quantization = QuantMode(local_metadata["tmq.quant"])
             self.training = False if self.compact else self.training
-            self._native = None
+            self.invalidate_native()
         else:
             self.compact = False
 
@@ -1059,6 +1059,10 @@ class ConvTranspose2d(Conv2d):
         # every phase written in place: the kernel's epilogue scatters its rows into the phase's pixels
         return ops.ternary_conv2d_into(y, x, None, scale=scale, bias=bias, phases=plan)
 
+    def invalidate_native(self):
+        super().invalidate_native()
+        self._phases = None                                          # holds the sub-kernels too
+
     def _phase_plan(self, x_shape, y_shape, phases, stride, padding):
         """The phases of _phase_weights as convolutions of an x_shape input into a y_shape output (ops.ConvPhases), and the
         first positions of the phases no tap reaches. The last plan is kept, for these shapes, stride and padding (attributes
@@ -1210,7 +1214,7 @@ def compressed_state_dict(module: nn.Module, strong=False, remove_prefix=""):
             layer._stream_device = layer.weight.device
             layer.weight = nn.Parameter(stream, requires_grad=False)
             layer.tensor_type = TensorType.COMPRESSED_TERNARY_32BIT
-        layer._native = None
+        layer.invalidate_native()
     state = module.state_dict()
     for full, _, _, layer in _tmq_layers(module):
         layer.compact_inference_mode()
@@ -1628,5 +1632,5 @@ def expand_compact_layers(module: nn.Module, for_training=False):
                 sub.weight = nn.Parameter(full, requires_grad=for_training)
                 sub.tensor_type = TensorType.FLOAT_32BIT
                 sub.compact = False
-                sub._native = None
+                sub.invalidate_native()
         expand_compact_layers(sub, for_training)
