@@ -234,6 +234,69 @@ def test_graph_replays_equal_eager(cuda):
         assert eager.item() == loss0.item()
 
 
+def test_one_registry_of_accumulators(cuda, monkeypatch):
+    """Every entry point that finishes a loss inside its launch takes the same buffer for a device and stream: a stream
+    that one of them has warmed needs nothing from a later capture of another."""
+    from tmq_amd import ops
+    ws = [torch.from_numpy(_inputs(n, 40 + i)[0]).to(cuda) for i, n in enumerate([9408, 36864, 2049])]
+    table = ops.SegmentTable(ws)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want, = ops.qloss_multi(table, 5.0, 5e-4)[1].tolist()          # warms the stream
+        state = ops.loss_state(cuda)
+        assert state.data_ptr() == ops.ext.loss_state(state.device.index).data_ptr()
+        asked = []
+        monkeypatch.setattr(ops, "loss_state", lambda device: asked.append(ops.ext.loss_state(torch.cuda.current_device())) or asked[-1])
+        with torch.cuda.graph(graph, stream=side):
+            _, loss = ops.softstep_fwd_all(ws, 2.236133, True, 5.0, 5e-4)
+            _, per = ops.qloss_multi(table, 5.0, 5e-4)
+        assert asked[0].data_ptr() == state.data_ptr()
+        eager, = ops.qloss_multi(table, 5.0, 5e-4)[1].tolist()         # between capture and first replay
+        assert eager == want and int(state.count_nonzero()) == 0
+    for rep in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert per.item() == want and abs(loss.item() - want) <= 1e-6 * abs(want), rep
+
+
+def test_capture_on_a_cold_stream_makes_no_accumulator(cuda):
+    """A stream captured before any loss ran on it has no accumulator, and none is made inside the graph: the capture takes
+    the form with a workspace, eager calls before the first replay are unharmed, and every replay gives the loss."""
+    from tmq_amd import ops
+    ws = [torch.from_numpy(_inputs(n, 50 + i)[0]).to(cuda) for i, n in enumerate([9408, 36864, 2049])]
+    ys0, loss0 = ops.softstep_fwd_all(ws, 2.236133, True, 5.0, 5e-4)
+    table = ops.SegmentTable(ws)
+    torch.cuda.synchronize()
+    calls = [lambda: ops.softstep_fwd_all(ws, 2.236133, True, 5.0, 5e-4), lambda: ops.ext.softstep_fwd_all(ws, 2.236133, True, 5.0, 5e-4),
+             lambda: ([], ops.qloss_multi(table, 5.0, 5e-4)[1]),
+             lambda: ([], ops.softstep_fused(ws[2], None, 2.236133, 5.0, 5e-4, 0.0, -1.0, 1.0, want_dw=False, in_launch=True)[3])]
+    for _ in range(32):                                                # (streams come from a pool: those no loss has run on yet)
+        if not calls:
+            break
+        graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.graph(graph, stream=side):
+            cold = ops.loss_state(cuda) is None
+            ys, loss = calls[0]()
+        if not cold:
+            continue
+        del calls[0]
+        with torch.cuda.stream(side):
+            assert ops.softstep_fwd_all(ws, 2.236133, True, 5.0, 5e-4)[1].item() == loss0.item()
+        values = []
+        for rep in range(3):
+            loss.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            values.append(loss.item())
+        assert values[0] == values[1] == values[2]
+        if loss.dtype == torch.float32:                                # (the fused pass sums one tensor, without the mean)
+            assert abs(values[0] - loss0.item()) <= 1e-6 * abs(loss0.item())
+        assert all(torch.equal(a, b) for a, b in zip(ys, ys0))
+    assert len(calls) < 4
+
+
 def test_full_size_fused_pass(cuda):
     """BASELINE configs[1] at its full 2^26 elements: the in-launch loss against the two-launch form."""
     n = 1 << 26

@@ -118,45 +118,76 @@ std::vector<torch::Tensor> step_weights(const std::vector<torch::Tensor> &weight
 }
 
 // The accumulator cells of the loss reductions that finish inside their launch: one zero-filled buffer per device
-// and stream, made on first use; every launch leaves it zero.
-torch::Tensor loss_state(const torch::Tensor &like) {
+// and stream, made on first use; every launch leaves it zero. The one registry of them (ops.loss_state asks here).
+// None while the stream is being captured and has none: a buffer made inside a graph is not zero before the first
+// replay, and eager launches on that stream would add to whatever it holds. The callers then take the form with a
+// workspace and a finalisation launch.
+c10::optional<torch::Tensor> loss_state(int64_t device_index) {
     static std::mutex guard;
     static std::map<std::pair<int, void *>, torch::Tensor> states;
-    const auto key = std::make_pair((int)like.device().index(), stream_of(like));
+    const c10::Device device(torch::kCUDA, (c10::DeviceIndex)device_index);
+    const c10::DeviceGuard on(device);
+    hipStream_t stream = at::hip::getCurrentHIPStream((c10::DeviceIndex)device_index).stream();
+    const auto key = std::make_pair((int)device_index, (void *)stream);
     std::lock_guard<std::mutex> lock(guard);
     auto it = states.find(key);
-    if (it == states.end())
-        it = states.emplace(key, torch::zeros({(int64_t)tmq_loss_state_bytes()}, like.options().dtype(torch::kUInt8))).first;
+    if (it == states.end()) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
+            (void)hipGetLastError();                    // the default stream while another one is being captured
+            return c10::nullopt;
+        }
+        if (capture != hipStreamCaptureStatusNone) return c10::nullopt;
+        it = states.emplace(key, torch::zeros({(int64_t)tmq_loss_state_bytes()}, torch::dtype(torch::kUInt8).device(device))).first;
+    }
     return it->second;
 }
 
-std::tuple<std::vector<torch::Tensor>, c10::optional<torch::Tensor>> softstep_fwd_all(
-        std::vector<torch::Tensor> weights, double digamma, bool want_loss, double sharpness, double strength) {
-    auto ws = step_weights(weights, "softstep_fwd_all");
+// y_l and the loss of dense fp32 weights on one device; a status of tmq_hip.h.
+int fwd_all(const std::vector<torch::Tensor> &ws, double digamma, bool want_loss, double sharpness, double strength,
+            std::vector<torch::Tensor> &parts, c10::optional<torch::Tensor> &loss) {
     const c10::DeviceGuard guard(ws[0].device());
     Carved ys = carve(ws);
     std::vector<tmq_step_tensor> table(ws.size());
     for (size_t i = 0; i < ws.size(); i++)
         table[i] = tmq_step_tensor{ws[i].data_ptr<float>(), nullptr, ys.parts[i].data_ptr<float>(), (uint64_t)ws[i].numel()};
-    c10::optional<torch::Tensor> loss;
+    parts = std::move(ys.parts);
     torch::Tensor workspace;
     if (want_loss) {
         loss = torch::empty({}, ws[0].options());
         // finished inside the launch where the shape allows (up to 64 tensors of up to 2^18 blocks each)
-        auto state = loss_state(ws[0]);
-        const int status = tmq_softstep_fwd_multi_inlaunch(table.data(), (int)table.size(), digamma, sharpness, strength,
-                                                           nullptr, loss->data_ptr<float>(), state.data_ptr(), stream_of(ws[0]));
-        if (status != TMQ_ERR_UNSUPPORTED) {
-            check(status, "softstep_fwd_all");
-            return {ys.parts, loss};
+        if (auto state = loss_state(ws[0].device().index())) {
+            const int status = tmq_softstep_fwd_multi_inlaunch(table.data(), (int)table.size(), digamma, sharpness, strength,
+                                                               nullptr, loss->data_ptr<float>(), state->data_ptr(), stream_of(ws[0]));
+            if (status != TMQ_ERR_UNSUPPORTED) return status;
         }
         workspace = torch::empty({(int64_t)tmq_softstep_multi_workspace_bytes(table.data(), (int)table.size())},
                                  ws[0].options().dtype(torch::kUInt8));
     }
-    check(tmq_softstep_fwd_multi(table.data(), (int)table.size(), digamma, sharpness, strength, nullptr,
-                                 want_loss ? loss->data_ptr<float>() : nullptr, want_loss ? workspace.data_ptr() : nullptr,
-                                 stream_of(ws[0])), "softstep_fwd_all");
-    return {ys.parts, loss};
+    return tmq_softstep_fwd_multi(table.data(), (int)table.size(), digamma, sharpness, strength, nullptr,
+                                  want_loss ? loss->data_ptr<float>() : nullptr, want_loss ? workspace.data_ptr() : nullptr,
+                                  stream_of(ws[0]));
+}
+
+// dw_l of dense fp32 weights and their gradients (undefined: none); a status of tmq_hip.h.
+int bwd_all(const std::vector<torch::Tensor> &ws, const std::vector<torch::Tensor> &gs, const float *upstream, double digamma,
+            double sharpness, double strength, std::vector<torch::Tensor> &parts) {
+    const c10::DeviceGuard guard(ws[0].device());
+    Carved dws = carve(ws);
+    std::vector<tmq_step_tensor> table(ws.size());
+    for (size_t i = 0; i < ws.size(); i++)
+        table[i] = tmq_step_tensor{ws[i].data_ptr<float>(), gs[i].defined() ? gs[i].data_ptr<float>() : nullptr,
+                                   dws.parts[i].data_ptr<float>(), (uint64_t)ws[i].numel()};
+    parts = std::move(dws.parts);
+    return tmq_softstep_bwd_multi(table.data(), (int)table.size(), digamma, sharpness, strength, upstream, stream_of(ws[0]));
+}
+
+std::tuple<std::vector<torch::Tensor>, c10::optional<torch::Tensor>> softstep_fwd_all(
+        std::vector<torch::Tensor> weights, double digamma, bool want_loss, double sharpness, double strength) {
+    std::vector<torch::Tensor> ys;
+    c10::optional<torch::Tensor> loss;
+    check(fwd_all(step_weights(weights, "softstep_fwd_all"), digamma, want_loss, sharpness, strength, ys, loss), "softstep_fwd_all");
+    return {ys, loss};
 }
 
 std::vector<c10::optional<torch::Tensor>> softstep_bwd_all(std::vector<torch::Tensor> weights,
@@ -173,31 +204,22 @@ std::vector<c10::optional<torch::Tensor>> softstep_bwd_all(std::vector<torch::Te
         up = loss_upstream->detach().to(torch::kFloat32).contiguous();
     }
     std::vector<size_t> live;
-    std::vector<torch::Tensor> like, gs;
-    for (size_t i = 0; i < ws.size(); i++)
-        if (grads[i].has_value() || up.defined()) {
-            live.push_back(i);
-            like.push_back(ws[i]);
-        }
+    std::vector<torch::Tensor> used, gs, dws;
+    for (size_t i = 0; i < ws.size(); i++) {
+        if (!grads[i].has_value() && !up.defined()) continue;
+        live.push_back(i);
+        used.push_back(ws[i]);
+        gs.emplace_back();
+        if (!grads[i].has_value()) continue;
+        const auto &g = *grads[i];
+        TORCH_CHECK(g.device() == ws[i].device() && g.scalar_type() == torch::kFloat32 && g.numel() == ws[i].numel(),
+                    "softstep_bwd_all: a gradient must match its weights in device, dtype and size");
+        gs.back() = g.detach().contiguous();
+    }
     std::vector<c10::optional<torch::Tensor>> out(ws.size());
     if (live.empty()) return out;
-    Carved dws = carve(like);
-    std::vector<tmq_step_tensor> table(live.size());
-    for (size_t k = 0; k < live.size(); k++) {
-        const size_t i = live[k];
-        const float *gp = nullptr;
-        if (grads[i].has_value()) {
-            const auto &g = *grads[i];
-            TORCH_CHECK(g.device() == ws[i].device() && g.scalar_type() == torch::kFloat32 && g.numel() == ws[i].numel(),
-                        "softstep_bwd_all: a gradient must match its weights in device, dtype and size");
-            gs.push_back(g.detach().contiguous());
-            gp = gs.back().data_ptr<float>();
-        }
-        table[k] = tmq_step_tensor{ws[i].data_ptr<float>(), gp, dws.parts[k].data_ptr<float>(), (uint64_t)ws[i].numel()};
-        out[i] = dws.parts[k];
-    }
-    check(tmq_softstep_bwd_multi(table.data(), (int)table.size(), digamma, sharpness, strength,
-                                 up.defined() ? up.data_ptr<float>() : nullptr, stream_of(ws[0])), "softstep_bwd_all");
+    check(bwd_all(used, gs, up.defined() ? up.data_ptr<float>() : nullptr, digamma, sharpness, strength, dws), "softstep_bwd_all");
+    for (size_t k = 0; k < live.size(); k++) out[live[k]] = dws[k];
     return out;
 }
 
@@ -580,20 +602,10 @@ bool plain_weights(const std::vector<torch::Tensor> &ws) {
 
 c10::optional<std::pair<std::vector<torch::Tensor>, Maybe>> plain_softstep_fwd(const std::vector<torch::Tensor> &ws, double digamma,
                                                                                bool want_loss, double sharpness, double strength) {
-    if (!plain_weights(ws)) return c10::nullopt;
-    const c10::DeviceGuard guard(ws[0].device());
-    Carved ys = carve(ws);
-    std::vector<tmq_step_tensor> table(ws.size());
-    for (size_t i = 0; i < ws.size(); i++)
-        table[i] = tmq_step_tensor{ws[i].data_ptr<float>(), nullptr, ys.parts[i].data_ptr<float>(), (uint64_t)ws[i].numel()};
+    std::vector<torch::Tensor> ys;
     Maybe loss;
-    if (want_loss) loss = torch::empty({}, ws[0].options());
-    const int status = want_loss ? tmq_softstep_fwd_multi_inlaunch(table.data(), (int)table.size(), digamma, sharpness, strength, nullptr,
-                                                                   loss->data_ptr<float>(), loss_state(ws[0]).data_ptr(), stream_of(ws[0]))
-                                 : tmq_softstep_fwd_multi(table.data(), (int)table.size(), digamma, sharpness, strength, nullptr, nullptr,
-                                                          nullptr, stream_of(ws[0]));
-    if (status != TMQ_OK) return c10::nullopt;
-    return std::make_pair(std::move(ys.parts), loss);
+    if (!plain_weights(ws) || fwd_all(ws, digamma, want_loss, sharpness, strength, ys, loss) != TMQ_OK) return c10::nullopt;
+    return std::make_pair(std::move(ys), loss);
 }
 
 c10::optional<std::vector<torch::Tensor>> plain_softstep_bwd(const std::vector<torch::Tensor> &ws, const std::vector<torch::Tensor> &gs,
@@ -604,15 +616,10 @@ c10::optional<std::vector<torch::Tensor>> plain_softstep_bwd(const std::vector<t
             return c10::nullopt;
     if (upstream.has_value() && (upstream->device() != ws[0].device() || upstream->scalar_type() != torch::kFloat32 || upstream->numel() != 1))
         return c10::nullopt;
-    const c10::DeviceGuard guard(ws[0].device());
-    Carved dws = carve(ws);
-    std::vector<tmq_step_tensor> table(ws.size());
-    for (size_t i = 0; i < ws.size(); i++)
-        table[i] = tmq_step_tensor{ws[i].data_ptr<float>(), gs[i].data_ptr<float>(), dws.parts[i].data_ptr<float>(), (uint64_t)ws[i].numel()};
-    if (tmq_softstep_bwd_multi(table.data(), (int)table.size(), digamma, sharpness, strength,
-                               upstream.has_value() ? upstream->data_ptr<float>() : nullptr, stream_of(ws[0])) != TMQ_OK)
+    std::vector<torch::Tensor> dws;
+    if (bwd_all(ws, gs, upstream.has_value() ? upstream->data_ptr<float>() : nullptr, digamma, sharpness, strength, dws) != TMQ_OK)
         return c10::nullopt;
-    return std::move(dws.parts);
+    return dws;
 }
 
 }  // namespace
@@ -631,6 +638,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     // additive: all layers of a training step in one launch
     m.def("softstep_fwd_all", &softstep_fwd_all);
     m.def("softstep_bwd_all", &softstep_bwd_all);
+    m.def("loss_state", &loss_state);
     // additive: the plain calls of tmq_amd/ops.py
     m.def("plain_linear", &plain_linear);
     m.def("plain_conv", &plain_conv);

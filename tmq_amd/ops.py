@@ -103,18 +103,24 @@ def ternarize_(weights: torch.Tensor, digamma: float = 0.0) -> torch.Tensor:
     return weights
 
 
-_loss_states = {}
+_loss_states = {}    # (without the extension, whose registry it is otherwise)
 
 
 def loss_state(device):
     """The accumulator cells of the loss reductions that finish inside their launch (tmq_*_inlaunch): one small
     zero-filled buffer per device and stream, made on first use. Every launch leaves it zero, so it is never
-    cleared again; launches on one stream are ordered, so they can share it."""
+    cleared again; launches on one stream are ordered, so they can share it. None while the stream is being captured
+    and has none yet: made inside a graph it would not be zero before the first replay."""
     device = torch.device(device)
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(device).cuda_stream)
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    if ext is not None:
+        return ext.loss_state(index)
+    key = (index, torch.cuda.current_stream(device).cuda_stream)
     st = _loss_states.get(key)
     if st is None:
+        with _capi.on_device(torch.device("cuda", index)):
+            if torch.cuda.is_current_stream_capturing():
+                return None
         st = _loss_states[key] = torch.zeros(_lib().tmq_loss_state_bytes(), dtype=torch.uint8, device=device)
     return st
 
@@ -145,10 +151,12 @@ def softstep_fused(weights, grad, digamma, sharpness, strength, gl, lo, hi, *, w
         if grad.numel() != n or grad.dtype != torch.float32:
             raise RuntimeError("softstep_fused: gradient must match the weights")
     if in_launch and loss is not None and n:
-        with _capi.on_device(w.device):
-            status = lib.tmq_softstep_fused_inlaunch(ptr(w), ptr(grad) if dw is not None else None, ptr(y), ptr(dw), ptr(wc),
-                                                     ptr(loss), ptr(loss_state(w.device)), n, float(digamma), float(sharpness),
-                                                     float(strength), ctypes.c_float(gl), float(lo), float(hi), stream_of(w))
+        state, status = loss_state(w.device), _capi.ERR_UNSUPPORTED
+        if state is not None:
+            with _capi.on_device(w.device):
+                status = lib.tmq_softstep_fused_inlaunch(ptr(w), ptr(grad) if dw is not None else None, ptr(y), ptr(dw), ptr(wc),
+                                                         ptr(loss), ptr(state), n, float(digamma), float(sharpness),
+                                                         float(strength), ctypes.c_float(gl), float(lo), float(hi), stream_of(w))
         if status != _capi.ERR_UNSUPPORTED:
             check(status, "softstep_fused_inlaunch")
             return y, dw, wc, loss
@@ -206,9 +214,10 @@ def qloss_multi(table: SegmentTable, sharpness: float, strength: float):
     tot = torch.empty(1, dtype=torch.float32, device=table.device)
     with _capi.on_device(table.device):
         # finished inside the launch where the shape allows (up to 64 tensors, 2^18 blocks), else two launches
+        state = loss_state(table.device) if table.total_blocks else None
         status = _lib().tmq_qloss_multi_inlaunch(ptr(table.table), table.nseg, table.total_blocks, float(sharpness),
-                                                 float(strength), ptr(per), ptr(tot), ptr(loss_state(table.device)),
-                                                 stream_of(table.table)) if table.total_blocks else _capi.ERR_UNSUPPORTED
+                                                 float(strength), ptr(per), ptr(tot), ptr(state),
+                                                 stream_of(table.table)) if state is not None else _capi.ERR_UNSUPPORTED
         if status != _capi.ERR_UNSUPPORTED:
             check(status, "qloss_multi_inlaunch")
             return per, tot
@@ -282,9 +291,11 @@ def softstep_fwd_all(weights, digamma: float, want_loss: bool = False, sharpness
     if want_loss:
         loss = torch.empty((), dtype=torch.float32, device=dev)
         # the loss finished inside the launch where the shape allows (up to 64 tensors of up to 2^18 blocks)
-        with _capi.on_device(dev):
-            status = lib.tmq_softstep_fwd_multi_inlaunch(arr, len(ws), float(digamma), float(sharpness), float(strength), None,
-                                                         ptr(loss), ptr(loss_state(dev)), stream_of(flat))
+        state, status = loss_state(dev), _capi.ERR_UNSUPPORTED
+        if state is not None:
+            with _capi.on_device(dev):
+                status = lib.tmq_softstep_fwd_multi_inlaunch(arr, len(ws), float(digamma), float(sharpness), float(strength), None,
+                                                             ptr(loss), ptr(state), stream_of(flat))
         if status != _capi.ERR_UNSUPPORTED:
             check(status, "softstep_fwd_all")
             return ys, loss
