@@ -383,6 +383,9 @@ int tmq_f32_to_f16_prescaled(const float *x, int64_t n, float *prescale, void *h
  * launch behind the scan (workspace: tmq_f32_to_f16_prescaled_workspace_bytes(B C HW) bytes).            */
 int tmq_f32_nchw_to_f16_nhwc_prescaled(const float *x, int64_t B, int64_t C, int64_t HW, float *prescale, void *hi,
                                        const float *scale_in, float *scale_out, int64_t channels, void *workspace, void *stream);
+/* 1 if that call is faster than tmq_f32_to_f16_prescaled followed by a strided copy (not for planes of a few pixels or
+ * large tensors of a few channels, whose tiles would be mostly empty). The values are the same either way.  */
+int tmq_f32_nchw_to_f16_nhwc_pays(const float *x, int64_t B, int64_t C, int64_t HW);
 
 /* 1 if M fp32 rows against a K x N layer are faster as two fp16 passes over tmq_split_f32's terms than
  * as one tmq_ternary_linear call with x_dtype TMQ_F32 (many rows, or a few rows over a large

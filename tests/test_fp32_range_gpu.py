@@ -240,6 +240,24 @@ def test_planar_input_converts_straight_into_channels_last(cuda, shape, shift):
     assert torch.equal(got.contiguous().view(torch.int16), want.view(torch.int16)) and torch.equal(adj, adj2)
 
 
+@pytest.mark.parametrize("shape,pays", [((64, 3, 224, 224), False), ((4, 3, 224, 224), True), ((1536, 8, 3, 3), False), ((1024, 8, 3, 3), True),
+                                        ((2000, 64, 1, 2), False), ((1100, 64, 8, 8), True), ((300, 100, 23, 23), True)])
+def test_planar_input_of_mostly_empty_tiles_takes_the_two_launches(cuda, shape, pays):
+    """Planes of a few pixels and large tensors of a few channels would leave the reordering launch's tiles mostly empty:
+    they are converted in place and copied. The bits are the same on both sides of the line, through the call itself and
+    through a convolution's one-call form."""
+    from tmq_amd import ops, _capi
+    B, C, H, W = shape
+    g = torch.Generator(device=cuda).manual_seed(sum(shape))
+    x = torch.randn(shape, device=cuda, generator=g) * 3e-5
+    assert _capi.load().tmq_f32_nchw_to_f16_nhwc_pays(_capi.ptr(x), B, C, H * W) == int(pays)
+    want, adj = ops.f32_to_f16_prescaled(x, None, 16)
+    got, adj2 = ops.f32_to_f16_prescaled(x, None, 16, channels_last=True)
+    assert got.is_contiguous(memory_format=torch.channels_last) and torch.equal(got, want) and torch.equal(adj, adj2)
+    nw = ops.NativeWeights(ops.compactify_ternary(torch.randint(-1, 2, (16, C, 1, 1), device=cuda, generator=g).float()), 16, (1, 1))
+    assert torch.equal(ops.ternary_conv2d(x, nw), ops.ternary_conv2d(got, nw, scale=adj))
+
+
 def test_switch_sends_many_rows_against_a_narrow_layer_to_the_one_pass_kernel(cuda):
     """With the prescale switched off (values promised to lie in fp16's range), a thousand fp32 rows or more against at
     most 128 channels skip the row-pair route, whose split pass would move the rows three times: same values to fp32

@@ -86,6 +86,7 @@ SIGNATURES = {
     "tmq_f32_to_f16_prescaled_workspace_bytes": (_sz, [_i64]),
     "tmq_f32_to_f16_prescaled": (_int, [_vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp]),
     "tmq_f32_nchw_to_f16_nhwc_prescaled": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp]),
+    "tmq_f32_nchw_to_f16_nhwc_pays": (_int, [_vp, _i64, _i64, _i64]),
     "tmq_f32_prescale": (_int, [_vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp]),
     "tmq_selfcheck_fastdiv": (_i64, [_u32, _vp, _i64]),
     "tmq_fp32_rows_prefer_split": (_int, [_i64, _i64, _i64]),

@@ -286,6 +286,7 @@ __global__ __launch_bounds__(256) void convert_prescaled_kernel(const float *__r
 // along the planes, all on their way while the partial maxima are reduced -- turns its block in registers, and the tile
 // goes out through LDS in pieces of 8 channels, 128-byte runs per pixel at CT = 64. Bound by memory: 4 bytes in, 2 out a
 // value. Converted in place and left to a strided copy before: [32, 128, 28, 28] 7.8 + 13.6 us in two launches; the layer (128 -> 128, 3 x 3) 38.3 -> 29.4 us.
+// (Where tiles are mostly empty the two launches are faster: planar_tiles_pay.)
 // vec: HW a multiple of 4 and x 16-byte aligned (a quad of pixels is one load); out_piece 8 / 4: C a multiple of 8 / 4 and
 // hi 16- / 8-byte aligned (pieces of 8 / 4 channels are one store); everything else element by element.
 template <int CT>
@@ -365,6 +366,24 @@ __global__ __launch_bounds__(256) void convert_prescaled_nhwc_kernel(const float
             }
         }
     }
+}
+
+// channels per tile: no more than there are, so that few channels don't leave most of a tile empty
+inline int planar_tile_channels(int64_t C) { return C <= 16 ? 16 : C <= 32 ? 32 : 64; }
+inline int64_t planar_tiles(int64_t B, int64_t C, int64_t HW) {
+    const int64_t CT = planar_tile_channels(C), PT = 4096 / CT;
+    return B * ((C + CT - 1) / CT) * ((HW + PT - 1) / PT);
+}
+inline bool planar_vec(const void *x, int64_t HW) { return HW % 4 == 0 && aligned16(x); }
+
+// Whether the reordering launch beats the conversion in place followed by a strided copy. Every tile costs a workgroup
+// that reduces the partial maxima again, however little of it exists (4.5 ns each beyond the first round, 5.6 without quad
+// loads), where the two launches cost 5 us more at rest and 2.7 ns per 4096 values. 618 shapes of 3e4, 1e6 and 1.2e7 values,
+// 2 .. 2048 channels, planes of 2 .. 111222 pixels, copy = 1: up to 1.00 where this says yes, 0.71 and more where it says no --
+// [64, 3, 224, 224] 1.94, [20000, 8, 3, 3] 5.8, [125000, 2, 2, 2] 38; against 0.38 for [32, 128, 28, 28], 0.42 for [64, 512, 7, 7].
+inline bool planar_tiles_pay(const void *x, int64_t B, int64_t C, int64_t HW) {
+    const int64_t n = B * C * HW, tiles = planar_tiles(B, C, HW);
+    return tiles <= 1024 + n / (planar_vec(x, HW) ? 2048 : 4096) || 8192 * tiles <= 3 * n;
 }
 
 // Many fp32 rows as fp16 row pairs in groups of eight, every group under a power of two s of its own: a workgroup
@@ -631,19 +650,22 @@ int tmq_f32_to_f16_prescaled(const float *x, int64_t n, float *prescale, void *h
     return check_launch();
 }
 
+int tmq_f32_nchw_to_f16_nhwc_pays(const float *x, int64_t B, int64_t C, int64_t HW) {
+    return B > 0 && C > 0 && HW > 0 && planar_tiles_pay(x, B, C, HW) ? 1 : 0;
+}
+
 int tmq_f32_nchw_to_f16_nhwc_prescaled(const float *x, int64_t B, int64_t C, int64_t HW, float *prescale, void *hi,
                                        const float *scale_in, float *scale_out, int64_t channels, void *workspace, void *stream) {
     if (B <= 0 || C <= 0 || HW <= 0 || !x || !prescale || !hi || !workspace || channels < 0 || (scale_out && channels == 0))
         return TMQ_ERR_INVALID_ARG;
     float *partials = static_cast<float *>(workspace);
-    // channels per tile: no more than there are, so that few channels don't leave most of a tile empty
-    const int CT = C <= 16 ? 16 : C <= 32 ? 32 : 64;
+    const int CT = planar_tile_channels(C);
     const int64_t tiles_p = (HW + 4096 / CT - 1) / (4096 / CT), tiles_c = (C + CT - 1) / CT;
     if (tiles_p > 0x7FFFFFFF || tiles_c > 0x7FFFFFFF) return TMQ_ERR_TOO_LARGE;
-    const int64_t tiles = B * tiles_p * tiles_c, groups = tiles < (1 << 20) ? tiles : (1 << 20);
+    const int64_t tiles = planar_tiles(B, C, HW), groups = tiles < (1 << 20) ? tiles : (1 << 20);
     const int blocks = launch_absmax(x, B * C * HW, partials, (int)aligned16(x), stream);
     if (int rc = check_launch()) return rc;
-    const int vec = HW % 4 == 0 && aligned16(x);
+    const int vec = planar_vec(x, HW);
     const uintptr_t at = reinterpret_cast<uintptr_t>(hi);
     const int piece = C % 8 == 0 && (at & 15u) == 0 ? 8 : C % 4 == 0 && (at & 7u) == 0 ? 4 : 1;
     auto kernel = CT == 16 ? convert_prescaled_nhwc_kernel<16> : CT == 32 ? convert_prescaled_nhwc_kernel<32> : convert_prescaled_nhwc_kernel<64>;

@@ -578,14 +578,15 @@ Maybe plain_conv(const torch::Tensor &input, const torch::Tensor &words, bool de
         const int64_t n = x.numel(), part = (int64_t)tmq_f32_to_f16_prescaled_workspace_bytes(n) / 4;
         scratch = at::empty({part + 4 + N}, x.options());
         float *ws = scratch.data_ptr<float>();
-        auto hi = at::empty({B, C, H, W}, x.options().dtype(torch::kFloat16).memory_format(last));
+        const bool reorder = !nhwc && tmq_f32_nchw_to_f16_nhwc_pays(x.data_ptr<float>(), B, C, H * W);
+        auto hi = at::empty({B, C, H, W}, x.options().dtype(torch::kFloat16).memory_format(nhwc || reorder ? last : at::MemoryFormat::Contiguous));
         const float *per = scale.has_value() ? scale->data_ptr<float>() : nullptr;
-        const int status = nhwc ? tmq_f32_to_f16_prescaled(x.data_ptr<float>(), n, ws + part, hi.data_ptr(), per, ws + part + 4, N, ws, stream_of(x))
-                                : tmq_f32_nchw_to_f16_nhwc_prescaled(x.data_ptr<float>(), B, C, H * W, ws + part, hi.data_ptr(), per,
-                                                                     ws + part + 4, N, ws, stream_of(x));
+        const int status = reorder ? tmq_f32_nchw_to_f16_nhwc_prescaled(x.data_ptr<float>(), B, C, H * W, ws + part, hi.data_ptr(), per,
+                                                                        ws + part + 4, N, ws, stream_of(x))
+                                   : tmq_f32_to_f16_prescaled(x.data_ptr<float>(), n, ws + part, hi.data_ptr(), per, ws + part + 4, N, ws, stream_of(x));
         if (status != TMQ_OK) return c10::nullopt;
         scale = scratch.narrow(0, part + 4, N);
-        x = hi;
+        x = hi.contiguous(last);
     }
     const tmq_epilogue ep = epilogue_of(scale, bias, residual, relu, y);
     const int status = depthwise ? tmq_ternary_dwconv2d(x.data_ptr(), &shape, reinterpret_cast<const uint32_t *>(words.data_ptr<int32_t>()), &ep, y.data_ptr(), stream_of(x))

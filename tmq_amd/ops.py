@@ -616,7 +616,7 @@ def f32_to_f16_prescaled(x: torch.Tensor, scale, channels: int, channels_last: b
     """One fp16 term of an fp32 activation tensor for the convolution kernels: (fp16 tensor of x's shape and
     memory format holding s x, scale / s) with the range prescale s, or (x.half(), scale) when the prescale
     is switched off. channels_last: a planar [B, C, H, W] tensor comes back in channels_last memory, reordered by
-    the launch that converts it."""
+    the launch that converts it where that is faster than a copy behind it."""
     if not _fp32_prescale or x.numel() == 0:      # nothing to scale in an empty batch
         return x.to(torch.float16), scale
     if not (x.is_contiguous() or x.is_contiguous(memory_format=torch.channels_last)):
@@ -629,7 +629,8 @@ def f32_to_f16_prescaled(x: torch.Tensor, scale, channels: int, channels_last: b
     ps = torch.empty(2, dtype=torch.float32, device=x.device)
     adj = torch.empty(channels, dtype=torch.float32, device=x.device) if channels else None
     ws = torch.empty(lib.tmq_f32_to_f16_prescaled_workspace_bytes(n), dtype=torch.uint8, device=x.device)
-    if channels_last and not x.is_contiguous(memory_format=torch.channels_last):
+    if channels_last and not x.is_contiguous(memory_format=torch.channels_last) and \
+            lib.tmq_f32_nchw_to_f16_nhwc_pays(ptr(x), x.shape[0], x.shape[1], x.shape[2] * x.shape[3]):
         B, C, H, W = x.shape
         hi = torch.empty((B, C, H, W), dtype=torch.float16, device=x.device, memory_format=torch.channels_last)
         with _capi.on_device(x.device):
@@ -640,6 +641,8 @@ def f32_to_f16_prescaled(x: torch.Tensor, scale, channels: int, channels_last: b
     with _capi.on_device(x.device):
         check(lib.tmq_f32_to_f16_prescaled(ptr(x), n, ptr(ps), ptr(hi), ptr(scale), ptr(adj), channels, ptr(ws), stream_of(x)),
               "f32_to_f16_prescaled")
+    if channels_last:
+        hi = hi.contiguous(memory_format=torch.channels_last)
     return hi, (adj if channels else scale)
 
 
