@@ -436,8 +436,8 @@ int tmq_ternary_conv2d_view(const void *x, const tmq_conv_shape *shape, const vo
 
 /* Several such convolutions of ONE input (same B, C, H, W and N; windows, padding and dilation of their own) written
  * into one destination: phase q goes to the view that starts `first` pixels into y (and into epilogue->residual).
- * The phases of a transposed convolution, tmq/tmq.py:1007-1042. Inputs of a multiple of 64 channels take one launch
- * for up to four phases, others one launch per phase.                                               */
+ * The phases of a transposed convolution, tmq/tmq.py:1007-1042. Up to four phases take one launch, for any number
+ * of channels; a phase alone in its group, and few tiles over long reductions, take one launch each.  */
 typedef struct tmq_conv_phase {
     tmq_conv_shape shape;
     tmq_output_view view;

@@ -231,3 +231,35 @@ def test_transposed_layer_follows_a_change_of_padding(cuda):
     for pad, opad in ((0, 0), (1, 2), (0, 0)):
         net[0].padding, net[0].output_padding = (pad, pad), (opad, opad)
         assert torch.equal(net(x).cpu(), F.conv_transpose2d(x.cpu().float(), w.cpu(), None, 3, pad, opad))
+
+
+@pytest.mark.parametrize("cin,cout,k,stride,pad,hw,batch", [
+    (64, 40, 3, 1, 1, (9, 7), 2), (24, 33, 2, 1, 0, (6, 9), 1),            # one phase: an ordinary convolution
+    (512, 48, (6, 6), (2, 2), (2, 2), (5, 6), 1),                              # four phases of few tiles and long reductions: one by one
+    (128, 70, (2, 4), (1, 2), (0, 1), (6, 5), 1), (64, 34, (1, 2), (1, 2), 0, (6, 5), 3),   # two, either way
+    (64, 30, (3, 3), (3, 3), 0, (6, 5), 1)])                                # nine: two groups of four, the last one alone
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_phases_alone_or_of_long_reductions_take_their_own_launches(cuda, cin, cout, k, stride, pad, hw, batch, dtype):
+    """Each side of the rule that sends the phases of a transposed convolution through one launch or through the route of an
+    ordinary convolution, with residual and ReLU, against F.conv_transpose2d (small integers: exact)."""
+    import tmq_amd as t
+    from tmq_amd import ops
+    torch.manual_seed(cin + cout)
+    net = torch.nn.Sequential(torch.nn.ConvTranspose2d(cin, cout, k, stride, pad, bias=True))
+    t.quantize_model(net, t.QuantizationControl())
+    net.to(cuda).eval()
+    net[0].weight.data = torch.randint(-1, 2, net[0].weight.shape, device=cuda).float()
+    net[0].bias.data = torch.randint(-4, 5, (cout,), device=cuda).float()
+    t.compressed_state_dict(net)
+    x = torch.randint(-2, 3, (batch, cin) + hw, device=cuda).half().contiguous(memory_format=torch.channels_last)
+    want = F.conv_transpose2d(x.cpu().float(), ops.expand_ternary(net[0].weight.data, net[0].original_shape).cpu(),
+                              net[0].bias.data.cpu(), stride, pad)
+    assert want.abs().max() < 2000
+    prev = t.set_compact_output_dtype(dtype)
+    try:
+        assert torch.equal(net(x).cpu(), want.to(dtype))
+    finally:
+        t.set_compact_output_dtype(prev)
+    res = torch.randint(-9, 10, want.shape, device=cuda).to(dtype).contiguous(memory_format=torch.channels_last)
+    got = ops.ternary_conv2d_into(torch.empty_like(res), x, None, bias=net[0].bias.data, residual=res, relu=True, phases=net[0]._phases[2])
+    assert torch.equal(got.cpu(), torch.relu(want + res.cpu().float()).to(dtype))

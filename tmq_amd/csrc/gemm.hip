@@ -1283,13 +1283,25 @@ int conv_plan(const tmq_conv_shape *s, const tmq_output_view *view, int32_t &ho,
     return TMQ_OK;
 }
 
-// The convolutions of tmq_ternary_conv2d_phases, kPhases to a launch. 64 x 64 tiles up to 64 channels, 64 x 128 beyond
-// (512 -> 256 on 14 x 14, batch 8: 17.8 us against 20.8 on 128 x 128 tiles); register loaders 128 x 128 beyond, where that
-// gives every CU one, all phases counted together. Against one launch
-// per phase, which few tiles sent to the split-reduction kernel -- 4 x 4 / 2 in fp16, one image or a batch: 128 -> 64
-// channels on 56 x 56, batch 32 61.7 -> 44.3 us; 256 -> 128 on 28 x 28, batch 16 41.9 -> 21.4; 64 -> 64 on 32 x 32, batch 8
-// 21.2 -> 7.9; 100 -> 64 on 28 x 28, batch 8 50.4 -> 16.6; 32 -> 32 on 56 x 56, batch 8 23.9 -> 9.6; 128 -> 64 on one 14 x 14
-// image 13.1 -> 7.7; and 512 -> 256 on one 7 x 7 image, where the split reduction is at its best, 16.5 -> 16.7.
+// Whether phases of a multiple of 64 channels share a launch: `count` of them, the longest reduction and all of them
+// together in 64-index tiles, and the work in 64 x 64 x 64 blocks. A launch of its own sends a phase of few tiles to the
+// split-reduction kernel, whose time hardly grows with the reduction, where a shared launch walks it in one workgroup per
+// tile. Fitted to 372 groups of two to four phases (64 .. 2048 channels, 16 .. 600 outputs, windows to 6 x 6, steps 1 .. 3,
+// one image to 32), us: 3.5 a launch + 0.022 a tile of the reductions + 0.2 per 256 blocks, against 6.2 + 0.345 a tile of
+// the longest + 0.06, the line then moved to where sharing is at most 1.03 of one by one (1.003 of the better on average).
+// 512 -> 256, 6 x 6 / 2 on one 7 x 7 image: 30.6 us shared, 23.9 one by one; 1024 -> 144, 5 x 5 / (1, 2) on 18 x 7: 92.3 and
+// 21.9; but 512 -> 256, 4 x 4 / 2 on 14 x 14, batch 8: 16.7 and 24.3.
+inline bool phases_share_a_launch(int count, int64_t longest, int64_t together, int64_t blocks) {
+    return 20 * longest + 260 <= 160 * count + together + 10 * (blocks / 256);
+}
+
+// The convolutions of tmq_ternary_conv2d_phases, kPhases to a launch. 128 x 32 tiles up to 32 channels, 64 x 64 up to 64,
+// 64 x 128 beyond (512 -> 256 on 14 x 14, batch 8: 17.8 us against 20.8 on 128 x 128 tiles); register loaders 128 x 128
+// beyond, where that gives every CU one, all phases counted together. Against one launch per phase, 4 x 4 / 2 in fp16:
+// 128 -> 64 channels on 56 x 56, batch 32 61.7 -> 44.3 us; 256 -> 128 on 28 x 28, batch 16 41.9 -> 21.4; 256 -> 256 on 28 x 28,
+// batch 32 73.6 -> 52.6; 64 -> 64 on 32 x 32, batch 8 21.2 -> 7.9; 100 -> 64 on 28 x 28, batch 8 50.4 -> 16.6; 32 -> 32 on
+// 56 x 56, batch 8 23.9 -> 9.6; 128 -> 64 on one 14 x 14 image 13.1 -> 7.7. A phase that is alone in its group (a step of 1,
+// the ninth of nine) is an ordinary convolution and takes that one's route: 512 -> 174, 2 x 2 / 1 on 48 x 9 4.6 us, 18.6 here.
 template <class Loader>
 int conv_phases(const _Float16 *x, const tmq_conv_phase *phases, int count, const tmq_epilogue &e, void *y, void *stream) {
     const int64_t N = phases[0].shape.N, elt = e.y_dtype == TMQ_F16 ? 2 : 4;
@@ -1297,7 +1309,8 @@ int conv_phases(const _Float16 *x, const tmq_conv_phase *phases, int count, cons
         PhaseSet<Loader, ViewEpilogue> set{};
         set.N = N;
         set.Nb = native_blocks_n(N);
-        [[maybe_unused]] int64_t squares = 0, longest = 0;          // 128 x 128 tiles; the longest reduction
+        [[maybe_unused]] int64_t squares = 0, longest = 0, together = 0, blocks = 0;   // 128 x 128 tiles; the longest reduction
+        int live[kPhases];
         for (int q = first; q < count && q < first + kPhases; q++) {
             const tmq_conv_phase &p = phases[q];
             const tmq_conv_shape &s = p.shape;
@@ -1306,6 +1319,7 @@ int conv_phases(const _Float16 *x, const tmq_conv_phase *phases, int count, cons
             if (int rc = conv_plan(&s, &p.view, ho, wo, map)) return rc;
             const int64_t M = (int64_t)s.B * ho * wo, K = (int64_t)s.C * s.ky * s.kx;
             if (M == 0 || p.view.h_cnt == 0 || p.view.w_cnt == 0) continue;
+            live[set.count] = q;
             auto &ph = set.phase[set.count++];
             ph.ld = Loader{x, M, K, s.B, s.C, s.H, s.W, ho, wo, s.ky, s.kx, s.sy, s.sx, s.py, s.px, s.dy, s.dx};
             if constexpr (Loader::kDirect) ph.ld = with_divisors(ph.ld);
@@ -1320,8 +1334,20 @@ int conv_phases(const _Float16 *x, const tmq_conv_phase *phases, int count, cons
                                  e.y_dtype == TMQ_F16 ? 1 : 0, map};
             squares += ((M + 127) / 128) * ((N + 127) / 128);
             if (K > longest) longest = K;
+            together += K / kBK;
+            blocks += ((M + 63) / 64) * ((N + 63) / 64) * (K / kBK);
         }
         if (set.count == 0) continue;
+        if (set.count == 1 || (std::is_same<Loader, ConvLoader64>::value && !phases_share_a_launch(set.count, longest / kBK, together, blocks))) {
+            for (int i = 0; i < set.count; i++) {
+                const tmq_conv_phase &p = phases[live[i]];
+                tmq_epilogue ep = e;
+                if (e.residual) ep.residual = static_cast<const unsigned char *>(e.residual) + p.first * N * elt;
+                if (int rc = tmq_ternary_conv2d_view(x, &p.shape, p.native, &ep, static_cast<unsigned char *>(y) + p.first * N * elt, &p.view, stream))
+                    return rc;
+            }
+            continue;
+        }
         int rc;
         if constexpr (Loader::kDirect) {
             rc = N > 64 ? launch_phases<4, 2, 1, 4, 1>(set, stream) : N > 32 ? launch_phases<4, 2, 1, 2, 1>(set, stream)
