@@ -187,22 +187,22 @@ def test_phases_in_one_launch_equal_one_launch_each(cuda, cin, cout, k, stride, 
 
 @pytest.mark.parametrize("B,C,hw,N,k", [
     (1, 64, (41, 50), 70, 1),          # short reduction: 64 x 128 tiles, a ragged last tile in rows and columns
-    (1, 64, (116, 127), 200, 1),       # 460 of them in whole 256 columns: 64 x 256
-    (1, 128, (190, 100), 300, 1),      # an odd number of 128s
+    (1, 64, (116, 127), 200, 1),       # 462 of them in two 128s: 64 x 256
+    (1, 128, (190, 100), 300, 1),      # 891 in three, N no multiple of 8: the general tiles
     (1, 64, (86, 96), 128, 3),         # 129 tiles at K = 576, where the split reduction ends: 64 x 128 solo
     (1, 64, (129, 128), 100, 3),       # 258 tiles, N <= 128: dma at K = 576 ...
     (1, 128, (129, 128), 128, 3),      # ... solo at K = 1152
     (1, 128, (96, 121), 130, 3),       # 129 .. 256 columns, 364 tiles: 64 x 128 solo
-    (1, 64, (82, 81), 300, 3),         # three 128s: solo up to 512 tiles ...
-    (1, 64, (107, 109), 300, 3),       # ... dma beyond
-    (1, 64, (71, 73), 400, 3),         # four 128s: 64 x 256
+    (1, 64, (82, 81), 300, 3),         # three 128s, short of K = 1024: dma ...
+    (1, 64, (107, 109), 300, 3),       # ... for any number of tiles
+    (1, 64, (71, 73), 400, 3),         # and four
     (2, 64, (97, 95), 32, 3),          # at most 32 columns: 128 x 32 tiles, a ragged last one, direct loads ...
     (3, 16, (31, 33), 17, 5), (1, 104, (40, 41), 24, 3),     # ... of few channels, through registers
     (1, 136, (19, 21), 30, 3), (2, 17, (15, 16), 5, 3)])     # (reduction of 1224: deeper prefetch; single elements)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_wide_tiles_at_their_edges(cuda, B, C, hw, N, k, dtype):
-    """Convolutions with more than 64 outputs on the tiles of 64 x 128 and 64 x 256, each rule of their choice once,
-    against F.conv2d: small integers, so every sum is exact (fp16 results: below 2^11)."""
+    """Convolutions on the tiles of 64 x 128 and 64 x 256 (more than 64 outputs) and 128 x 32 (at most 32), the rules of
+    their choice, against F.conv2d: small integers, so every sum is exact (fp16 results: below 2^11)."""
     from tmq_amd import ops
     g = torch.Generator(device=cuda).manual_seed(C + N + k)
     Wt = torch.randint(-1, 2, (N, C, k, k), device=cuda, generator=g).float()
@@ -263,3 +263,24 @@ def test_phases_alone_or_of_long_reductions_take_their_own_launches(cuda, cin, c
     res = torch.randint(-9, 10, want.shape, device=cuda).to(dtype).contiguous(memory_format=torch.channels_last)
     got = ops.ternary_conv2d_into(torch.empty_like(res), x, None, bias=net[0].bias.data, residual=res, relu=True, phases=net[0]._phases[2])
     assert torch.equal(got.cpu(), torch.relu(want + res.cpu().float()).to(dtype))
+
+
+@pytest.mark.parametrize("B,C,hw,N,k", [
+    (1, 128, (82, 81), 300, 3),        # three 128s from K = 1024 on: 312 tiles, solo
+    (1, 128, (70, 73), 500, 3),        # four: 320
+    (1, 128, (110, 100), 504, 3),      # 688
+    (1, 128, (120, 116), 400, 3),      # 872: the general tiles
+    (1, 128, (150, 151), 264, 3),      # three, 1062: dma
+    (1, 64, (131, 141), 250, 3),       # two, 578: 64 x 256 solo, at K = 576 ...
+    (1, 128, (131, 141), 250, 3),      # ... and 1152
+    (1, 128, (112, 113), 104, 3),      # one, 198, where the split reduction ends: solo
+    (1, 64, (62, 64), 1032, 1),        # nine 128s: dma
+    (1, 128, (81, 83), 170, 1),        # two, 212: dma
+    (1, 128, (50, 51), 1024, 3),       # eight, 320: solo
+    (1, 64, (40, 41), 1033, 1),        # (an odd width)
+    (1, 64, (23, 25), 2050, 1),        # beyond 2048: the general tiles
+    (1, 64, (313, 315), 76, 1)])       # 1541 of one 128: dma
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_wide_tiles_by_rows_reduction_and_width(cuda, B, C, hw, N, k, dtype):
+    """The other lines of that choice, tile counts that are no multiple of 8 among them (their order over the XCDs)."""
+    test_wide_tiles_at_their_edges(cuda, B, C, hw, N, k, dtype)

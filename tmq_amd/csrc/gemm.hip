@@ -577,6 +577,17 @@ __device__ __forceinline__ void load_to_lds(const void *src, unsigned char *dst)
 #endif
 }
 
+// Whether a convolution's tiles of WM x WN fragments (16 rows, 16 columns each) go to the XCDs in contiguous runs for any
+// number of tiles, not only for multiples of 8: those of 64 rows x 128 columns, whose neighbours share most of their input
+// (256 -> 256, 1 x 1, 13671 rows, 428 tiles: 13.8 us without, 11.1 with; 128 -> 348, 3 x 3, 8960 rows, 420 tiles 15.9 and
+// 12.7), and the taller ones where at least three share a row's input over a long reduction (0.72 .. 1.04 over 85 shapes;
+// with one or two 0.86 .. 1.16).
+template <int WM, int WN, class Loader>
+__device__ __forceinline__ bool runs_per_xcd(int tiles_n, int64_t K) {
+    if constexpr (!Loader::kConv || WN != 8) return false;
+    else return WM == 4 || (tiles_n >= 3 && K >= 1024);
+}
+
 // Rows of a BM-row tile as loaded: BM rounded up to whole chunk rounds of T threads (a 112-row tile of four wavefronts
 // is loaded as 128 rows: the 16 extra rows are the next tile's, fetched and never read).
 constexpr int rows_loaded(int BM, int T) { return (BM * 8 + T - 1) / T * T / 8; }
@@ -717,7 +728,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, WGM * WGN > 4 ? 1 : 2) void tile_dm
     __shared__ __attribute__((aligned(16))) _Float16 As[2 * P][rows_loaded(BM, 64 * WGM * WGN) * kPitch];
     int id = blockIdx.x;
     const int G = tiles_m * tiles_n;
-    if ((G & 7) == 0) id = (id & 7) * (G >> 3) + (id >> 3);
+    if ((G & 7) == 0 || runs_per_xcd<WM * WGM, WN * WGN, Loader>(tiles_n, K)) id = xcd_contiguous(id, G);
     const int tm = id / tiles_n, tn = id % tiles_n;
     tile_dma_body<WM, WN, WGM, WGN, P>(ld, native, M, K, N, Kb, Nb, ep, (int64_t)tm * BM, (int64_t)tn * BN, As);
 }
@@ -797,7 +808,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void tile_solo_kernel(Loader ld,
 
     int id = blockIdx.x;
     const int G = tiles_m * tiles_n;
-    if ((G & 7) == 0) id = (id & 7) * (G >> 3) + (id >> 3);
+    if ((G & 7) == 0 || runs_per_xcd<WM * WGM, WN * WGN, Loader>(tiles_n, K)) id = xcd_contiguous(id, G);
     const int tm = id / tiles_n, tn = id % tiles_n;
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
 
@@ -1365,34 +1376,40 @@ int conv_phases(const _Float16 *x, const tmq_conv_phase *phases, int count, cons
 
 // Tiles of 64 rows x 128 or 256 columns for convolutions over a multiple of 64 channels with more than 64 outputs: an
 // im2col tile is fetched once per 128 (256) columns instead of once per 64, and half as many rows per workgroup as in a
-// 128 x 128 tile leave fewer CUs idle in the last wave. Where the line lies, from a sweep over N = 96 .. 512, 64 .. 512
-// channels, 1 x 1 and 3 x 3, 4096 .. 65536 rows (fp16 out, residual and ReLU; what took the shape before = 1):
-//   reductions below 512                            64 x 128 dma   0.76 .. 0.98
-//     ... in whole 256 columns, 448 .. 1100 tiles   64 x 256 solo  0.77 .. 0.93 (64 x 128: 0.80 .. 0.97)
-//     ... in whole 256 columns, more tiles          the old choice (64 x 128: 0.92 .. 0.98, but up to 1.19 into fp32)
-//   up to 512 tiles of 64 x 64 (split reduction)    64 x 128 solo  0.83 .. 0.89 from 192 tiles on up to K = 1536 (K = 4608: 0.97 .. 1.03;
-//                                                   128 tiles: 0.89 .. 0.95 at K <= 640, 1.05 at 1152, 1.2 at 2304)
-//   more of them: N <= 128, up to 512 tiles         0.82 .. 0.89 (dma to K = 768, then solo; 1024 tiles: 0.96 .. 1.04)
-//   129 .. 256                                      64 x 128 solo 0.94 below 448 tiles from K = 1024 on (K = 512: 1.07), else
-//                                                   64 x 256 solo as before
-//   an odd number of 128s (256-wide tiles waste)    solo 0.86 .. 0.94 up to 512 tiles, dma 0.79 .. 0.93 beyond
-//   other widths, up to 1100 tiles                  64 x 256 solo 0.79 .. 1.00
-// 128 -> 128, 3 x 3 on 28 x 28, batch 32: 14.7 -> 13.7 us; 320 -> 76, 1 x 1 on 54 x 54, batch 34: 23.9 -> 18.4.
+// 128 x 128 tile leave fewer CUs idle in the last wave. Where the lines lie, from 1120 shapes (N = 65 .. 2048, odd ones
+// among them, 64 .. 2048 channels, 1 x 1 .. 5 x 5, 300 .. 300000 rows, fp16 and fp32 out; the choice without these tiles = 1):
+//   K < 512: 257 columns and more, any number of tiles      dma   0.57 .. 0.99 (an even number of 128s: up to 1536)
+//            129 .. 256, up to 1024 tiles of 64 x 128       dma   0.75 .. 0.97; from 448 on 64 x 256 solo 0.70 .. 0.95 (more: to 1.21)
+//            65 .. 128, up to 768 and from 1536 on          dma   0.62 .. 0.99 (768 .. 1024: N a multiple of 8 0.82 .. 0.96,
+//                                                           others to 1.06; up to 1536: to 1.10)
+//   where the split reduction is at home, one tile a CU     solo  0.81 .. 0.99 for N a multiple of 8 (others: to 1.48; 64 x 64
+//                                                           tiles of it fill 65 .. 96 of 128 columns; K > 1152: 0.86 .. 1.58)
+//   N <= 128, up to 512 tiles                               dma 0.62 .. 0.96 below K = 1024, solo 0.43 .. 1.02 from there on
+//                                                           (more tiles: 0.74 .. 1.20)
+//   129 .. 256, fewer than 448 tiles from K = 1024 on       solo  0.87 .. 0.99 (more: 64 x 256, the choice without the others)
+//   wider, K < 1024                                         dma   0.49 .. 0.99
+//   wider, up to 768 tiles                                  solo  0.40 .. 0.98 (64 x 256 up to 1.45 here: 257 .. 384 of them
+//                                                           are a second round of the chip for a few)
+//   an odd number of 128s, from 1024 tiles on               dma   0.57 .. 1.03 (others: 0.70 .. 1.17)
+// 128 -> 128, 3 x 3 on 28 x 28, batch 32: 14.7 -> 13.7 us; 320 -> 76, 1 x 1 on 54 x 54, batch 34: 23.9 -> 18.4;
+// 3072 -> 768, 1 x 1 on 14 x 14, batch 32: 32.7 -> 30.1. (All with the tiles in XCD runs, runs_per_xcd.)
 enum class WideTile { kNone, kDma128, kSolo128, kSolo256 };
 WideTile wide_tile(int64_t M, int64_t K, int64_t N) {
-    if (N <= 64) return WideTile::kNone;
+    if (N <= 64 || N > 2048) return WideTile::kNone;
     const int64_t tm = (M + 63) / 64, t64 = tm * ((N + 63) / 64), n128 = (N + 127) / 128, t = tm * n128;
-    const bool whole256 = n128 % 2 == 0;
+    if (split_reduction_pays(M, K, N))
+        return K >= 512 && N % 8 == 0 && t <= 256 && ((t >= 192 && K <= 1152) || (t >= 128 && t64 >= 256 && K <= 640)) ? WideTile::kSolo128
+                                                                                                                   : WideTile::kNone;
     if (K < 512) {
-        if (t64 <= K / 2) return WideTile::kNone;                  // the split reduction's
-        return !whole256 || t < 448 ? WideTile::kDma128 : t <= 1100 ? WideTile::kSolo256 : WideTile::kNone;
+        if (n128 == 2 && t >= 448 && t <= 1024) return WideTile::kSolo256;
+        const bool small = n128 == 1 ? t <= 768 || (t <= 1024 && N % 8 == 0) : t <= (n128 == 2 ? 1024 : 1536);
+        return small || (n128 % 2 == 1 && (n128 > 1 || t > 1536)) ? WideTile::kDma128 : WideTile::kNone;
     }
-    if (t64 <= 512)
-        return (t >= 192 && K <= 1536) || (t >= 128 && t64 >= 256 && K <= 640) ? WideTile::kSolo128 : WideTile::kNone;
-    if (n128 == 1) return t > 512 ? WideTile::kNone : K <= 768 ? WideTile::kDma128 : WideTile::kSolo128;
+    if (n128 == 1) return t > 512 ? WideTile::kNone : K < 1024 ? WideTile::kDma128 : WideTile::kSolo128;
     if (n128 == 2) return t < 448 && K >= 1024 ? WideTile::kSolo128 : WideTile::kSolo256;
-    if (!whole256) return t <= 512 ? WideTile::kSolo128 : WideTile::kDma128;
-    return t <= 1100 ? WideTile::kSolo256 : WideTile::kNone;
+    if (K < 1024) return WideTile::kDma128;
+    if (t <= 768) return WideTile::kSolo128;
+    return n128 % 2 == 1 && t > 1024 ? WideTile::kDma128 : WideTile::kNone;
 }
 // What those tiles' loader takes.
 bool wide_conv_ok(const void *x, const tmq_conv_shape *s, int64_t M) {
