@@ -284,3 +284,20 @@ def test_phases_alone_or_of_long_reductions_take_their_own_launches(cuda, cin, c
 def test_wide_tiles_by_rows_reduction_and_width(cuda, B, C, hw, N, k, dtype):
     """The other lines of that choice, tile counts that are no multiple of 8 among them (their order over the XCDs)."""
     test_wide_tiles_at_their_edges(cuda, B, C, hw, N, k, dtype)
+
+
+@pytest.mark.parametrize("M,K,N", [(16448, 4096, 24), (16448, 4032, 30), (129, 4100, 7)])
+def test_few_outputs_on_either_tile(cuda, M, K, N):
+    """Dense rows into at most 32 outputs below and from K = 4096 on (128 x 32 and 64 x 64 tiles), and single elements: exact."""
+    from tmq_amd import ops
+    g = torch.Generator(device=cuda).manual_seed(M + K)
+    Wt = torch.randint(-1, 2, (N, K), device=cuda, generator=g).float()
+    x = torch.randint(-2, 3, (M, K), device=cuda, generator=g).half()
+    nw = ops.NativeWeights(ops.compactify_ternary(Wt), N)
+    assert torch.equal(ops.ternary_linear(x, nw).cpu(), (x.cpu().float() @ Wt.cpu().t()))
+
+
+@pytest.mark.parametrize("B,C,hw,N", [(1, 34, (99, 28), 14), (1, 36, (99, 28), 14), (2, 134, (9, 28), 31)])
+def test_few_outputs_of_odd_channels_on_either_tile(cuda, B, C, hw, N):
+    """Convolutions into at most 32 outputs that read single elements (64 x 64 tiles) and halves of 8 bytes (128 x 32)."""
+    test_wide_tiles_at_their_edges(cuda, B, C, hw, N, 3, torch.float32)

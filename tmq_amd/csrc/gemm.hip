@@ -1064,8 +1064,12 @@ int dispatch_tile(const Loader &ld, const void *native, int64_t M, int64_t K, in
     // At most 32 columns: 128 x 32 tiles, four wavefronts of 32 rows each, where a 64 x 64 tile's second wavefront would
     // multiply columns that don't exist. Convolutions into 16, 24 and 32 channels against 64 x 64 tiles (rows 784 .. 50176):
     // 64 -> 32, 3 x 3 on 56 x 56, batch 16 10.1 -> 8.6 us; 16 -> 16, 5 x 5 9.1 -> 7.9; 104 -> 24, 3 x 3 18.3 -> 16.3; 256 -> 16,
-    // 1 x 1 on 28 x 28, batch 16 5.8 -> 5.1; 0.85 .. 0.98 throughout, 17 -> 32 (single elements) 0.95 .. 1.02.
-    if (N <= 32) {
+    // 1 x 1 on 28 x 28, batch 16 5.8 -> 5.1; 0.85 .. 1.01 throughout. Not for dense rows from K = 4096 on (K = 4096, M = 60000
+    // 103.9 -> 112.1 us; shorter ones 0.73 .. 1.02) or through registers (K = 520, M = 30000 8.7 -> 10.2), nor where single
+    // elements are read (190 -> 13, 5 x 5, 5712 rows 415 -> 456; 0.88 .. 1.10).
+    bool narrow = N <= 32 && (Loader::kConv || (Loader::kDirect && K < 4096));
+    if constexpr (std::is_same<Loader, ConvLoader<false>>::value) narrow = narrow && ld.quads;
+    if (narrow) {
         if constexpr (Loader::kDirect) return launch_tile_dma<2, 2, 4, 1, 1>(ld, native, M, K, N, ep, stream);
         else return K >= 16 * kBK ? launch_tile<2, 2, 4, 1, 2>(ld, native, M, K, N, ep, stream) : launch_tile<2, 2, 4, 1, 1>(ld, native, M, K, N, ep, stream);
     }
