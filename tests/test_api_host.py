@@ -194,3 +194,38 @@ def test_phase_plan_goes_with_the_native_weights():
         layer._native = ("key", layer.__dict__.pop("_test_phases"))
         drop()
         assert layer._native is None and layer._phases is None and held() is None
+
+
+def test_native_one_call_forms_release_the_interpreter_lock():
+    """ops' one-call forms launch without the interpreter lock, as calls through ctypes do: another thread runs while the
+    main one does nothing but call them (with the switch interval out of the way, a thread only gets the lock when it is
+    released). CPU tensors, which they decline."""
+    import sys
+    import threading
+    import time
+    ops = pytest.importorskip("tmq_amd.ops")
+    ext = ops.ext
+    if ext is None:
+        pytest.skip("the extension is not built")
+    x, w = torch.zeros(1, 64), torch.zeros(1024, dtype=torch.uint8)
+    image, words = x.view(1, 1, 8, 8), torch.zeros(1, dtype=torch.int32)      # (made here: torch's own calls release it too)
+    calls = [lambda: ext.plain_linear(x, w, 64, 16, None, None, None, False, False, True),
+             lambda: ext.plain_conv(image, words, True, 1, 1, 1, 1, (1, 1, 0, 0, 0, 0, 1, 1), None, None, None, False, False, True),
+             lambda: ext.plain_softstep_fwd([x], 3.0, False, 5.0, 0.0), lambda: ext.plain_softstep_bwd([x], [x], None, 3.0, 5.0, 0.0)]
+    interval = sys.getswitchinterval()
+    for call in calls:
+        gate, ran = threading.Lock(), []
+        gate.acquire()
+        other = threading.Thread(target=lambda: (gate.acquire(), ran.append(True)))
+        other.start()
+        sys.setswitchinterval(1000.0)
+        try:
+            gate.release()
+            end = time.monotonic() + 5.0
+            while not ran and time.monotonic() < end:
+                assert call() is None
+            got = bool(ran)
+        finally:
+            sys.setswitchinterval(interval)
+        other.join()
+        assert got

@@ -640,11 +640,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("softstep_fwd_all", &softstep_fwd_all);
     m.def("softstep_bwd_all", &softstep_bwd_all);
     m.def("loss_state", &loss_state);
-    // additive: the plain calls of tmq_amd/ops.py
-    m.def("plain_linear", &plain_linear);
-    m.def("plain_conv", &plain_conv);
-    m.def("plain_softstep_fwd", &plain_softstep_fwd);
-    m.def("plain_softstep_bwd", &plain_softstep_bwd);
+    // additive: the plain calls of tmq_amd/ops.py (without the interpreter lock, which the ctypes route releases too: a
+    // launch may wait for room in its queue)
+    typedef pybind11::call_guard<pybind11::gil_scoped_release> unlocked;
+    m.def("plain_linear", &plain_linear, unlocked());
+    m.def("plain_conv", &plain_conv, unlocked());
+    m.def("plain_softstep_fwd", &plain_softstep_fwd, unlocked());
+    m.def("plain_softstep_bwd", &plain_softstep_bwd, unlocked());
     // tmq_native (tmq/tmq_native.cpp:550-555)
     m.def("compactify_ternary", &compactify_ternary);
     m.def("compress_ternary", &compress_ternary);
