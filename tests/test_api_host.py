@@ -229,3 +229,15 @@ def test_native_one_call_forms_release_the_interpreter_lock():
             sys.setswitchinterval(interval)
         other.join()
         assert got
+
+
+@pytest.mark.parametrize("given", [dict(nw=object()), dict(stride=2), dict(padding=1), dict(dilation=(1, 2)), dict(first=(0, 1))])
+def test_phases_come_with_their_own_geometry(given):
+    """ternary_conv2d_into(phases=...) refuses the arguments of a single convolution instead of ignoring them."""
+    from types import SimpleNamespace
+    from tmq_amd import ops
+    plan = SimpleNamespace(run=lambda *a: "ran")
+    args = dict(nw=None)
+    assert ops.ternary_conv2d_into(None, None, **args, stride=1, padding=(0, 0), dilation=(1, 1), phases=plan) == "ran"
+    with pytest.raises(ValueError, match="phases"):
+        ops.ternary_conv2d_into(None, None, **{**args, **given}, phases=plan)

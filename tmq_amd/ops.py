@@ -794,11 +794,13 @@ def ternary_conv2d_into(out: torch.Tensor, x: torch.Tensor, nw: NativeWeights, s
     fp32, e.g. big[:, :, 1::2, 0::2]): output position (first[0] + i, first[1] + j) of the convolution goes to
     out[:, :, i, j]; positions of the convolution outside that h x w window are dropped. `residual`, when given, is a
     view with out's shape and strides. One launch, no temporary. x must already be fp16.
-    phases (then nw is None and `out` the whole dense channels_last tensor): several convolutions of x, each with weights,
-    padding and a share of `out` of its own, as a ConvPhases."""
-    if phases is not None:
-        return phases.run(out, x, scale, bias, residual, relu)
+    phases (then nw is None, the geometry is left at its defaults and `out` is the whole dense channels_last tensor):
+    several convolutions of x, each with weights, padding and a share of `out` of its own, as a ConvPhases."""
     pair = lambda v: tuple(v) if isinstance(v, (tuple, list)) else (v, v)
+    if phases is not None:
+        if nw is not None or (pair(stride), pair(padding), pair(dilation), pair(first)) != ((1, 1), (0, 0), (1, 1), (0, 0)):
+            raise ValueError("ternary_conv2d_into: phases have weights and geometry of their own")
+        return phases.run(out, x, scale, bias, residual, relu)
     (sy, sx), (py, px), (dy, dx) = pair(stride), pair(padding), pair(dilation)
     (py, py_end), (px, px_end) = pair(py), pair(px)
     if not x.is_cuda or x.dim() != 4 or out.dim() != 4 or out.device != x.device:
