@@ -104,3 +104,71 @@ def test_soft_weights(cuda, by_ctypes):
         ops.softstep_fwd_all([ws[0].half()], 3.5)
     with pytest.raises(RuntimeError):
         ops.softstep_fwd_all([ws[0].cpu()], 3.5)
+
+
+def test_linear_form_is_taken_and_declined(cuda):
+    """plain_linear itself: a tensor for the plain case, None for everything else."""
+    from tmq_amd import ops
+    K, N = 512, 48
+    nw = ops.NativeWeights(_weights(cuda, (N, K), 1), N)
+    call = lambda x, scale=None, bias=None, residual=None, prescale=True: ops.ext.plain_linear(x, nw.buf, K, N, scale, bias, residual, False, False,
+                                                                                               prescale)
+    row, per = torch.randn(3, K, device=cuda), torch.ones(N, device=cuda)
+    for x in (row, row[:1], row.half(), row[0], row.half().view(1, 3, K), torch.randn(40, K, device=cuda), torch.randn(40, K, device=cuda).half()):
+        y = call(x, per, per)
+        assert y is not None and y.shape == x.shape[:-1] + (N,)
+        assert torch.equal(y, ops.ternary_linear(x, nw, scale=per, bias=per))
+    flat = torch.randn(3 * K + 1, device=cuda)
+    res = torch.zeros(3, N, device=cuda)
+    assert call(row, residual=res) is not None
+    for declined in (lambda: call(flat[1:].view(3, K)),                          # fp32 rows off a 16-byte boundary: the splitter's route
+                     lambda: call(torch.randn(1100, K, device=cuda), prescale=False),     # the one-pass kernel's
+                     lambda: call(row.double()), lambda: call(row.cpu()), lambda: call(row.t().contiguous().t()), lambda: call(row[:0]),
+                     lambda: call(row[:, :-1].contiguous()), lambda: call(row, scale=per.cpu()), lambda: call(row, bias=per.double()),
+                     lambda: call(row, scale=per[:-1]), lambda: call(row, bias=torch.ones(2 * N, device=cuda)[::2]),
+                     lambda: call(row, residual=res[:2]), lambda: call(row, residual=res.half()), lambda: call(row, residual=res.t().contiguous().t())):
+        assert declined() is None
+
+
+@pytest.mark.parametrize("depthwise", [False, True])
+def test_convolution_form_is_taken_and_declined(cuda, depthwise):
+    from tmq_amd import ops
+    C = 24
+    N = C if depthwise else 40
+    words = _weights(cuda, (N, 1 if depthwise else C, 3, 3), 2)
+    w = words if depthwise else ops.NativeWeights(words, N, (3, 3)).buf
+    geometry = (1, 1, 1, 1, 1, 1, 1, 1)
+    call = lambda x, scale=None, bias=None, residual=None, prescale=True, words=w, geometry=geometry: \
+        ops.ext.plain_conv(x, words, depthwise, C, N, 3, 3, geometry, scale, bias, residual, False, False, prescale)
+    planar = torch.randn(2, C, 9, 8, device=cuda)
+    last, per = planar.contiguous(memory_format=torch.channels_last), torch.ones(N, device=cuda)
+    for x in (planar, last, last.half()):
+        y = call(x, per, per)
+        assert y is not None and y.shape == (2, N, 9, 8) and y.is_contiguous(memory_format=torch.channels_last)
+    res = torch.zeros_like(y)
+    assert call(last, residual=res) is not None and call(last.half(), prescale=False) is not None
+    for declined in (lambda: call(planar.half()), lambda: call(planar, prescale=False), lambda: call(last.cpu()), lambda: call(last.double()),
+                     lambda: call(planar.transpose(2, 3)), lambda: call(planar[0]), lambda: call(planar[:0]), lambda: call(planar[:, :-1].contiguous()),
+                     lambda: call(last, scale=per.cpu()), lambda: call(last, bias=per[:-1]), lambda: call(last, scale=per.double()),
+                     lambda: call(last, residual=res.contiguous()), lambda: call(last, residual=res[:1]), lambda: call(last, residual=res.half()),
+                     lambda: call(last, words=w.cpu()), lambda: call(last, geometry=(1, 1, -9, 1, -9, 1, 1, 1))):
+        assert declined() is None
+
+
+def test_soft_weight_forms_are_taken_and_declined(cuda):
+    from tmq_amd import ops
+    ws = [torch.rand(n, device=cuda) for n in (5, 4096)]
+    gs = [torch.randn_like(w) for w in ws]
+    up = torch.ones(1, device=cuda)
+    fwd = lambda w, loss=True: ops.ext.plain_softstep_fwd(w, 3.5, loss, 5.0, 1e-3)
+    bwd = lambda w, g, u=None: ops.ext.plain_softstep_bwd(w, g, u, 3.5, 5.0, 1e-3)
+    assert fwd(ws) is not None and fwd(ws, False)[1] is None and bwd(ws, gs) is not None and bwd(ws, gs, up) is not None
+    many = [torch.rand(7, device=cuda) for _ in range(100)]                      # beyond the in-launch loss: with a workspace
+    ys, loss = fwd(many)
+    assert len(ys) == 100 and abs(loss.item() - sum(fwd([w])[1].item() for w in many)) <= 1e-5 * abs(loss.item())
+    square = torch.rand(8, 8, device=cuda)
+    for declined in (lambda: fwd([]), lambda: fwd([ws[0], ws[1].half()]), lambda: fwd([ws[0].cpu()]), lambda: fwd([square.t()]),
+                     lambda: bwd(ws, gs[:1]), lambda: bwd(ws, [gs[0], gs[1].half()]), lambda: bwd(ws, [gs[1], gs[0]]),
+                     lambda: bwd(ws, [gs[0], gs[1].cpu()]), lambda: bwd([square], [square.t()]), lambda: bwd(ws, gs, up.cpu()),
+                     lambda: bwd(ws, gs, up.double()), lambda: bwd(ws, gs, torch.ones(2, device=cuda))):
+        assert declined() is None
