@@ -502,8 +502,8 @@ def bench_layers(args, torch):
     finally:
         t.set_compact_output_dtype(prev)
     byts = (xt[0].numel() + y.numel()) * 2
-    res["convtranspose_128_64_k4s2"] = {"us": round(us, 3), "launches": 4, "out_MB": round(y.numel() * 2 / 1e6, 1), "gbs": round(byts / us / 1e3, 1),
-                                        "note": "one stride-1 implicit-GEMM convolution per output phase, written in place (tmq_ternary_conv2d_view)"}
+    res["convtranspose_128_64_k4s2"] = {"us": round(us, 3), "launches": 1, "out_MB": round(y.numel() * 2 / 1e6, 1), "gbs": round(byts / us / 1e3, 1),
+                                        "note": "a stride-1 implicit-GEMM convolution per output phase, the four in one launch, written in place (tmq_ternary_conv2d_phases)"}
     # a small-image network's opening (3 -> 64, 3 x 3, stride 1, 32 x 32, batch 128, NCHW fp16 in, fp16 NHWC out): the
     # pixel-pair form of Conv2d.compact_forward (repack launch + one convolution launch; tmq/tmq.py:822-871)
     first = torch.nn.Sequential(torch.nn.Conv2d(3, 64, 3, 1, 1, bias=True))
