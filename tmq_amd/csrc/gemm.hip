@@ -579,9 +579,9 @@ __device__ __forceinline__ void load_to_lds(const void *src, unsigned char *dst)
 
 // Whether a convolution's tiles of WM x WN fragments (16 rows, 16 columns each) go to the XCDs in contiguous runs for any
 // number of tiles, not only for multiples of 8: those of 64 rows x 128 columns, whose neighbours share most of their input
-// (256 -> 256, 1 x 1, 13671 rows, 428 tiles: 13.8 us without, 11.1 with; 128 -> 348, 3 x 3, 8960 rows, 420 tiles 15.9 and
-// 12.7), and the taller ones where at least three share a row's input over a long reduction (0.72 .. 1.04 over 85 shapes;
-// with one or two 0.86 .. 1.16).
+// (1024 -> 256, 1 x 1, 13671 rows, 428 tiles: 14.0 us without, 12.1 with; 43 shapes of 129 .. 256 columns 0.95 .. 1.20 of the
+// choice without these tiles, in runs 0.87 .. 0.99), and the taller ones where at least three share a row's input over a long
+// reduction (0.72 .. 1.04 over 85 shapes; with one or two 0.86 .. 1.16).
 template <int WM, int WN, class Loader>
 __device__ __forceinline__ bool runs_per_xcd(int tiles_n, int64_t K) {
     if constexpr (!Loader::kConv || WN != 8) return false;
@@ -1396,7 +1396,8 @@ int conv_phases(const _Float16 *x, const tmq_conv_phase *phases, int count, cons
 //                                                           are a second round of the chip for a few)
 //   an odd number of 128s, from 1024 tiles on               dma   0.57 .. 1.03 (others: 0.70 .. 1.17)
 // 128 -> 128, 3 x 3 on 28 x 28, batch 32: 14.7 -> 13.7 us; 320 -> 76, 1 x 1 on 54 x 54, batch 34: 23.9 -> 18.4;
-// 3072 -> 768, 1 x 1 on 14 x 14, batch 32: 32.7 -> 30.1. (All with the tiles in XCD runs, runs_per_xcd.)
+// 3072 -> 768, 1 x 1, 6314 rows: 42.5 -> 32.0. (All with the tiles in XCD runs, runs_per_xcd. The lines as they are, over 1940
+// shapes: 0.92 on average, 1.08 at most.)
 enum class WideTile { kNone, kDma128, kSolo128, kSolo256 };
 WideTile wide_tile(int64_t M, int64_t K, int64_t N) {
     if (N <= 64 || N > 2048) return WideTile::kNone;

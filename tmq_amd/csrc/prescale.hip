@@ -379,7 +379,7 @@ inline bool planar_vec(const void *x, int64_t HW) { return HW % 4 == 0 && aligne
 // Whether the reordering launch beats the conversion in place followed by a strided copy. Every tile costs a workgroup
 // that reduces the partial maxima again, however little of it exists (4.5 ns each beyond the first round, 5.6 without quad
 // loads), where the two launches cost 5 us more at rest and 2.7 ns per 4096 values. 618 shapes of 3e4, 1e6 and 1.2e7 values,
-// 2 .. 2048 channels, planes of 2 .. 111222 pixels, copy = 1: up to 1.00 where this says yes, 0.71 and more where it says no --
+// 2 .. 2048 channels, planes of 2 .. 111222 pixels, copy = 1: up to 1.00 where this says yes, 0.78 and more where it says no --
 // [64, 3, 224, 224] 1.94, [20000, 8, 3, 3] 5.8, [125000, 2, 2, 2] 38; against 0.38 for [32, 128, 28, 28], 0.42 for [64, 512, 7, 7].
 inline bool planar_tiles_pay(const void *x, int64_t B, int64_t C, int64_t HW) {
     const int64_t n = B * C * HW, tiles = planar_tiles(B, C, HW);
