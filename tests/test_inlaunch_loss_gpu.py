@@ -310,3 +310,31 @@ def test_full_size_fused_pass(cuda):
         assert _same_bits(a, b)
     assert abs(got[3].item() - want[3].item()) <= 1e-7 * abs(want[3].item())
     assert int(state.count_nonzero()) == 0
+
+
+def test_threads_on_streams_of_their_own(cuda):
+    """The loss of several threads at once, each on its stream with an accumulator made on first use: every value is the one of
+    a thread alone, and the accumulators end at zero."""
+    import threading
+    from tmq_amd import ops
+    ws = [torch.from_numpy(_inputs(n, 30 + i)[0]).to(cuda) for i, n in enumerate([9408, 36864, 2049])]
+    want = ops.softstep_fwd_all(ws, 2.236133, True, 5.0, 5e-4)[1].item()
+    torch.cuda.synchronize()
+    got, states, start = [], [], threading.Barrier(4)
+
+    def work():
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            start.wait()
+            losses = [ops.softstep_fwd_all(ws, 2.236133, True, 5.0, 5e-4)[1] for _ in range(50)]
+            states.append(ops.loss_state(cuda))
+        side.synchronize()
+        got.extend(v.item() for v in losses)
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(got) == 200 and set(got) == {want}
+    assert all(int(s.count_nonzero()) == 0 for s in states)

@@ -129,18 +129,21 @@ c10::optional<torch::Tensor> loss_state(int64_t device_index) {
     const c10::DeviceGuard on(device);
     hipStream_t stream = at::hip::getCurrentHIPStream((c10::DeviceIndex)device_index).stream();
     const auto key = std::make_pair((int)device_index, (void *)stream);
-    std::lock_guard<std::mutex> lock(guard);
-    auto it = states.find(key);
-    if (it == states.end()) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
-            (void)hipGetLastError();                    // the default stream while another one is being captured
-            return c10::nullopt;
-        }
-        if (capture != hipStreamCaptureStatusNone) return c10::nullopt;
-        it = states.emplace(key, torch::zeros({(int64_t)tmq_loss_state_bytes()}, torch::dtype(torch::kUInt8).device(device))).first;
+    {
+        std::lock_guard<std::mutex> lock(guard);
+        const auto it = states.find(key);
+        if (it != states.end()) return it->second;
     }
-    return it->second;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
+        (void)hipGetLastError();                        // the default stream while another one is being captured
+        return c10::nullopt;
+    }
+    if (capture != hipStreamCaptureStatusNone) return c10::nullopt;
+    // (made without the lock: an allocation may call into Python, and callers come with and without the interpreter lock)
+    auto made = torch::zeros({(int64_t)tmq_loss_state_bytes()}, torch::dtype(torch::kUInt8).device(device));
+    std::lock_guard<std::mutex> lock(guard);
+    return states.emplace(key, std::move(made)).first->second;
 }
 
 // y_l and the loss of dense fp32 weights on one device; a status of tmq_hip.h.
