@@ -285,7 +285,7 @@ typedef struct tmq_epilogue {
  * magnitude go through tmq_f32_prescale first (exact power-of-two scaling, undone in the per-channel scale of
  * the epilogue); the Python / PyTorch bindings of this library always do, because the reference multiplies
  * fp32 activations in fp32 and has no such limit. One case needs no prescale: fp32 rows for which
- * tmq_fp32_rows_self_scaled_for returns 1 (one row, or two over a small layer) are scaled inside the kernel, each by
+ * tmq_fp32_rows_one_launch returns 1 (one row, or a few short ones) are scaled inside the kernel, each by
  * its own power of two, and may have any magnitude.
  * Arithmetic: exact products, fp32 accumulation. One fp16 row (M == 1) with K a multiple of 256 from 2048 to 16384
  * runs on the 8-bit matrix instructions (weights as fp8, the row as four exact bf8 terms); there the hardware adds
@@ -303,8 +303,8 @@ int tmq_ternary_linear(const void *x, int x_dtype, int64_t M, int64_t K, const v
  * workgroups -- today 17 .. 32 fp16 rows over 2^28 weights or more -- runs as slices of whole 256-index weight
  * blocks with fp32 partial sums in the workspace, added in slice order by a second launch (deterministic, no
  * atomics). fp32 rows (the reference's kernels take fp32 activations, tmq/tmq_cuda.cu:242-427) use the workspace
- * differently, unless tmq_ternary_linear scales them itself in one launch (tmq_fp32_rows_self_scaled_for). Up to
- * sixteen rows: a first launch splits every row into two fp16 rows (hi = fp16(s x), lo = fp16(s x - hi), s the row's
+ * differently, unless tmq_ternary_linear scales them itself in one launch (tmq_fp32_rows_one_launch). Other rows, up to
+ * sixteen: a first launch splits every row into two fp16 rows (hi = fp16(s x), lo = fp16(s x - hi), s the row's
  * own power of two: any magnitude, 22 significant bits), the fp16 weight-stream kernel then runs once over twice the
  * rows (from nine rows: twice, over about half of them each) and adds each pair in its epilogue (256 + 4 M K" bytes,
  * K" = K rounded up to a multiple of 256: the pairs of a ragged length are written with zeros behind). Seventeen
@@ -345,6 +345,12 @@ int tmq_fp32_rows_self_scaled(const void *x, int64_t M, int64_t K);
 /* The same question for a layer of N channels: also 1 for two 16-byte aligned rows with K a multiple of 256 up to
  * 6144 and N <= 6144 (each row scaled by its own power of two inside the one launch). */
 int tmq_fp32_rows_self_scaled_for(const void *x, int64_t M, int64_t K, int64_t N);
+/* 1 when tmq_ternary_linear(x, TMQ_F32, M, K, ...) takes these 16-byte aligned rows in one launch whatever their
+ * magnitude: the rows of tmq_fp32_rows_self_scaled_for, and up to sixteen short ones (1 .. 8 rows of up to 2048 values
+ * against up to 3 2^23 weights, of up to 4096 values against up to 4096 channels; 9 .. 16 of up to 2048 against up to
+ * 2^25 weights), each scaled by its own power of two and split into two fp16 terms by the workgroups that multiply it.
+ * A workspace is not used. */
+int tmq_fp32_rows_one_launch(const void *x, int64_t M, int64_t K, int64_t N);
 
 /* Range handling for fp32 activations (no counterpart in the reference, whose kernels multiply fp32
  * activations in fp32, tmq/tmq_cuda.cu:242-427). Scans n fp32 values and writes prescale[0] = s,

@@ -1229,8 +1229,7 @@ int launch_rows_split(const void *x, int64_t M, int64_t K, const void *native, i
 // Two to sixteen fp32 rows over whole weight blocks: split once into fp16 row pairs (prescale.hip), then one pass of
 // the fp16 weight-stream kernel over twice the rows (mid.hip; two passes of about half the rows each from nine rows)
 // -- against the kernel that splits every block's activations on the fly in each workgroup: 8192^2, 4 rows
-// 17.4 -> 10.8 us, 8 rows 25.5 -> 11.7 us; and on short reductions against a prescale launch in front of the skinny
-// kernels: K = 1024, N = 4096, 4 rows 7.9 -> 6.0 us, 8 rows 9.5 -> 6.4, 16 rows 12.3 -> 9.4.
+// 17.4 -> 10.8 us, 8 rows 25.5 -> 11.7 us. Short rows are split by the launch that multiplies them (rows32.hip).
 int launch_split_rows(const float *x, int64_t M, int64_t K, int64_t Kp, int64_t group, void *x16, float *row_scale, void *stream);
 inline int64_t padded_blocks(int64_t K) { return (K + kKB - 1) / kKB * kKB; }   // the weight stream wants whole 256-index blocks
 int launch_stream_pairs(const void *x16, int64_t M, int64_t K, const void *native, int64_t N, const float *row_scale,
@@ -1470,6 +1469,8 @@ size_t tmq_ternary_linear_workspace_bytes(int x_dtype, int64_t M, int64_t K, int
 
 int tmq_ternary_linear_ws(const void *x, int x_dtype, int64_t M, int64_t K, const void *native, int64_t N,
                           const tmq_epilogue *epilogue, void *y, void *workspace, size_t workspace_bytes, void *stream) {
+    if (x_dtype == TMQ_F32 && tmq_fp32_rows_one_launch(x, M, K, N))                  // nothing to prepare
+        return tmq_ternary_linear(x, x_dtype, M, K, native, N, epilogue, y, stream);
     if (x && native && y && x_dtype == TMQ_F32 && N > 0 && workspace && aligned16(workspace) && aligned16(native) &&
         row_pairs_ok(x, M, K, N) && workspace_bytes >= row_pairs_bytes(M, K)) {
         tmq_epilogue e = {nullptr, nullptr, nullptr, 0, TMQ_F32};

@@ -10,19 +10,13 @@
 // precision of 2^-35 of that maximum, which is below the rounding of the fp32 accumulation.
 #include "common.h"
 #include "mfma.h"
-
-#include <math.h>
+#include "range.h"
 
 namespace tmq {
 namespace {
 
 constexpr int kPartials = 1024;           // partial maxima of the multi-block scan
 constexpr int64_t kSingleMax = 1 << 16;   // up to here one workgroup does everything in one launch
-
-__device__ __forceinline__ float finite_abs(float v) {
-    const float a = __builtin_fabsf(v);
-    return a < INFINITY ? a : 0.f;          // NaN and Inf take no part in the maximum (they propagate anyway)
-}
 
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
@@ -43,19 +37,6 @@ __device__ __forceinline__ float block_max(float v, float *lds /* >= 17 floats *
     }
     __syncthreads();
     return lds[16];
-}
-
-// s = 2^(11 - e) for amax in [2^(e-1), 2^e), kept inside the normal range together with its reciprocal.
-__device__ __forceinline__ void make_prescale(float amax, float &s, float &inv) {
-    s = 1.f;
-    inv = 1.f;
-    if (!(amax > 0.f)) return;
-    int e;
-    (void)frexpf(amax, &e);
-    int p = 11 - e;
-    p = p > 126 ? 126 : (p < -126 ? -126 : p);
-    s = ldexpf(1.f, p);
-    inv = ldexpf(1.f, -p);
 }
 
 __device__ __forceinline__ float scan_abs_max(const float *__restrict__ x, int64_t n, int64_t first, int64_t stride, bool vec) {

@@ -274,7 +274,7 @@ void check_mm_args(const torch::Tensor &lhs, const torch::Tensor &weights, int64
 // rows run the fp16 kernels over the two fp16 terms, y = W hi + W lo, and few rows the kernels that split on the fly.
 torch::Tensor linear_f32(const torch::Tensor &x, int64_t M, int64_t K, const torch::Tensor &native, int64_t columns,
                          torch::Tensor &y, const char *name) {
-    if (tmq_fp32_rows_self_scaled_for(x.data_ptr(), M, K, columns)) {   // one row (two over a small layer) the kernel scales itself: one launch
+    if (tmq_fp32_rows_one_launch(x.data_ptr(), M, K, columns)) {   // one row, or a few short ones, the kernel scales itself
         check(tmq_ternary_linear(x.data_ptr(), TMQ_F32, M, K, native.data_ptr(), columns, nullptr, y.data_ptr(), stream_of(x)), name);
         return y;
     }
@@ -533,7 +533,7 @@ Maybe plain_linear(const torch::Tensor &x, const torch::Tensor &native, int64_t 
     size_t bytes = 0;
     if (!f32) {
         bytes = M > 16 && (M <= 32 || K % 64) ? tmq_ternary_linear_workspace_bytes(TMQ_F16, M, K, N) : 0;
-    } else if (!(M <= 2 && tmq_fp32_rows_self_scaled_for(x.data_ptr(), M, K, N))) {
+    } else if (!(M <= 16 && tmq_fp32_rows_one_launch(x.data_ptr(), M, K, N))) {
         if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 || (!prescale && M >= 1024 && N <= 128)) return c10::nullopt;
         bytes = tmq_ternary_linear_workspace_bytes(TMQ_F32, M, K, N);
         if (!bytes) return c10::nullopt;

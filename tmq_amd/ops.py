@@ -660,9 +660,9 @@ def ternary_linear(x: torch.Tensor, nw: NativeWeights, scale=None, bias=None, re
         raise RuntimeError(f"ternary_linear: activations have {x.shape[-1]} features, weights expect {nw.K}")
     M = x.numel() // nw.K if nw.K else 0
     pairs = 0
-    if (x.dtype == torch.float32 and 1 <= M <= 2 and x.is_contiguous()
-            and _lib().tmq_fp32_rows_self_scaled_for(ptr(x), M, nw.K, nw.N)):
-        pass            # one row (two over a small layer) the kernel scales itself, any magnitude: one launch
+    if (x.dtype == torch.float32 and 1 <= M <= 16 and x.is_contiguous()
+            and _lib().tmq_fp32_rows_one_launch(ptr(x), M, nw.K, nw.N)):
+        pass            # one row, or a few short ones, the kernel scales itself, any magnitude: one launch
     elif (x.dtype == torch.float32 and M >= 1 and x.is_contiguous() and x.data_ptr() % 16 == 0
           and not (not _fp32_prescale and M >= 1024 and nw.N <= 128)
           and _lib().tmq_ternary_linear_workspace_bytes(_capi.F32, M, nw.K, nw.N)):
