@@ -30,6 +30,14 @@
 #include <type_traits>
 
 namespace tmq {
+
+// ring.hip: most of these problems, with everything a workgroup waits for asked for at once
+bool ring_ok(int64_t M, int64_t K, int64_t N, const float *scale, const float *bias, const void *residual, const void *y);
+int launch_ring_dense(const void *x, int64_t M, int64_t K, const void *native, int64_t N, const float *scale, const float *bias,
+                      const void *residual, int relu, void *y, int y_f16, const PairMap *pairs, void *stream);
+int launch_ring_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale, const float *bias,
+                     const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream);
+
 namespace {
 
 __device__ const u32x4 kZeroChunk[8] = {};   // 128 zero bytes: the source of padding taps / the K tail
@@ -1068,6 +1076,8 @@ bool mid_dense_ok(const void *x, int64_t M, int64_t K) {
 
 int launch_mid_dense(const void *x, int64_t M, int64_t K, const void *native, int64_t N, const float *scale,
                      const float *bias, const void *residual, int relu, void *y, int y_f16, void *stream) {
+    if (ring_ok(M, K, N, scale, bias, residual, y))
+        return launch_ring_dense(x, M, K, native, N, scale, bias, residual, relu, y, y_f16, nullptr, stream);
     MidEpilogue ep{scale, bias, residual, y, relu, y_f16};
     return dispatch(DenseRows{static_cast<const _Float16 *>(x), M, K}, native, M, K, N, ep, stream);
 }
@@ -1076,7 +1086,10 @@ int launch_mid_dense(const void *x, int64_t M, int64_t K, const void *native, in
 int launch_mid_dense_pairs(const void *x16, int64_t M16, int64_t K, const void *native, int64_t N, const float *scale,
                            const float *bias, const void *residual, int relu, void *y, int y_f16, int64_t rows_out,
                            const float *group_scale, void *stream) {
-    MidEpilogueT<PairMap> ep{scale, bias, residual, y, relu, y_f16, PairMap{rows_out, group_scale}};
+    const PairMap map{rows_out, group_scale};
+    if (ring_ok(M16, K, N, scale, bias, residual, y))
+        return launch_ring_dense(x16, M16, K, native, N, scale, bias, residual, relu, y, y_f16, &map, stream);
+    MidEpilogueT<PairMap> ep{scale, bias, residual, y, relu, y_f16, map};
     return dispatch(DenseRows{static_cast<const _Float16 *>(x16), M16, K}, native, M16, K, N, ep, stream);
 }
 
@@ -1149,6 +1162,8 @@ bool mid_conv_ok(const void *x, const tmq_conv_shape *s) {
 int launch_mid_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale,
                     const float *bias, const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream) {
     const int64_t M = (int64_t)s->B * ho * wo, K = (int64_t)s->C * s->ky * s->kx;
+    if (ring_ok(M, K, s->N, scale, bias, residual, y))
+        return launch_ring_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, map, stream);
     const ConvRows rows{static_cast<const _Float16 *>(x), M, K, s->B, s->C, s->H, s->W, ho, wo, s->ky, s->kx, s->sy,
                         s->sx, s->py, s->px, s->dy, s->dx, FastDiv((uint32_t)wo), FastDiv((uint32_t)ho),
                         FastDiv((uint32_t)s->C), FastDiv((uint32_t)s->kx)};
