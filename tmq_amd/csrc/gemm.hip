@@ -29,6 +29,11 @@ namespace tmq {
 bool mid_conv_ok(const void *x, const tmq_conv_shape *s);
 int launch_mid_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale,
                     const float *bias, const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream);
+// patch.hip: stride-1 convolutions over 128, 256 or 512 channels that are one well-filled round of its workgroups
+bool patch_conv_ok(const void *x, const tmq_conv_shape *s, int ho, int wo, const float *scale, const float *bias, const void *residual,
+                   const void *y, int y_f16);
+int launch_patch_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale, const float *bias,
+                      const void *residual, int relu, void *y, int y_f16, void *stream);
 
 namespace {
 
@@ -1572,6 +1577,8 @@ int tmq_ternary_conv2d_view(const void *x, const tmq_conv_shape *s, const void *
     const int64_t M = (int64_t)s->B * ho * wo, K = (int64_t)s->C * s->ky * s->kx;
     if (M == 0 || (view && (view->h_cnt == 0 || view->w_cnt == 0))) return TMQ_OK;
     const int y_f16 = y_dtype == TMQ_F16 ? 1 : 0;
+    if (!view && patch_conv_ok(x, s, ho, wo, scale, bias, residual, y, y_f16))
+        return launch_patch_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, stream);
     // few output tiles: split the reduction inside the workgroup (mid.hip)
     if (mid_conv_ok(x, s) && split_reduction_pays(M, K, s->N) &&
         !(wide_conv_ok(x, s, M) && wide_tile(M, K, s->N) != WideTile::kNone))
