@@ -290,8 +290,8 @@ struct RingTile {
 constexpr RingTile kRingTiles[] = {{1, 1, 4, 5}, {1, 1, 8, 4}, {1, 2, 4, 4}, {1, 2, 8, 4}, {2, 2, 4, 3}, {2, 2, 8, 2},
                                    {1, 4, 4, 4}, {2, 4, 8, 2}, {2, 4, 4, 3}, {4, 4, 4, 2}, {4, 4, 8, 2}};
 
-// Microseconds a launch is expected to take, fitted to 1200 shapes (convolutions of 64 .. 512 channels, 1 x 1 .. 5 x 5, and
-// dense rows; 17 .. 15000 rows, 16 .. 4096 columns) with eleven tiles each: the launch, the chain of a wavefront's pairs for
+// Microseconds a launch is expected to take, fitted to 1700 shapes (convolutions of 64 .. 512 channels, 1 x 1 .. 5 x 5, dense rows,
+// fp32 row pairs; 17 .. 15000 rows, 16 .. 8192 columns) with eleven tiles each: the launch, the chain of a wavefront's pairs for
 // every round of workgroups, and what shares a CU -- vector-memory instructions, products, sums. The tile it picks takes 1.01 of
 // the fastest one's time on average.
 double ring_cost(const RingTile &t, int64_t M, int64_t pairs, int64_t N, bool conv) {
@@ -299,9 +299,9 @@ double ring_cost(const RingTile &t, int64_t M, int64_t pairs, int64_t N, bool co
     int64_t resident = 160 * 1024 / ring_lds(t.wm, t.wn, t.waves, t.depth);
     if (resident > 32 / t.waves) resident = 32 / t.waves;
     const double rounds = (double)((groups + 256 * resident - 1) / (256 * resident)), chain = (double)((pairs + t.waves - 1) / t.waves);
-    const double per_cu = groups <= 512 ? (double)((groups + 255) / 256) : groups / 256.0, frags = t.wm * t.wn;
-    return 2.04 + (conv ? 0.46 : 0.0) + rounds * (0.657 + 0.0662 * frags + chain * (0.119 + 0.01145 * frags)) +
-           per_cu * (0.193 + 0.00639 * t.waves * frags + pairs * (0.00671 * (2 * t.wm + t.wn) + 0.00146 * frags + (conv ? 0.00202 * t.wm : 0.0)));
+    const double per_cu = (double)((groups + 255) / 256), frags = t.wm * t.wn;
+    return 2.35 + (conv ? 0.46 : 0.0) + rounds * (0.416 + 0.0684 * frags + chain * (0.112 + 0.00901 * frags)) +
+           per_cu * (0.168 + 0.006 * t.waves * frags + pairs * (0.00623 * (2 * t.wm + t.wn) + 0.00214 * frags + (conv ? 0.00218 * t.wm : 0.0)));
 }
 
 template <bool CONV, class Map>
