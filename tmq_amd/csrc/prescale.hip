@@ -18,12 +18,6 @@ namespace {
 constexpr int kPartials = 1024;           // partial maxima of the multi-block scan
 constexpr int64_t kSingleMax = 1 << 16;   // up to here one workgroup does everything in one launch
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
 // maximum over the workgroup, valid in every thread
 __device__ __forceinline__ float block_max(float v, float *lds /* >= 17 floats */) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
@@ -429,7 +423,8 @@ __global__ __launch_bounds__(1024) void split_groups_kernel(const float *__restr
     }
 }
 
-// Partial maxima of n values for the converting kernels; returns how many. vec: x is 16-byte aligned.
+}  // namespace
+
 int launch_absmax(const float *x, int64_t n, float *partials, int vec, void *stream) {
     const int64_t per = vec ? 4096 : 8192;                 // 16 or 32 values per thread and round
     int64_t blocks = (n + per - 1) / per;
@@ -440,8 +435,6 @@ int launch_absmax(const float *x, int64_t n, float *partials, int vec, void *str
         hipLaunchKernelGGL(absmax_partial_kernel, dim3((uint32_t)blocks), dim3(256), 0, as_stream(stream), x, n, partials, 0);
     return (int)blocks;
 }
-
-}  // namespace
 
 // The same split for rows of any length and alignment, written as rows of Kp >= K values (Kp a multiple of 8) with
 // zeros behind the K-th: one workgroup per group of eight rows, element-wise reads, one 16-byte piece of a hi row and

@@ -12,24 +12,25 @@
 //
 // Work split: a workgroup (4 wavefronts) owns the 15 x 17 patch of convolution outputs that 7 x 8 pooled
 // positions need (rows 14 th - 1 .. 14 th + 13, columns 16 tw - 1 .. 16 tw + 15 of image b); neighbouring
-// patches share their border row and column, 255 positions computed for 224 new ones. The patch is a
-// 256-row GEMM tile by up to 64 output channels; a wavefront takes 128 rows x 32 channels. Rows 16 f .. 16 f + 15
+// patches share their border row and column, 255 positions computed for 224 new ones (a few images have patches of
+// 7 x 17 for 3 x 8 pooled positions instead, for the sake of more workgroups). The patch is a 256-row (128-row) GEMM
+// tile by up to 64 output channels; a wavefront takes a quarter of the rows, all channels. Rows 16 f .. 16 f + 15
 // (one MFMA row fragment) are columns 0 .. 15 of patch row f < 15 -- neighbouring pixels of the window, so the
 // 16 lanes of an operand read touch 16 consecutive pieces, every LDS bank once -- and rows 240 .. 254 are column
 // 16 of the 15 patch rows (row 255 repeats row 254 and is never pooled). The results go, as fp16, into a
-// [256][64] tile in LDS (over the input window, which is no longer needed), and the workgroup pools that.
+// [rows][64] tile in LDS (over the input window, which is no longer needed), and the workgroup pools that.
 #include "common.h"
 #include "mfma.h"
+#include "range.h"
 
 namespace tmq {
 namespace {
 
-constexpr int kPoolH = 7, kPoolW = 8;                                  // pooled positions per patch
-constexpr int kPatchH = 2 * kPoolH + 1, kPatchW = 2 * kPoolW + 1;       // convolution outputs per patch
-constexpr int kTilePitch = 144;                                         // bytes per row of the fp16 [256][64] tile (16 of padding)
-constexpr int kTileBytes = 256 * kTilePitch;
+constexpr int kPoolW = 8, kPatchW = 2 * kPoolW + 1;                     // pooled columns and convolution columns per patch
+constexpr int kTilePitch = 144;                                         // bytes per row of the fp16 [rows][64] tile (16 of padding)
 constexpr int kThreads = 256;
 constexpr int kMaxLds = 64 * 1024;
+constexpr int kBatch = 3;                                               // fp32 window pieces a thread asks for at once
 
 struct StemShape {
     const _Float16 *x;
@@ -46,17 +47,26 @@ struct StemShape {
     FastDiv by_tw, by_th, by_kx, by_row;   // patches per image row / column, kernel width, 16-byte pieces per window row
     int planes;                  // 0: x is NHWC; 1 .. 4: x is the network's own NCHW fp16 input with that many channels, read as
                                  // 8-channel "super-pixels" of two neighbouring pixels x 4 channels (cshift == 3, W = width / 2)
+    const float *xf;             // planes in fp32 (kernels with F32; x is not read), prescaled on the way into LDS
+    const float *partials;       // their partial maxima, from the launch before
+    int partial_count;
 };
 
-template <int WM, int WN>
+// F32: the planes are fp32. fp16(s x) with the tensor's power-of-two prescale s is made while the window is gathered, from
+// the partial maxima of the scan in front (at most 1024, which every wavefront reduces itself while its pixels are on their
+// way), and 1 / s goes into the channels' scales: the launch that wrote an fp16 copy of the image for this one to read is
+// gone (64 channels, 224 x 224, with the scan: one image 10.9 -> 7.9 us, 8 15.1 -> 11.4, 64 52.0 -> 47.5).
+template <int kPoolH, bool F32>
 __global__ __launch_bounds__(kThreads, 3) void stem_pool_kernel(StemShape p, const uint32_t *__restrict__ native, int N,
                                                                 const float *__restrict__ scale, const float *__restrict__ bias,
                                                                 _Float16 *__restrict__ y, int tiles) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    constexpr int WGN = 4 / WN, D = WM / 2;          // wavefronts side by side; how many row fragments ahead the operand reads run
-    static_assert(WM * WN == 16 && (WN == 2 || WN == 4), "a wavefront takes 16 WM rows x 16 WN channels of the 256 x 64 tile");
-    const int wm = wv / WGN, wn = wv % WGN;
+    constexpr int kPatchH = 2 * kPoolH + 1;          // convolution rows per patch, one row fragment each and one for column 16
+    constexpr int WM = (kPatchH + 1) / 4, WN = 4;    // row and column fragments of a wavefront (16 WM rows x 64 channels)
+    constexpr int D = WM > 1 ? WM / 2 : 1;           // how many row fragments ahead the operand reads run
+    static_assert((kPatchH + 1) % 4 == 0, "the four wavefronts share the row fragments evenly");
+    const int wm = wv;
     const int r16 = lane & 15, g = lane >> 4;
 
     // patch of this workgroup; the workgroups of one XCD (one L2) take neighbouring patches, which share input rows
@@ -66,10 +76,71 @@ __global__ __launch_bounds__(kThreads, 3) void stem_pool_kernel(StemShape p, con
     const int oh0 = 2 * kPoolH * th - 1, ow0 = 2 * kPoolW * tw - 1;
     const int ih_base = oh0 * p.sy - p.py, iw_base = ow0 * p.sx - p.px;
 
+    // ---- weights (the whole reduction is one native block) and the lane's channel's constants ----
+    const int Nb = (N + 15) >> 4;
+    u32x4 wblk[WN];
+#pragma unroll
+    for (int j = 0; j < WN; j++) {
+        const int nb = j < Nb ? j : Nb - 1;         // columns past N: finite bits, never pooled
+        wblk[j] = *reinterpret_cast<const u32x4 *>(native + nb * 256 + lane * 4);
+    }
+    float c_scale = 1.f, c_bias = 0.f;
+    if (tid < N) {
+        if (scale) c_scale = scale[tid];
+        if (bias) c_bias = bias[tid];
+    }
+
     // ---- the input window -> LDS, 16 bytes per lane; pixels outside the image (padding) arrive as zeros ----
     const BufferResource rsrc = make_buffer_resource(p.x, p.x_bytes);
     const int sub_mask = (1 << (p.cshift - 3)) - 1;
-    if (p.planes) {
+    float inv = 1.f;                                // 1 / prescale
+    if constexpr (F32) {
+        const int64_t plane = (int64_t)p.H * p.W;                       // pixel pairs per plane
+        const floatx2 *img = reinterpret_cast<const floatx2 *>(p.xf) + (int64_t)b * p.planes * plane;
+        float s = 1.f;
+        for (int c0 = 0; c0 < p.chunks; c0 += kBatch * kThreads) {      // (one pass for a 7 x 7 / 2 opening: 700 pieces)
+            floatx2 v[kBatch][4];
+#pragma unroll
+            for (int r = 0; r < kBatch; r++) {
+                const int c = c0 + r * kThreads + tid;
+                int rc;
+                const int prow = (int)p.by_row.divmod((uint32_t)c, rc);
+                const int ih = ih_base + prow, iw = iw_base + rc;
+                const bool in = (c < p.chunks) & ((unsigned)ih < (unsigned)p.H) & ((unsigned)iw < (unsigned)p.W);
+                const floatx2 *src = img + (int64_t)ih * p.W + iw;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    v[r][q] = floatx2{0.f, 0.f};
+                    if (in && q < p.planes) v[r][q] = src[q * plane];
+                }
+            }
+            if (c0 == 0) {
+                float m = 0.f;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    if (k * 256 >= p.partial_count) break;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int at = k * 256 + i * 64 + lane;
+                        m = fmaxf(m, at < p.partial_count ? p.partials[at] : 0.f);
+                    }
+                }
+                make_prescale(wave_max(m), s, inv);
+            }
+#pragma unroll
+            for (int r = 0; r < kBatch; r++) {
+                const int c = c0 + r * kThreads + tid;
+                if (c >= p.chunks) break;
+                half8 h;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    h[q] = (_Float16)(v[r][q][0] * s);
+                    h[4 + q] = (_Float16)(v[r][q][1] * s);
+                }
+                *reinterpret_cast<half8 *>(lds + c * 16) = h;
+            }
+        }
+    } else if (p.planes) {
         // Planar input: a piece of the window is two neighbouring pixels of up to four planes. One 4-byte load per plane
         // (the pixel pair), interleaved in registers to (c0 c1 c2 c3 | c0 c1 c2 c3) and written to the place the
         // 16-byte copy of the NHWC path would have filled: no repacked copy of the input ever exists in memory.
@@ -107,21 +178,13 @@ __global__ __launch_bounds__(kThreads, 3) void stem_pool_kernel(StemShape p, con
     if (p.zero_off)
         for (int c = tid; c < p.chunks; c += kThreads) *reinterpret_cast<u32x4 *>(lds + p.zero_off + c * 16) = u32x4{0u, 0u, 0u, 0u};
 
-    // ---- while that is on its way: weights (the whole reduction is one native block), constants, addresses ----
-    const int Nb = (N + 15) >> 4;
-    u32x4 wblk[WN];
-#pragma unroll
-    for (int j = 0; j < WN; j++) {
-        int nb = wn * WN + j;
-        nb = nb < Nb ? nb : Nb - 1;                 // columns past N: finite bits, never pooled
-        wblk[j] = *reinterpret_cast<const u32x4 *>(native + nb * 256 + lane * 4);
-    }
+    // ---- while that is on its way: addresses and constants ----
     // LDS byte offset of the window origin of the lane's row in each of its row fragments
     int rowbase[WM];
     const int pixel_shift = p.cshift + 1, lane_col = (r16 * p.sx) << pixel_shift;
 #pragma unroll
     for (int i = 0; i < WM; i++) rowbase[i] = ((((wm * WM + i) * p.sy) * p.PC) << pixel_shift) + lane_col;
-    if (wm == 16 / WM - 1)                          // the last fragment: column 16 of the 15 patch rows
+    if (wm == 3)                                    // the last fragment: column 16 of the patch rows
         rowbase[WM - 1] = (((r16 < kPatchH ? r16 : kPatchH - 1) * p.sy) * p.PC + (kPatchW - 1) * p.sx) << pixel_shift;
     // Displacement of piece u of the reduction (indices 8 u .. 8 u + 7 = one tap, 8 channels): a table, since a lane needs
     // piece 4 s + g in MFMA step s. Pieces past K point into the zeroed region.
@@ -135,8 +198,9 @@ __global__ __launch_bounds__(kThreads, 3) void stem_pool_kernel(StemShape p, con
     // trip to memory ends while the window is on its way, where a load in the epilogue would make every wavefront wait.
     float *const constants = reinterpret_cast<float *>(lds + p.const_off);
     if (tid < 64) {
-        constants[tid] = (tid < N && scale ? scale[tid] : 1.f) * (1.0f / kWeightUnit);
-        constants[64 + tid] = tid < N && bias ? bias[tid] : 0.f;
+        if constexpr (F32) c_scale *= inv;
+        constants[tid] = c_scale * (1.0f / kWeightUnit);
+        constants[64 + tid] = c_bias;
     }
     const int S = (p.kchunks + 3) >> 2;
 
@@ -181,13 +245,13 @@ __global__ __launch_bounds__(kThreads, 3) void stem_pool_kernel(StemShape p, con
     floatx4 sc[WN], bi[WN];
 #pragma unroll
     for (int j = 0; j < WN; j++) {
-        sc[j] = *reinterpret_cast<const floatx4 *>(constants + (wn * WN + j) * 16 + g * 4);
-        bi[j] = *reinterpret_cast<const floatx4 *>(constants + 64 + (wn * WN + j) * 16 + g * 4);
+        sc[j] = *reinterpret_cast<const floatx4 *>(constants + j * 16 + g * 4);
+        bi[j] = *reinterpret_cast<const floatx4 *>(constants + 64 + j * 16 + g * 4);
     }
     __syncthreads();                                // everybody is done with the window: the tile goes over it
 
     // ---- results -> fp16 tile: the value the convolution alone would store before its ReLU ----
-    unsigned char *dst = lds + (wm * WM * 16 + r16) * kTilePitch + (wn * WN * 16 + g * 4) * 2;
+    unsigned char *dst = lds + (wm * WM * 16 + r16) * kTilePitch + g * 8;
 #pragma unroll
     for (int i = 0; i < WM; i++)
 #pragma unroll
@@ -208,10 +272,10 @@ __global__ __launch_bounds__(kThreads, 3) void stem_pool_kernel(StemShape p, con
         const int c8 = item & 7, q = item >> 3, pw_ = ((q & 1) << 2) | ((q >> 1) & 3), ph_ = q >> 3;
         const int ph = th * kPoolH + ph_, pw = tw * kPoolW + pw_;
         if (ph >= p.Po || pw >= p.Pwo || c8 * 8 >= N) continue;
-        // tile row of patch position (r, c): 16 r + c, or 240 + r for c = 16 (the third column of the last pooled column)
+        // tile row of patch position (r, c): 16 r + c, or 16 kPatchH + r for c = 16 (the third column of the last pooled column)
         const unsigned char *src = lds + ((2 * ph_) * 16 + 2 * pw_) * kTilePitch + c8 * 16;
         const bool edge = pw_ == kPoolW - 1;
-        const unsigned char *third = edge ? lds + (240 + 2 * ph_) * kTilePitch + c8 * 16 : src + 2 * kTilePitch;
+        const unsigned char *third = edge ? lds + (16 * kPatchH + 2 * ph_) * kTilePitch + c8 * 16 : src + 2 * kTilePitch;
         const int third_step = edge ? kTilePitch : 16 * kTilePitch;
         auto tap = [&](int e) {
             return *reinterpret_cast<const half8 *>(e % 3 == 2 ? third + (e / 3) * third_step : src + ((e / 3) * 16 + e % 3) * kTilePitch);
@@ -235,18 +299,10 @@ __global__ __launch_bounds__(kThreads, 3) void stem_pool_kernel(StemShape p, con
     }
 }
 
-}  // namespace
-
-extern "C" {
-
-int tmq_ternary_conv2d_relu_maxpool(const void *x, const tmq_conv_shape *s, const void *native, const float *scale,
-                                    const float *bias, void *y, void *stream) {
-    return tmq_ternary_conv2d_relu_maxpool_planar(x, 0, s, native, scale, bias, y, stream);
-}
-
-int tmq_ternary_conv2d_relu_maxpool_planar(const void *x, int32_t planes, const tmq_conv_shape *s, const void *native,
-                                           const float *scale, const float *bias, void *y, void *stream) {
-    if (!s || !x || !native || !y || !aligned16(native) || planes < 0 || planes > 4) return TMQ_ERR_INVALID_ARG;
+// xf: fp32 planes in x's place, whose partial maxima go through `workspace`
+int launch_opening(const void *x, const float *xf, int32_t planes, const tmq_conv_shape *s, const void *native, const float *scale,
+                   const float *bias, void *y, void *workspace, void *stream) {
+    if (!s || (!x && !xf) || !native || !y || !aligned16(native) || planes < 0 || planes > 4) return TMQ_ERR_INVALID_ARG;
     if (planes && (s->C != 8 || (reinterpret_cast<uintptr_t>(x) & 3u))) return TMQ_ERR_UNSUPPORTED;
     int32_t ho, wo;
     const int rc = tmq_conv2d_out_hw(s, &ho, &wo);
@@ -266,31 +322,70 @@ int tmq_ternary_conv2d_relu_maxpool_planar(const void *x, int32_t planes, const 
     p.sy = s->sy; p.sx = s->sx; p.py = s->py; p.px = s->px; p.dy = s->dy; p.dx = s->dx;
     p.Po = (ho - 1) / 2 + 1;
     p.Pwo = (wo - 1) / 2 + 1;
+    // The patch's height: 3 pooled rows while all such patches run at once (three on a CU), 7 beyond, where a patch of 7
+    // reads fewer window rows twice. 64 channels, 224 x 224, fp16 planes: one image 6.4 us at 7 rows, 4.8 at 3; two 6.5
+    // and 5.5; five (665 patches of 3) 7.4 and 6.7; six (798) 7.6 and 7.5; eight 7.8 and 8.5; 64 31.7 and 40.5. Patches
+    // of 1 row 4.7 for one image, 6.0 for two; of 5 rows in between everywhere.
+    const int tw = (p.Pwo + kPoolW - 1) / kPoolW;
+    const int64_t columns = (int64_t)s->B * tw;
+    const int pool_h = columns * ((p.Po + 2) / 3) <= 3 * 256 ? 3 : 7;
+    const int th = (p.Po + pool_h - 1) / pool_h;
     // the input window of a patch: its first and last output rows / columns and the kernel's extent
-    const int64_t PR = (int64_t)(kPatchH - 1) * s->sy + (int64_t)(s->ky - 1) * s->dy + 1;
     const int64_t PC = (int64_t)(kPatchW - 1) * s->sx + (int64_t)(s->kx - 1) * s->dx + 1;
-    const int64_t chunks = PR * PC * (s->C / 8), padded = (chunks + kThreads - 1) / kThreads * kThreads;
     const bool ragged = (K / 8) % 4 != 0;                 // the last MFMA step reaches past K
-    const int64_t lds_window = padded * 16 + (ragged ? chunks * 16 : 0) + 32 * 4;   // window, zeros, displacement table
-    if (lds_window + 128 * 4 > kMaxLds) return TMQ_ERR_UNSUPPORTED;
+    auto window = [&](int h) { return ((int64_t)2 * h * s->sy + (int64_t)(s->ky - 1) * s->dy + 1) * PC * (s->C / 8); };
+    auto lds_bytes = [&](int h) {                         // window, zeros, displacement table
+        return (window(h) + kThreads - 1) / kThreads * kThreads * 16 + (ragged ? window(h) * 16 : 0) + 32 * 4;
+    };
+    if (lds_bytes(7) + 128 * 4 > kMaxLds) return TMQ_ERR_UNSUPPORTED;     // whatever the height
+    const int64_t chunks = window(pool_h), lds_window = lds_bytes(pool_h), tile_bytes = (int64_t)(2 * pool_h + 2) * 16 * kTilePitch;
     p.PC = (int)PC;
     p.chunks = (int)chunks;
-    p.zero_off = ragged ? (int)(padded * 16) : 0;
+    p.zero_off = ragged ? (int)((chunks + kThreads - 1) / kThreads * kThreads * 16) : 0;
     p.tab_off = (int)(lds_window - 32 * 4);
     p.kchunks = (int)(K / 8);
-    const int th = (p.Po + kPoolH - 1) / kPoolH, tw = (p.Pwo + kPoolW - 1) / kPoolW;
     p.by_tw = FastDiv((uint32_t)tw);
     p.by_th = FastDiv((uint32_t)th);
     p.by_kx = FastDiv((uint32_t)s->kx);
     p.by_row = FastDiv((uint32_t)(PC * (s->C / 8)));
-    const int64_t tiles = (int64_t)s->B * th * tw;
+    const int64_t tiles = columns * th;
     if (tiles > (int64_t)0x7FFFFFFF) return TMQ_ERR_TOO_LARGE;
     if (tiles == 0) return TMQ_OK;
-    p.const_off = (int)(lds_window > kTileBytes ? lds_window : kTileBytes);
+    p.const_off = (int)(lds_window > tile_bytes ? lds_window : tile_bytes);
     const size_t lds = (size_t)p.const_off + 128 * 4;
-    hipLaunchKernelGGL((stem_pool_kernel<4, 4>), dim3((uint32_t)tiles), dim3(kThreads), lds, as_stream(stream), p,
-                       static_cast<const uint32_t *>(native), (int)s->N, scale, bias, static_cast<_Float16 *>(y), (int)tiles);
+    if (xf) {
+        p.xf = xf;
+        p.partials = static_cast<const float *>(workspace);
+        p.partial_count = launch_absmax(xf, (int64_t)s->B * planes * s->H * s->W * 2, static_cast<float *>(workspace), aligned16(xf), stream);
+        if (int rc2 = check_launch()) return rc2;
+    }
+    auto kernel = pool_h == 7 ? (xf ? stem_pool_kernel<7, true> : stem_pool_kernel<7, false>)
+                              : (xf ? stem_pool_kernel<3, true> : stem_pool_kernel<3, false>);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles), dim3(kThreads), lds,
+                       as_stream(stream), p, static_cast<const uint32_t *>(native), (int)s->N, scale, bias,
+                       static_cast<_Float16 *>(y), (int)tiles);
     return check_launch();
+}
+
+}  // namespace
+
+extern "C" {
+
+int tmq_ternary_conv2d_relu_maxpool(const void *x, const tmq_conv_shape *s, const void *native, const float *scale,
+                                    const float *bias, void *y, void *stream) {
+    return tmq_ternary_conv2d_relu_maxpool_planar(x, 0, s, native, scale, bias, y, stream);
+}
+
+int tmq_ternary_conv2d_relu_maxpool_planar(const void *x, int32_t planes, const tmq_conv_shape *s, const void *native,
+                                           const float *scale, const float *bias, void *y, void *stream) {
+    return launch_opening(x, nullptr, planes, s, native, scale, bias, y, nullptr, stream);
+}
+
+int tmq_ternary_conv2d_relu_maxpool_planar_f32(const float *x, int32_t planes, const tmq_conv_shape *s, const void *native,
+                                               const float *scale, const float *bias, void *y, void *workspace, void *stream) {
+    if (!x || !workspace || planes < 1) return TMQ_ERR_INVALID_ARG;
+    if (reinterpret_cast<uintptr_t>(x) & 7u) return TMQ_ERR_UNSUPPORTED;
+    return launch_opening(nullptr, x, planes, s, native, scale, bias, y, workspace, stream);
 }
 
 }  // extern "C"

@@ -912,11 +912,13 @@ def ternary_conv2d_relu_maxpool(x: torch.Tensor, nw: NativeWeights, stride=1, pa
 
 
 def ternary_conv2d_relu_maxpool_planar(x: torch.Tensor, nw: NativeWeights, stride=1, padding=0, dilation=1, scale=None,
-                                       bias=None) -> torch.Tensor:
+                                       bias=None, prescale=False) -> torch.Tensor:
     """ternary_conv2d_relu_maxpool on the network's own input: x is NCHW fp16 [B, C <= 4, H, W] (W even), nw the weights of
     the convolution over 8-channel "super-pixels" (two neighbouring pixels x 4 channels) that stride, padding and dilation
     describe -- what nchw_to_nhwc4(x).view(B, H, W / 2, 8) would feed the other call, without that copy of the input.
-    Same bits as the two-step form, which it falls back to where the one-kernel opening does not apply."""
+    Same bits as the two-step form, which it falls back to where the one-kernel opening does not apply.
+    prescale: an fp32 x is brought into fp16's range first, exactly as f32_to_f16_prescaled does it and with its result,
+    but inside the opening."""
     pair = lambda v: tuple(v) if isinstance(v, (tuple, list)) else (v, v)
     (sy, sx), (py, px), (dy, dx) = pair(stride), pair(padding), pair(dilation)
     (py, py_end), (px, px_end) = pair(py), pair(px)
@@ -928,7 +930,9 @@ def ternary_conv2d_relu_maxpool_planar(x: torch.Tensor, nw: NativeWeights, strid
         B, C, H, W = x.shape
         xs = nchw_to_nhwc4(x).view(B, H, W // 2, 8).permute(0, 3, 1, 2)      # [B, 8, H, W / 2], channels_last memory
         return ternary_conv2d_relu_maxpool(xs, nw, stride, padding, dilation, scale, bias)
-    if x.dtype != torch.float16:
+    if x.dtype == torch.float32 and prescale and not (_fp32_prescale and x.numel() and x.data_ptr() % 8 == 0 and x.is_contiguous()):
+        x, scale = f32_to_f16_prescaled(x, scale, nw.N)
+    if x.dtype != torch.float16 and not (prescale and x.dtype == torch.float32):
         return two_step()
     x = x.contiguous()
     B, C, H, W = x.shape
@@ -944,9 +948,16 @@ def ternary_conv2d_relu_maxpool_planar(x: torch.Tensor, nw: NativeWeights, strid
     if B == 0:
         return y
     with _capi.on_device(x.device):
-        status = lib.tmq_ternary_conv2d_relu_maxpool_planar(ptr(x), C, ctypes.byref(shp), ptr(nw.buf), ep.scale, ep.bias, ptr(y),
-                                                            stream_of(x))
+        if x.dtype == torch.float32:
+            ws = torch.empty(lib.tmq_f32_to_f16_prescaled_workspace_bytes(x.numel()), dtype=torch.uint8, device=x.device)
+            status = lib.tmq_ternary_conv2d_relu_maxpool_planar_f32(ptr(x), C, ctypes.byref(shp), ptr(nw.buf), ep.scale, ep.bias,
+                                                                    ptr(y), ptr(ws), stream_of(x))
+        else:
+            status = lib.tmq_ternary_conv2d_relu_maxpool_planar(ptr(x), C, ctypes.byref(shp), ptr(nw.buf), ep.scale, ep.bias,
+                                                                ptr(y), stream_of(x))
     if status == _capi.ERR_UNSUPPORTED:
+        if x.dtype == torch.float32:
+            x, scale = f32_to_f16_prescaled(x, scale, nw.N)
         return two_step()
     check(status, "ternary_conv2d_relu_maxpool_planar")
     return y

@@ -832,11 +832,12 @@ class Conv2d(nn.Module, TMQLayer):
             # pixels of the 4-channel NHWC image are read as one pixel of 8 channels, see _superpixel_plan
             nw, kxs, pl, pr = sp
             B, C, H, W = x.shape
+            (sy, _), (py, _) = _pair(self.stride), _pair(self.padding)
+            if pool:      # the one-kernel opening gathers the pixel pairs from the NCHW planes itself, and prescales fp32 ones
+                return ops.ternary_conv2d_relu_maxpool_planar(x, nw, (sy, 1), ((py, py), (pl, pr)), 1, scale=scale, bias=bias,
+                                                              prescale=True)
             if x.dtype == torch.float32:
                 x, scale = ops.f32_to_f16_prescaled(x, scale, int(self.original_shape[0]))
-            (sy, _), (py, _) = _pair(self.stride), _pair(self.padding)
-            if pool:      # the one-kernel opening gathers the pixel pairs from the NCHW planes itself
-                return ops.ternary_conv2d_relu_maxpool_planar(x, nw, (sy, 1), ((py, py), (pl, pr)), 1, scale=scale, bias=bias)
             xs = ops.nchw_to_nhwc4(x).view(B, H, W // 2, 8).permute(0, 3, 1, 2)
             return ops.ternary_conv2d(xs, nw, (sy, 1), ((py, py), (pl, pr)), 1, scale=scale, bias=bias,
                                       residual=residual, relu=relu, out_dtype=_compact_out)
