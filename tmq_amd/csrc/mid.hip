@@ -1,5 +1,7 @@
 // Ternary GEMM / implicit-GEMM convolution for outputs too small to fill the chip with big tiles
-// (a few hundred 64 x 64 tiles): the reduction is split over the wavefronts of a workgroup.
+// (a few hundred 64 x 64 tiles): the reduction is split over the wavefronts of a workgroup. Most such problems go on to
+// ring.hip (ring_ok says which and what both measure); what follows serves the longest reductions and results that are no
+// whole aligned quads.
 //
 // A workgroup of WAVES wavefronts owns a (16 WM) x (16 WN) output tile; wavefront kg multiplies the
 // whole tile over the "pairs" (64 reduction indices each) kg, kg + WAVES, ... and the partial tiles
