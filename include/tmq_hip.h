@@ -440,6 +440,11 @@ typedef struct tmq_output_view {
 int tmq_ternary_conv2d_view(const void *x, const tmq_conv_shape *shape, const void *native,
                             const tmq_epilogue *epilogue, void *y, const tmq_output_view *view, void *stream);
 
+/* Which kernel tmq_ternary_conv2d launches for a convolution whose operands are all 16-byte aligned: for profiles and tests
+ * (host only, nothing is launched). A TMQ_KERNEL_ value, or a negative status. */
+enum { TMQ_KERNEL_TILES = 0, TMQ_KERNEL_SPLIT = 1, TMQ_KERNEL_PATCH = 2 };
+int tmq_ternary_conv2d_kernel(const tmq_conv_shape *shape, int y_dtype);
+
 /* Several such convolutions of ONE input (same B, C, H, W and N; windows, padding and dilation of their own) written
  * into one destination: phase q goes to the view that starts `first` pixels into y (and into epilogue->residual).
  * The phases of a transposed convolution, tmq/tmq.py:1007-1042. Up to four phases take one launch, for any number

@@ -1,0 +1,30 @@
+"""Which kernel a convolution is sent to (tmq_ternary_conv2d_kernel, host only)."""
+import ctypes
+
+import pytest
+
+TILES, SPLIT, PATCH = 0, 1, 2
+
+
+def kernel_of(B, C, H, W, N, k, pad, d=1, s=1, f16=True):
+    """k: (ky, kx); pad: ((top, bottom), (left, right)) or one number."""
+    from tmq_amd import _capi
+    (pt, pb), (pl, pr) = pad if isinstance(pad, tuple) else ((pad, pad), (pad, pad))
+    shape = _capi.ConvShape(B, C, H, W, N, k[0], k[1], s, s, pt, pl, d, d, pb, pr)
+    return _capi.load().tmq_ternary_conv2d_kernel(ctypes.byref(shape), _capi.F16 if f16 else _capi.F32)
+
+
+# the largest distance of a tap in the padded image, 2 d (14 + d) + 2 d, passes 2^31 from d = 32761 on
+@pytest.mark.parametrize("d", [1000, 30000, 32759, 32760, 32768, 33000, 40000, 46341, 65536])
+def test_far_taps_do_not_fit_a_patch(d):
+    assert kernel_of(64, 256, 14, 14, 256, (3, 3), 1) == PATCH
+    assert kernel_of(64, 256, 14, 14, 256, (3, 3), d, d) != PATCH
+    assert kernel_of(64, 256, 14, 14, 256, (1, 9), ((0, 0), (4 * d, 4 * d)), d) != PATCH
+    assert kernel_of(64, 256, 14, 14, 256, (9, 1), ((4 * d, 4 * d), (0, 0)), d) != PATCH
+
+
+def test_refuses_what_the_convolution_refuses():
+    from tmq_amd import _capi
+    assert kernel_of(1, 64, 3, 3, 64, (5, 5), 0) == -1 and kernel_of(1, 64, 0, 3, 64, (1, 1), 0) == -1
+    assert _capi.load().tmq_ternary_conv2d_kernel(None, _capi.F32) == -1
+    assert kernel_of(0, 64, 8, 8, 64, (3, 3), 1) >= 0          # an empty batch is nothing to launch

@@ -112,6 +112,7 @@ SIGNATURES = {
     "tmq_avgpool_linear": (_int, [_vp, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _vp]),
     "tmq_ternary_conv2d": (_int, [_vp, ctypes.POINTER(ConvShape), _vp, _vp, _vp, _vp]),
     "tmq_ternary_conv2d_view": (_int, [_vp, ctypes.POINTER(ConvShape), _vp, _vp, _vp, ctypes.POINTER(OutputView), _vp]),
+    "tmq_ternary_conv2d_kernel": (_int, [ctypes.POINTER(ConvShape), _int]),
     "tmq_ternary_conv2d_phases": (_int, [_vp, ctypes.POINTER(ConvPhase), _int, _vp, _vp, _vp]),
     "tmq_ternary_conv2d_relu_maxpool": (_int, [_vp, ctypes.POINTER(ConvShape), _vp, _vp, _vp, _vp, _vp]),
     "tmq_ternary_conv2d_relu_maxpool_planar": (_int, [_vp, ctypes.c_int32, ctypes.POINTER(ConvShape), _vp, _vp, _vp, _vp, _vp]),

@@ -1426,6 +1426,11 @@ bool wide_conv_ok(const void *x, const tmq_conv_shape *s, int64_t M) {
            M < (int64_t)0x7FFFFFFF;
 }
 
+// Few output tiles: the reduction is split inside the workgroup (mid.hip).
+bool conv_splits_reduction(const void *x, const tmq_conv_shape *s, int64_t M, int64_t K) {
+    return mid_conv_ok(x, s) && split_reduction_pays(M, K, s->N) && !(wide_conv_ok(x, s, M) && wide_tile(M, K, s->N) != WideTile::kNone);
+}
+
 // The tile kernels behind tmq_ternary_conv2d for an epilogue with consecutive rows (Epilogue) or rows scattered into a
 // strided destination (ViewEpilogue).
 template <class Ep>
@@ -1579,12 +1584,20 @@ int tmq_ternary_conv2d_view(const void *x, const tmq_conv_shape *s, const void *
     const int y_f16 = y_dtype == TMQ_F16 ? 1 : 0;
     if (!view && patch_conv_ok(x, s, ho, wo, scale, bias, residual, y, y_f16))
         return launch_patch_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, stream);
-    // few output tiles: split the reduction inside the workgroup (mid.hip)
-    if (mid_conv_ok(x, s) && split_reduction_pays(M, K, s->N) &&
-        !(wide_conv_ok(x, s, M) && wide_tile(M, K, s->N) != WideTile::kNone))
+    if (conv_splits_reduction(x, s, M, K))
         return launch_mid_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, view ? &map : nullptr, stream);
     if (view) return conv_tiles(x, s, ho, wo, native, ViewEpilogue{scale, bias, residual, y, relu, y_f16, map}, stream);
     return conv_tiles(x, s, ho, wo, native, Epilogue{scale, bias, residual, y, relu, y_f16, {}}, stream);
+}
+
+int tmq_ternary_conv2d_kernel(const tmq_conv_shape *s, int y_dtype) {
+    if (!s || (y_dtype != TMQ_F16 && y_dtype != TMQ_F32)) return TMQ_ERR_INVALID_ARG;
+    int32_t ho, wo;
+    RowMap map;
+    if (const int rc = conv_plan(s, nullptr, ho, wo, map)) return rc;
+    const int64_t M = (int64_t)s->B * ho * wo, K = (int64_t)s->C * s->ky * s->kx;
+    if (M && patch_conv_ok(nullptr, s, ho, wo, nullptr, nullptr, nullptr, nullptr, y_dtype == TMQ_F16)) return TMQ_KERNEL_PATCH;
+    return conv_splits_reduction(nullptr, s, M, K) ? TMQ_KERNEL_SPLIT : TMQ_KERNEL_TILES;
 }
 
 int tmq_ternary_conv2d_phases(const void *x, const tmq_conv_phase *phases, int count, const tmq_epilogue *epilogue, void *y,

@@ -400,7 +400,8 @@ int launch(PatchConv cv, const Epilogue &ep, int64_t bytes, int64_t groups, void
 }
 
 struct PatchPlan {
-    int slabs, columns, Hp, Wp, reach;     // 64-channel slabs; column groups of 64 in a workgroup
+    int slabs, columns;                    // 64-channel slabs; column groups of 64 in a workgroup
+    int64_t Hp, Wp, reach;                 // the padded image and the largest distance of a tap: any padding and dilation comes here
     int64_t rows, groups, pixels, bytes;   // output pixels and LDS of a workgroup, workgroups
 };
 
@@ -410,8 +411,8 @@ struct PatchPlan {
 // below that, or over several rounds, up to 1.6; windows of fewer than nine taps don't pay for their ends.
 bool patch_plan(const tmq_conv_shape *s, int ho, int wo, PatchPlan &p) {
     if (s->sy != 1 || s->sx != 1 || !(s->C == 128 || s->C == 256 || s->C == 512) || s->ky * s->kx < 9) return false;
-    const int top = s->py, left = s->px, bottom = ho - 1 - top + (s->ky - 1) * s->dy - (s->H - 1),
-              right = wo - 1 - left + (s->kx - 1) * s->dx - (s->W - 1);
+    const int64_t down = (int64_t)(s->ky - 1) * s->dy, across = (int64_t)(s->kx - 1) * s->dx;
+    const int64_t top = s->py, left = s->px, bottom = ho - 1 - top + down - (s->H - 1), right = wo - 1 - left + across - (s->W - 1);
     // one row / column of padding serves the end of a row and the start of the next
     p.Hp = s->H + (top > bottom ? top : bottom);
     p.Wp = s->W + (left > right ? left : right);
@@ -427,7 +428,8 @@ bool patch_plan(const tmq_conv_shape *s, int ho, int wo, PatchPlan &p) {
     // the pixels spread evenly over the round
     p.rows = (M + slots / tn - 1) / (slots / tn);
     p.groups = (M + p.rows - 1) / p.rows * tn;
-    p.reach = (s->ky - 1) * s->dy * p.Wp + (s->kx - 1) * s->dx;
+    p.reach = down * p.Wp + across;
+    if (s->B * p.Hp * p.Wp + p.reach >= (int64_t)1 << 31) return false;     // places in the padded images are 32 bits
     p.pixels = patch_pixels(p.rows, ho, wo, p.Hp, p.Wp, p.reach);
     p.bytes = p.slabs * p.pixels * kPixelBytes;
     const int64_t sums = (int64_t)waves * 4096 * 4;
@@ -456,8 +458,8 @@ int launch_patch_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, co
     cv.Nb = (int32_t)native_blocks_n(s->N);
     cv.M = (int32_t)((int64_t)s->B * ho * wo);
     cv.N = s->N; cv.C = s->C; cv.H = s->H; cv.W = s->W; cv.B = s->B;
-    cv.py = s->py; cv.px = s->px; cv.Hp = p.Hp; cv.Wp = p.Wp;
-    cv.ky = s->ky; cv.kx = s->kx; cv.dy = s->dy; cv.dx = s->dx; cv.reach = p.reach;
+    cv.py = s->py; cv.px = s->px; cv.Hp = (int32_t)p.Hp; cv.Wp = (int32_t)p.Wp;
+    cv.ky = s->ky; cv.kx = s->kx; cv.dy = s->dy; cv.dx = s->dx; cv.reach = (int32_t)p.reach;
     cv.pixels = (int32_t)p.pixels;
     cv.rows = (int32_t)p.rows;
     cv.x_bytes = (uint32_t)((int64_t)s->B * s->H * s->W * s->C * 2);
