@@ -23,6 +23,13 @@ def test_far_taps_do_not_fit_a_patch(d):
     assert kernel_of(64, 256, 14, 14, 256, (9, 1), ((4 * d, 4 * d), (0, 0)), d) != PATCH
 
 
+# half of such workgroups' reduction, and at most 64 outputs are two rounds of the chip where the plan counts one
+@pytest.mark.parametrize("B,H,W,N", [(64, 28, 28, 128), (32, 56, 56, 64), (162, 27, 25, 64), (32, 83, 10, 244), (28, 109, 3, 640)])
+@pytest.mark.parametrize("f16", [False, True])
+def test_128_channels_stay_out_of_patches(B, H, W, N, f16):
+    assert kernel_of(B, 128, H, W, N, (3, 3), 1, f16=f16) != PATCH
+
+
 def test_refuses_what_the_convolution_refuses():
     from tmq_amd import _capi
     assert kernel_of(1, 64, 3, 3, 64, (5, 5), 0) == -1 and kernel_of(1, 64, 0, 3, 64, (1, 1), 0) == -1

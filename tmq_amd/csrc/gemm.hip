@@ -29,7 +29,7 @@ namespace tmq {
 bool mid_conv_ok(const void *x, const tmq_conv_shape *s);
 int launch_mid_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale,
                     const float *bias, const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream);
-// patch.hip: stride-1 convolutions over 128, 256 or 512 channels that are one well-filled round of its workgroups
+// patch.hip: stride-1 convolutions over 256 or 512 channels that are one well-filled round of its workgroups
 bool patch_conv_ok(const void *x, const tmq_conv_shape *s, int ho, int wo, const float *scale, const float *bias, const void *residual,
                    const void *y, int y_f16);
 int launch_patch_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale, const float *bias,

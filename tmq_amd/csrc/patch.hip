@@ -1,9 +1,9 @@
-// Stride-1 ternary convolutions over 128, 256 or 512 channels out of input patches in LDS, one round of workgroups, for gfx950.
+// Stride-1 ternary convolutions over 256 or 512 channels out of input patches in LDS, one round of workgroups, for gfx950.
 //
 // The im2col kernels (gemm.hip, mid.hip) fetch an input pixel once per filter tap and column tile through L1, and a wavefront
 // of theirs expands every weight for 64 rows. Here a workgroup fetches the input its output pixels' windows cover once, and a
 // wavefront multiplies a unit of 112 pixels (7 fragments of 16) x 64 channels over ONE 64-channel slab of the input, all taps:
-// the workgroup's wavefronts split the slabs (two, four or eight) and sum through LDS.
+// the workgroup's wavefronts split the slabs (four or eight) and sum through LDS.
 //   * Patch: the padded images as one run of positions (one row / column of padding serves the end of a row and the start of
 //     the next), so consecutive outputs' windows are one contiguous piece and a tap is a constant distance in it. A pixel's slab
 //     is 128 bytes in a pitch of 144: linear addresses that still spread sixteen pixels over all banks. Pixels go global ->
@@ -15,7 +15,7 @@
 //   * Everybody fetches, multiplies and stores at the same time, so a second round would add both ends again: worth it for one
 //     round that fills the chip. Clock stamps for 256 -> 256 on 14 x 14, batch 64, us: patch in LDS at 3.3, products 11.0 (1.87
 //     GHz, MFMAs 80 % of the time), sums and stores 3.4.
-// Batch 64, 3 x 3, us: 256 -> 256 on 14 x 14 20.2 -> 17.7; 512 -> 512 on 7 x 7 25.0 -> 19.8; 128 -> 128 on 28 x 28 20.4 -> 19.4.
+// Batch 64, 3 x 3, us: 256 -> 256 on 14 x 14 20.2 -> 17.7; 512 -> 512 on 7 x 7 25.0 -> 19.8.
 #include "common.h"
 #include "mfma.h"
 #include "tile_epilogue.h"
@@ -405,12 +405,15 @@ struct PatchPlan {
     int64_t rows, groups, pixels, bytes;   // output pixels and LDS of a workgroup, workgroups
 };
 
-// Whether the convolution is one well-filled round of units, and how it is cut. Workgroups of eight wavefronts, one a CU, from
-// 256 channels on, four and two a CU at 128. 1200 shapes, 64 .. 512 outputs: with 0.6 of the chip's units taken 0.75 .. 1.04 of the
-// im2col kernels' time at 256 channels (0.91 on average), with 0.55 0.80 .. 0.84 at 512, with 0.8 0.82 .. 1.03 at 128 (0.93);
-// below that, or over several rounds, up to 1.6; windows of fewer than nine taps don't pay for their ends.
+// Whether the convolution is one well-filled round of units, and how it is cut. Workgroups of eight wavefronts, one a CU (256
+// channels to at most 64 outputs: four wavefronts, two a CU). 1200 shapes, 64 .. 512 outputs: with 0.6 of the chip's units taken
+// 0.75 .. 1.04 of the im2col kernels' time at 256 channels (0.91 on average), with 0.55 0.80 .. 0.84 at 512; below that, or over
+// several rounds, up to 1.6; windows of fewer than nine taps don't pay for their ends. Nor do 128 channels: a wavefront's share
+// of the reduction is half as long, and 190 shapes that fill 0.8 of a round took 0.83 .. 1.33 (0.98 on average; to at most 64
+// outputs 0.95 .. 1.52, half of whose workgroups do not fit beside each other); 128 -> 128 on 28 x 28, batch 64, as part of
+// ResNet-18's second stage 81.0 us against 81.4 without.
 bool patch_plan(const tmq_conv_shape *s, int ho, int wo, PatchPlan &p) {
-    if (s->sy != 1 || s->sx != 1 || !(s->C == 128 || s->C == 256 || s->C == 512) || s->ky * s->kx < 9) return false;
+    if (s->sy != 1 || s->sx != 1 || !(s->C == 256 || s->C == 512) || s->ky * s->kx < 9) return false;
     const int64_t down = (int64_t)(s->ky - 1) * s->dy, across = (int64_t)(s->kx - 1) * s->dx;
     const int64_t top = s->py, left = s->px, bottom = ho - 1 - top + down - (s->H - 1), right = wo - 1 - left + across - (s->W - 1);
     // one row / column of padding serves the end of a row and the start of the next
@@ -424,7 +427,7 @@ bool patch_plan(const tmq_conv_shape *s, int ho, int wo, PatchPlan &p) {
     const int64_t units = (M + 16 * kFragments - 1) / (16 * kFragments) * tn;
     if (units > slots || tn > slots || M >= (int64_t)1 << 30 || M * s->N * 4 >= (int64_t)kNone) return false;
     const double filled = (double)units / slots * s->N / (64.0 * p.columns * tn);
-    if (filled < (p.slabs == 8 ? 0.55 : p.slabs == 4 ? 0.6 : 0.8)) return false;
+    if (filled < (p.slabs == 8 ? 0.55 : 0.6)) return false;
     // the pixels spread evenly over the round
     p.rows = (M + slots / tn - 1) / (slots / tn);
     p.groups = (M + p.rows - 1) / p.rows * tn;
@@ -474,8 +477,7 @@ int launch_patch_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, co
     const Epilogue ep{scale, bias, residual, y, relu, y_f16, {}};
 #define TMQ_PATCH(cg, sg) (y_f16 ? launch<cg, sg, true>(cv, ep, p.bytes, p.groups, stream) : launch<cg, sg, false>(cv, ep, p.bytes, p.groups, stream))
     if (p.slabs == 8) return TMQ_PATCH(1, 8);
-    if (p.slabs == 4) return p.columns == 2 ? TMQ_PATCH(2, 4) : TMQ_PATCH(1, 4);
-    return p.columns == 2 ? TMQ_PATCH(2, 2) : TMQ_PATCH(1, 2);
+    return p.columns == 2 ? TMQ_PATCH(2, 4) : TMQ_PATCH(1, 4);
 #undef TMQ_PATCH
 }
 
