@@ -30,6 +30,13 @@ def test_128_channels_stay_out_of_patches(B, H, W, N, f16):
     assert kernel_of(B, 128, H, W, N, (3, 3), 1, f16=f16) != PATCH
 
 
+# 512 channels: 0.57, 0.56, 0.57 of a round, then 0.6
+def test_less_than_six_tenths_of_a_round_stays_out_of_patches():
+    for B, H, W, N in [(47, 16, 8, 448), (25, 23, 3, 576), (35, 4, 23, 320)]:
+        assert kernel_of(B, 512, H, W, N, (3, 3), 1 if H != 16 else 0) != PATCH
+    assert kernel_of(43, 512, 5, 8, 640, (3, 3), 1) == PATCH
+
+
 def test_refuses_what_the_convolution_refuses():
     from tmq_amd import _capi
     assert kernel_of(1, 64, 3, 3, 64, (5, 5), 0) == -1 and kernel_of(1, 64, 0, 3, 64, (1, 1), 0) == -1
