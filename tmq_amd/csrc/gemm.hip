@@ -30,10 +30,10 @@ bool mid_conv_ok(const void *x, const tmq_conv_shape *s);
 int launch_mid_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale,
                     const float *bias, const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream);
 // patch.hip: stride-1 convolutions over 256 or 512 channels that are one well-filled round of its workgroups
-bool patch_conv_ok(const void *x, const tmq_conv_shape *s, int ho, int wo, const float *scale, const float *bias, const void *residual,
-                   const void *y, int y_f16);
-int launch_patch_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale, const float *bias,
-                      const void *residual, int relu, void *y, int y_f16, void *stream);
+bool patch_conv_ok(const tmq_conv_shape *s, int ho, int wo, int y_f16);      // (operands 16-byte aligned)
+// False if it does not take the call, else its status.
+bool launch_patch_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale, const float *bias,
+                       const void *residual, int relu, void *y, int y_f16, void *stream, int *status);
 
 namespace {
 
@@ -1582,8 +1582,8 @@ int tmq_ternary_conv2d_view(const void *x, const tmq_conv_shape *s, const void *
     const int64_t M = (int64_t)s->B * ho * wo, K = (int64_t)s->C * s->ky * s->kx;
     if (M == 0 || (view && (view->h_cnt == 0 || view->w_cnt == 0))) return TMQ_OK;
     const int y_f16 = y_dtype == TMQ_F16 ? 1 : 0;
-    if (!view && patch_conv_ok(x, s, ho, wo, scale, bias, residual, y, y_f16))
-        return launch_patch_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, stream);
+    int status;
+    if (!view && launch_patch_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, stream, &status)) return status;
     if (conv_splits_reduction(x, s, M, K))
         return launch_mid_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, view ? &map : nullptr, stream);
     if (view) return conv_tiles(x, s, ho, wo, native, ViewEpilogue{scale, bias, residual, y, relu, y_f16, map}, stream);
@@ -1596,7 +1596,7 @@ int tmq_ternary_conv2d_kernel(const tmq_conv_shape *s, int y_dtype) {
     RowMap map;
     if (const int rc = conv_plan(s, nullptr, ho, wo, map)) return rc;
     const int64_t M = (int64_t)s->B * ho * wo, K = (int64_t)s->C * s->ky * s->kx;
-    if (M && patch_conv_ok(nullptr, s, ho, wo, nullptr, nullptr, nullptr, nullptr, y_dtype == TMQ_F16)) return TMQ_KERNEL_PATCH;
+    if (M && patch_conv_ok(s, ho, wo, y_dtype == TMQ_F16)) return TMQ_KERNEL_PATCH;
     return conv_splits_reduction(nullptr, s, M, K) ? TMQ_KERNEL_SPLIT : TMQ_KERNEL_TILES;
 }
 

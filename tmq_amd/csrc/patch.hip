@@ -52,16 +52,6 @@ __device__ __forceinline__ void static_for(F &&f) {
     static_for_impl(f, std::make_integer_sequence<int, N_>{});
 }
 
-// A barrier of the workgroup for LDS alone: unlike __syncthreads it does not wait for loads and stores to memory.
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0xC07F);           // lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::: "memory");
-}
-
 typedef float float2v __attribute__((ext_vector_type(2)));
 
 // Eight channels of a lane, half h of its sixteen: n0 + 32 h + 8 g .. + 7 for fp16 results (one 16-byte piece), n0 + 32 h +
@@ -155,7 +145,8 @@ __global__ __launch_bounds__(64 * CG * SG, 2) void patch_conv_kernel(PatchConv c
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sg = wv % SG, n0 = (tn * CG + wv / SG) * 64;
     const int r16 = lane & 15, g = lane >> 4;
-    const int slabs = cv.C / kSlab, taps = cv.ky * cv.kx, patch_bytes = cv.pixels * kPixelBytes;
+    constexpr int slabs = SG;               // a wavefront's unit is one slab
+    const int taps = cv.ky * cv.kx, patch_bytes = cv.pixels * kPixelBytes;
 
     struct Place { int b, u, v; };          // image, row and column of a result in the grid
     auto place = [&](int m) {
@@ -268,20 +259,16 @@ __global__ __launch_bounds__(64 * CG * SG, 2) void patch_conv_kernel(PatchConv c
 
     {
         half8 a[kAhead], b0[WN], b1[WN];
-        const int steps = taps * (slabs / SG);
-        // a step is one tap of one slab; `at` walks them one ahead of the multiplication
-        struct Step { int slab, ti, tj; } at{sg, 0, 0};
+        // a step is one tap of the wavefront's slab; `at` walks them one ahead of the multiplication
+        struct Step { int ti, tj; } at{0, 0};
         auto advance = [&](int step) {                            // to the step behind `step`; the last one stays
-            if (step + 1 >= steps) return;
+            if (step + 1 >= taps) return;
             if (++at.tj == cv.kx) {
                 at.tj = 0;
-                if (++at.ti == cv.ky) {
-                    at.ti = 0;
-                    at.slab += SG;
-                }
+                ++at.ti;
             }
         };
-        auto distance = [&] { return (uint32_t)(at.slab * patch_bytes + (at.ti * cv.dy * cv.Wp + at.tj * cv.dx) * kPixelBytes); };
+        auto distance = [&] { return (uint32_t)(sg * patch_bytes + (at.ti * cv.dy * cv.Wp + at.tj * cv.dx) * kPixelBytes); };
         uint32_t off = distance(), noff;
         advance(0);
         noff = distance();
@@ -289,8 +276,8 @@ __global__ __launch_bounds__(64 * CG * SG, 2) void patch_conv_kernel(PatchConv c
         for (int q = 0; q < kAhead; q++) a[q] = load_a(q, off);
 #pragma unroll
         for (int j = 0; j < WN; j++) b0[j] = decode_step(w[j], 0);
-        for (int step = 0; step < steps; step++) {
-            load_w(wnext, (at.ti * cv.kx + at.tj) * slabs + at.slab);
+        for (int step = 0; step < taps; step++) {
+            load_w(wnext, (at.ti * cv.kx + at.tj) * slabs + sg);
             advance(step + 1);
             const uint32_t noff2 = distance();
             __builtin_amdgcn_sched_barrier(0);
@@ -441,20 +428,23 @@ bool patch_plan(const tmq_conv_shape *s, int ho, int wo, PatchPlan &p) {
     return p.bytes <= (waves > 4 ? 160 : 80) * 1024;
 }
 
-}  // namespace
-
-bool patch_conv_ok(const void *x, const tmq_conv_shape *s, int ho, int wo, const float *scale, const float *bias, const void *residual,
-                   const void *y, int y_f16) {
-    PatchPlan p;
-    return s->N % (y_f16 ? 8 : 4) == 0 && aligned16(x) && aligned16(y) && aligned16(residual) && aligned16(scale) && aligned16(bias) &&
-           (int64_t)s->B * s->H * s->W * s->C < (int64_t)0x7FFFFFF0 && native_blocks_n(s->N) * native_blocks_k((int64_t)s->C * s->ky * s->kx) < (1 << 21) &&
-           patch_plan(s, ho, wo, p);
+bool patch_conv_ok(const tmq_conv_shape *s, int ho, int wo, int y_f16, PatchPlan &p) {
+    return s->N % (y_f16 ? 8 : 4) == 0 && (int64_t)s->B * s->H * s->W * s->C < (int64_t)0x7FFFFFF0 &&
+           native_blocks_n(s->N) * native_blocks_k((int64_t)s->C * s->ky * s->kx) < (1 << 21) && patch_plan(s, ho, wo, p);
 }
 
-int launch_patch_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale, const float *bias,
-                      const void *residual, int relu, void *y, int y_f16, void *stream) {
+}  // namespace
+
+bool patch_conv_ok(const tmq_conv_shape *s, int ho, int wo, int y_f16) {
     PatchPlan p;
-    if (!patch_plan(s, ho, wo, p)) return TMQ_ERR_UNSUPPORTED;
+    return patch_conv_ok(s, ho, wo, y_f16, p);
+}
+
+bool launch_patch_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale, const float *bias,
+                       const void *residual, int relu, void *y, int y_f16, void *stream, int *status) {
+    PatchPlan p;
+    if (!(aligned16(x) && aligned16(y) && aligned16(residual) && aligned16(scale) && aligned16(bias) && patch_conv_ok(s, ho, wo, y_f16, p)))
+        return false;
     PatchConv cv{};
     cv.x = static_cast<const _Float16 *>(x);
     cv.native = static_cast<const uint32_t *>(native);
@@ -477,9 +467,9 @@ int launch_patch_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, co
     cv.jobs = (s->W + kJobPixels - 1) / kJobPixels;
     const Epilogue ep{scale, bias, residual, y, relu, y_f16, {}};
 #define TMQ_PATCH(cg, sg) (y_f16 ? launch<cg, sg, true>(cv, ep, p.bytes, p.groups, stream) : launch<cg, sg, false>(cv, ep, p.bytes, p.groups, stream))
-    if (p.slabs == 8) return TMQ_PATCH(1, 8);
-    return p.columns == 2 ? TMQ_PATCH(2, 4) : TMQ_PATCH(1, 4);
+    *status = p.slabs == 8 ? TMQ_PATCH(1, 8) : p.columns == 2 ? TMQ_PATCH(2, 4) : TMQ_PATCH(1, 4);
 #undef TMQ_PATCH
+    return true;
 }
 
 }  // namespace tmq

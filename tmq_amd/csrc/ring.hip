@@ -50,15 +50,6 @@ __device__ __forceinline__ void dword_to_lds(BufferResource rsrc, uint32_t lane_
 #endif
 }
 
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0xC07F);           // lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::: "memory");
-}
-
 // Waits until at most r * kN loads are outstanding (r uniform, 0 .. kMax).
 template <int kN, int kMax>
 __device__ __forceinline__ void wait_younger(int r) {
