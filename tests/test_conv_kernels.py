@@ -30,11 +30,12 @@ def test_128_channels_stay_out_of_patches(B, H, W, N, f16):
     assert kernel_of(B, 128, H, W, N, (3, 3), 1, f16=f16) != PATCH
 
 
-# 512 channels: 0.57, 0.56, 0.57 of a round, then 0.6
-def test_less_than_six_tenths_of_a_round_stays_out_of_patches():
-    for B, H, W, N in [(47, 16, 8, 448), (25, 23, 3, 576), (35, 4, 23, 320)]:
-        assert kernel_of(B, 512, H, W, N, (3, 3), 1 if H != 16 else 0) != PATCH
-    assert kernel_of(43, 512, 5, 8, 640, (3, 3), 1) == PATCH
+# 512 channels: at most 256 tiles of 64 x 64, then more of them (0.57 to 0.59 of a round of units)
+def test_one_round_of_tiles_stays_out_of_patches():
+    for B, H, W, N, pad in [(47, 16, 8, 448, 0), (25, 23, 3, 576, 1), (40, 10, 5, 512, 1), (31, 7, 8, 572, 1)]:
+        assert kernel_of(B, 512, H, W, N, (3, 3), pad, f16=False) != PATCH
+    for B, H, W, N in [(32, 12, 6, 456), (44, 7, 6, 576), (20, 35, 4, 384)]:
+        assert kernel_of(B, 512, H, W, N, (3, 3), 1) == PATCH
 
 
 def test_refuses_what_the_convolution_refuses():

@@ -393,13 +393,14 @@ struct PatchPlan {
 };
 
 // Whether the convolution is one well-filled round of units, and how it is cut. Workgroups of eight wavefronts, one a CU (256
-// channels to at most 64 outputs: four wavefronts, two a CU). Against the im2col kernels, 4 .. 640 outputs: with 0.6 of the
-// chip's units taken 0.68 .. 1.05 of their time at 256 channels (268 shapes, 0.89 on average) and 0.70 .. 0.88 at 512 (98, 0.80);
-// with 0.55 to 0.6 0.73 .. 1.09 at 512 (narrow images above 1: 512 -> 448 on 14 x 6, batch 47 17.4 -> 18.7 us); below that, or over several
-// rounds, up to 1.6; windows of fewer than nine taps don't pay for their ends. Nor do 128 channels: a wavefront's share
-// of the reduction is half as long, and 190 shapes that fill 0.8 of a round took 0.83 .. 1.33 (0.98 on average; to at most 64
-// outputs 0.95 .. 1.52, half of whose workgroups do not fit beside each other); 128 -> 128 on 28 x 28, batch 64, as part of
-// ResNet-18's second stage 81.0 us against 81.4 without.
+// channels to at most 64 outputs: four wavefronts, two a CU). Against the im2col kernels, 4 .. 640 outputs: at 256 channels with
+// 0.6 of the chip's units taken 0.68 .. 1.05 of their time (268 shapes, 0.89 on average); at 512, where a round of theirs is 256
+// tiles of 64 x 64, 0.70 .. 0.88 beyond one round (130 shapes, 0.79) and 0.92 .. 1.09 up to there (512 -> 576 on 23 x 3, batch 25:
+// 243 tiles, 17.4 us and 19.1; on 7 x 6, batch 44: 261, 23.1 and 18.0); with less filled, or over several rounds, up to 1.6;
+// windows of fewer than nine taps don't pay for their ends. Nor do 128 channels: a wavefront's share of the reduction is half
+// as long, and 190 shapes that fill 0.8 of a round took 0.83 .. 1.33 (0.98 on average; to at most 64 outputs 0.95 .. 1.52, half
+// of whose workgroups do not fit beside each other); 128 -> 128 on 28 x 28, batch 64, as part of ResNet-18's second stage 81.0 us
+// against 81.4 without.
 bool patch_plan(const tmq_conv_shape *s, int ho, int wo, PatchPlan &p) {
     if (s->sy != 1 || s->sx != 1 || !(s->C == 256 || s->C == 512) || s->ky * s->kx < 9) return false;
     const int64_t down = (int64_t)(s->ky - 1) * s->dy, across = (int64_t)(s->kx - 1) * s->dx;
@@ -415,7 +416,7 @@ bool patch_plan(const tmq_conv_shape *s, int ho, int wo, PatchPlan &p) {
     const int64_t units = (M + 16 * kFragments - 1) / (16 * kFragments) * tn;
     if (units > slots || tn > slots || M >= (int64_t)1 << 30 || M * s->N * 4 >= (int64_t)kNone) return false;
     const double filled = (double)units / slots * s->N / (64.0 * p.columns * tn);
-    if (filled < 0.6) return false;
+    if (filled < (p.slabs == 8 ? 0.55 : 0.6) || (p.slabs == 8 && (M + 63) / 64 * ((s->N + 63) / 64) <= 256)) return false;
     // the pixels spread evenly over the round
     p.rows = (M + slots / tn - 1) / (slots / tn);
     p.groups = (M + p.rows - 1) / p.rows * tn;
