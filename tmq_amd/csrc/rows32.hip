@@ -243,8 +243,9 @@ template <int SETS, int WN>
 int by_pairs(const Rows32 &a, void *stream) {
     if (a.pairs <= 8) return launch<SETS, WN, 1, 1>(a, stream);
     if (a.pairs <= 16) return launch<SETS, WN, 2, 2>(a, stream);
-    if (SETS == 2 || a.pairs <= 32) return launch<SETS, WN, 4, 4>(a, stream);
-    return launch<SETS, WN, 8, 8>(a, stream);
+    if constexpr (SETS == 1 && WN == 1)                        // (rows32_ok: more than 2048 values, at most 4096 channels)
+        if (a.pairs > 32) return launch<SETS, WN, 8, 8>(a, stream);
+    return launch<SETS, WN, 4, 4>(a, stream);
 }
 
 // One pass of workgroups over the CUs where that can be had: every workgroup prepares all the rows, whatever it multiplies.
@@ -264,10 +265,15 @@ int by_width(const Rows32 &a, void *stream) {
 // nine rows on), and every workgroup prepares them again, which wide layers over long rows pay for: against the split in a
 // launch of its own, 600 shapes, 0.85 of its time at the median of 1 .. 8 rows and 0.5 of 9 .. 16 inside these lines (1.07 at
 // most), 1.08 .. 1.65 beyond (2304 x 25768, 6 rows 10.6 -> 14.0 us). 16 rows x 512 -> 512: 9.1 -> 3.9 us; 8 rows x 2048 -> 2048
-// 6.9 -> 5.0; 3 rows x 4096 -> 4096 7.5 -> 6.7.
+// 6.9 -> 5.0; 3 rows x 4096 -> 4096 7.5 -> 6.7. So do the widest layers over rows of any length, from the second round of
+// workgroups on (their sums leave room for one a CU; 360 shapes of 12000 columns and more): up to 32768 columns 0.42 .. 0.90 for
+// 9 .. 16 rows, beyond 0.81 .. 0.95 for up to 12 short ones to 65536 and 0.93 .. 1.36 for the others (16 rows x 40 -> 338116
+// 65.6 -> 84.4); 5 .. 8 rows 0.50 .. 0.99 to 131072 columns and to 32768 for more than 512 values, 0.79 .. 1.05 from there on;
+// fewer rows 0.40 .. 0.85 at any width. More than 1024 values against more than 16384 columns 1.04 .. 1.12 from three rows on.
 bool rows32_ok(const void *x, int64_t M, int64_t K, int64_t N) {
     if (M < 1 || M > 16 || K < 1 || N < 1 || !aligned16(x)) return false;
-    if (M > 8) return K <= 2048 && K * N <= (int64_t)1 << 25;
+    if (M > 8) return K <= 2048 && K * N <= (int64_t)1 << 25 && (N <= 32768 || (M <= 12 && N <= 65536 && K <= 512));
+    if ((M > 4 && N > (K > 512 ? 32768 : 131072)) || (M > 2 && K > 1024 && N > 16384)) return false;
     return K <= 2048 ? K * N <= (int64_t)3 << 23 : K <= 4096 && N <= 4096;
 }
 
