@@ -16,10 +16,12 @@
 // 64 -> 64, 3 x 3 on one 56 x 56 image 4.5 -> 4.1; 128 rows x 400 -> 1024 5.2 -> 3.9; 333 fp32 rows, 2000 -> 1000 10.8 -> 9.7.
 #include "common.h"
 #include "mfma.h"
-#include <type_traits>
-
+#include <utility>
 
 namespace tmq {
+
+int ring_tile(int64_t M, int64_t K, int64_t N, bool conv);
+
 namespace {
 
 struct RingPlace {               // conv: geometry of the im2col view; dense: K alone
@@ -280,44 +282,53 @@ struct RingTile {
 };
 constexpr RingTile kRingTiles[] = {{1, 1, 4, 5}, {1, 1, 8, 4}, {1, 2, 4, 4}, {1, 2, 8, 4}, {2, 2, 4, 3}, {2, 2, 8, 2},
                                    {1, 4, 4, 4}, {2, 4, 8, 2}, {2, 4, 4, 3}, {4, 4, 4, 2}, {4, 4, 8, 2}};
+constexpr int kTiles = sizeof(kRingTiles) / sizeof(kRingTiles[0]);
 
 // Microseconds a launch is expected to take, fitted to 1700 shapes (convolutions of 64 .. 512 channels, 1 x 1 .. 5 x 5, dense rows,
 // fp32 row pairs; 17 .. 15000 rows, 16 .. 8192 columns) with eleven tiles each: the launch, the chain of a wavefront's pairs for
 // every round of workgroups, and what shares a CU -- vector-memory instructions, products, sums. The tile it picks takes 1.01 of
-// the fastest one's time on average.
-double ring_cost(const RingTile &t, int64_t M, int64_t pairs, int64_t N, bool conv) {
+// the fastest one's time on average. The tile is a constant here: no division is left of the eleven evaluations.
+template <int I>
+double ring_cost(int64_t M, int64_t pairs, int64_t N, bool conv) {
+    constexpr RingTile t = kRingTiles[I];
+    constexpr int64_t fit = 160 * 1024 / ring_lds(t.wm, t.wn, t.waves, t.depth), resident = fit < 32 / t.waves ? fit : 32 / t.waves;
+    constexpr double frags = t.wm * t.wn;
     const int64_t groups = ((M + 16 * t.wm - 1) / (16 * t.wm)) * ((N + 16 * t.wn - 1) / (16 * t.wn));
-    int64_t resident = 160 * 1024 / ring_lds(t.wm, t.wn, t.waves, t.depth);
-    if (resident > 32 / t.waves) resident = 32 / t.waves;
     const double rounds = (double)((groups + 256 * resident - 1) / (256 * resident)), chain = (double)((pairs + t.waves - 1) / t.waves);
-    const double per_cu = (double)((groups + 255) / 256), frags = t.wm * t.wn;
+    const double per_cu = (double)((groups + 255) / 256);
     return 2.35 + (conv ? 0.46 : 0.0) + rounds * (0.416 + 0.0684 * frags + chain * (0.112 + 0.00901 * frags)) +
            per_cu * (0.168 + 0.006 * t.waves * frags + pairs * (0.00623 * (2 * t.wm + t.wn) + 0.00214 * frags + (conv ? 0.00218 * t.wm : 0.0)));
 }
 
+template <int... I>
+int cheapest_tile(int64_t M, int64_t pairs, int64_t N, bool conv, std::integer_sequence<int, I...>) {
+    const double us[] = {ring_cost<I>(M, pairs, N, conv)...};
+    int best = 0;
+    for (int i = 1; i < kTiles; i++)
+        if (us[i] < us[best]) best = i;
+    return best;
+}
+
+template <bool CONV, int I, class Map>
+int launch_tile(const RingArgs<Map> &a, void *stream) {
+    constexpr RingTile t = kRingTiles[I];
+    return launch<t.wm, t.wn, t.waves, t.depth, CONV>(a, stream);
+}
+
 template <bool CONV, class Map>
 int by_cost(const RingArgs<Map> &a, void *stream) {
-    int best = 0;
-    double least = 1e30;
-    for (int i = 0; i < (int)(sizeof(kRingTiles) / sizeof(kRingTiles[0])); i++) {
-        const double us = ring_cost(kRingTiles[i], a.M, a.pairs, a.N, CONV);
-        if (us < least) {
-            least = us;
-            best = i;
-        }
-    }
-    switch (best) {
-        case 0: return launch<1, 1, 4, 5, CONV>(a, stream);
-        case 1: return launch<1, 1, 8, 4, CONV>(a, stream);
-        case 2: return launch<1, 2, 4, 4, CONV>(a, stream);
-        case 3: return launch<1, 2, 8, 4, CONV>(a, stream);
-        case 4: return launch<2, 2, 4, 3, CONV>(a, stream);
-        case 5: return launch<2, 2, 8, 2, CONV>(a, stream);
-        case 6: return launch<1, 4, 4, 4, CONV>(a, stream);
-        case 7: return launch<2, 4, 8, 2, CONV>(a, stream);
-        case 8: return launch<2, 4, 4, 3, CONV>(a, stream);
-        case 9: return launch<4, 4, 4, 2, CONV>(a, stream);
-        default: return launch<4, 4, 8, 2, CONV>(a, stream);
+    switch (ring_tile(a.M, a.K, a.N, CONV)) {
+        case 0: return launch_tile<CONV, 0>(a, stream);
+        case 1: return launch_tile<CONV, 1>(a, stream);
+        case 2: return launch_tile<CONV, 2>(a, stream);
+        case 3: return launch_tile<CONV, 3>(a, stream);
+        case 4: return launch_tile<CONV, 4>(a, stream);
+        case 5: return launch_tile<CONV, 5>(a, stream);
+        case 6: return launch_tile<CONV, 6>(a, stream);
+        case 7: return launch_tile<CONV, 7>(a, stream);
+        case 8: return launch_tile<CONV, 8>(a, stream);
+        case 9: return launch_tile<CONV, 9>(a, stream);
+        default: return launch_tile<CONV, 10>(a, stream);
     }
 }
 
@@ -354,6 +365,11 @@ bool ring_ok(int64_t M, int64_t K, int64_t N, const float *scale, const float *b
     const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
     return K % 64 == 0 && K <= (tiles64 >= 192 ? 3583 : 4608) && N % 4 == 0 && N < (1 << 20) && M < (int64_t)0x7FFFFFFF && aligned16(y) &&
            aligned16(residual) && aligned16(scale) && aligned16(bias);
+}
+
+// Its tile for a problem, an index into kRingTiles.
+int ring_tile(int64_t M, int64_t K, int64_t N, bool conv) {
+    return cheapest_tile(M, K / 64, N, conv, std::make_integer_sequence<int, kTiles>{});
 }
 
 int launch_ring_dense(const void *x, int64_t M, int64_t K, const void *native, int64_t N, const float *scale, const float *bias,
