@@ -353,6 +353,11 @@ int tmq_fp32_rows_self_scaled_for(const void *x, int64_t M, int64_t K, int64_t N
  * its own power of two and split into two fp16 terms by the workgroups that multiply it. A workspace is not used. */
 int tmq_fp32_rows_one_launch(const void *x, int64_t M, int64_t K, int64_t N);
 
+/* Which kernel multiplies 17 rows or more behind tmq_ternary_linear_ws, given its workspace and 16-byte aligned operands: for
+ * profiles and tests (host only). TMQ_KERNEL_TILES, _SPLIT or _RING + tile (tmq_ternary_conv2d_kernel's values), or a negative
+ * status (TMQ_ERR_UNSUPPORTED: cut across workgroups, or too large to prepare). */
+int tmq_ternary_rows_kernel(int x_dtype, int64_t M, int64_t K, int64_t N);
+
 /* Range handling for fp32 activations (no counterpart in the reference, whose kernels multiply fp32
  * activations in fp32, tmq/tmq_cuda.cu:242-427). Scans n fp32 values and writes prescale[0] = s,
  * prescale[1] = 1 / s (device, 2 floats): s is the power of two that brings the largest finite |x| into
@@ -443,7 +448,7 @@ int tmq_ternary_conv2d_view(const void *x, const tmq_conv_shape *shape, const vo
 
 /* Which kernel tmq_ternary_conv2d launches for a convolution whose operands are all 16-byte aligned: for profiles and tests
  * (host only, nothing is launched). A TMQ_KERNEL_ value, or a negative status. */
-enum { TMQ_KERNEL_TILES = 0, TMQ_KERNEL_SPLIT = 1, TMQ_KERNEL_PATCH = 2 };
+enum { TMQ_KERNEL_TILES = 0, TMQ_KERNEL_SPLIT = 1, TMQ_KERNEL_PATCH = 2, TMQ_KERNEL_RING = 16 /* + its tile, 0 .. 10 */ };
 int tmq_ternary_conv2d_kernel(const tmq_conv_shape *shape, int y_dtype);
 
 /* Several such convolutions of ONE input (same B, C, H, W and N; windows, padding and dilation of their own) written

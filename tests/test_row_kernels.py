@@ -15,3 +15,22 @@ def test_wide_layers_over_few_fp32_rows():
     for M in (3, 4):
         assert [one(None, M, K, N) for K, N in ((8, 1 << 20), (1025, 16384), (1025, 16385))] == [1, 1, 0]
     assert one(None, 2, 1025, 16385) == 1
+
+
+def test_long_reductions_on_the_same_tile_stay_with_mid():
+    """Where ring.hip would take mid.hip's own tile, a long reduction is faster in mid.hip: whole weight blocks (K a multiple of
+    2048), and single pairs from K = 2048 (16 x 32 tiles) or 2560 (32 x 64) on."""
+    from tmq_amd import _capi
+    kernel, SPLIT, RING = _capi.load().tmq_ternary_rows_kernel, 1, 16
+    rows = lambda M, K, N: kernel(_capi.F16, M, K, N)
+    for M, N in ((32, 4096), (64, 2048), (64, 4096), (82, 4160), (128, 4096), (256, 2048)):
+        assert rows(M, 4096, N) == SPLIT, (M, N)
+        assert rows(M, 1024, N) >= RING, (M, N)
+    assert rows(80, 2048, 8192) == SPLIT and rows(48, 2048, 11008) >= RING          # one round of 64 x 64 tiles; two of 32 x 64
+    assert [rows(17, K, 4096) >= RING for K in (1984, 2304)] == [True, False]       # 16 x 32
+    assert [rows(128, K, 3072) >= RING for K in (2496, 2560)] == [True, False]      # 32 x 64
+    assert [rows(621, K, 1536) >= RING for K in (640, 704)] == [True, False]        # 32 x 64, four wavefronts, two rounds
+    assert rows(17, 64, 16) >= RING
+    # fp32 row pairs: only whole weight blocks
+    assert kernel(_capi.F32, 60, 3584, 4096) >= RING and kernel(_capi.F32, 64, 4096, 4096) == SPLIT
+    assert kernel(_capi.F16, 16, 64, 64) < 0

@@ -92,6 +92,7 @@ SIGNATURES = {
     "tmq_fp32_rows_prefer_split": (_int, [_i64, _i64, _i64]),
     "tmq_fp32_rows_self_scaled": (_int, [_vp, _i64, _i64]),
     "tmq_fp32_rows_self_scaled_for": (_int, [_vp, _i64, _i64, _i64]),
+    "tmq_ternary_rows_kernel": (_int, [_int, _i64, _i64, _i64]),
     "tmq_fp32_rows_one_launch": (_int, [_vp, _i64, _i64, _i64]),
     "tmq_multi_plan": (_int, [ctypes.POINTER(Segment), _int, ctypes.POINTER(_u32)]),
     "tmq_qloss_multi_workspace_bytes": (_sz, [_u32]),

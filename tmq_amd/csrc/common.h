@@ -39,6 +39,11 @@ inline bool split_reduction_pays(int64_t M, int64_t K, int64_t N) {
     return K >= 512 ? tiles64 <= ((K >= 8192 && N >= 2048) ? 640 : 512) : tiles64 <= K / 2;
 }
 
+// A tile of the split-reduction kernel of ring.hip: fragments of 16 rows and of 16 columns, wavefronts, pairs in flight.
+struct RingTile {
+    int wm, wn, waves, depth;
+};
+
 // 16 bytes per lane from global memory straight into LDS through a buffer resource: lane l's 16 bytes at byte
 // `offset` of the buffer go to byte 16 l of the (uniform) destination; a lane whose offset lies past the end of
 // the buffer gets zeros. The padding taps of a convolution then cost a select of the offset instead of a select

@@ -27,6 +27,7 @@ namespace tmq {
 
 // mid.hip: split-reduction kernel for outputs of a few hundred 64 x 64 tiles
 bool mid_conv_ok(const void *x, const tmq_conv_shape *s);
+int split_reduction_tile(int64_t M, int64_t K, int64_t N, bool conv, bool pairs);   // of ring.hip, or -1: mid.hip's own
 int launch_mid_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale,
                     const float *bias, const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream);
 // patch.hip: stride-1 convolutions over 256 or 512 channels that are one well-filled round of its workgroups
@@ -1459,12 +1460,25 @@ int conv_tiles(const void *x, const tmq_conv_shape *s, int ho, int wo, const voi
                          native, M, K, s->N, ep, stream);
 }
 
+int split_kernel(int64_t M, int64_t K, int64_t N, bool conv, bool pairs) {
+    const int tile = split_reduction_tile(M, K, N, conv, pairs);
+    return tile < 0 ? TMQ_KERNEL_SPLIT : TMQ_KERNEL_RING + tile;
+}
+
 }  // namespace
 }  // namespace tmq
 
 using namespace tmq;
 
 extern "C" {
+
+int tmq_ternary_rows_kernel(int x_dtype, int64_t M, int64_t K, int64_t N) {
+    if ((x_dtype != TMQ_F16 && x_dtype != TMQ_F32) || M <= 16 || K <= 0 || N <= 0) return TMQ_ERR_INVALID_ARG;
+    const bool pairs = x_dtype == TMQ_F32;
+    const int64_t rows = pairs ? pair_rows16(M) : M, Kp = padded_k(K);
+    if (rows * Kp >= (int64_t)0x7FFFFFFF || (!pairs && rows_split_slices(nullptr, M, K, N))) return TMQ_ERR_UNSUPPORTED;
+    return split_reduction_pays(rows, Kp, N) ? split_kernel(rows, Kp, N, false, pairs) : TMQ_KERNEL_TILES;
+}
 
 size_t tmq_ternary_linear_workspace_bytes(int x_dtype, int64_t M, int64_t K, int64_t N) {
     if (M <= 0 || K <= 0 || N <= 0) return 0;
@@ -1597,7 +1611,7 @@ int tmq_ternary_conv2d_kernel(const tmq_conv_shape *s, int y_dtype) {
     if (const int rc = conv_plan(s, nullptr, ho, wo, map)) return rc;
     const int64_t M = (int64_t)s->B * ho * wo, K = (int64_t)s->C * s->ky * s->kx;
     if (M && patch_conv_ok(s, ho, wo, y_dtype == TMQ_F16)) return TMQ_KERNEL_PATCH;
-    return conv_splits_reduction(nullptr, s, M, K) ? TMQ_KERNEL_SPLIT : TMQ_KERNEL_TILES;
+    return conv_splits_reduction(nullptr, s, M, K) ? split_kernel(M, K, s->N, true, false) : TMQ_KERNEL_TILES;
 }
 
 int tmq_ternary_conv2d_phases(const void *x, const tmq_conv_phase *phases, int count, const tmq_epilogue *epilogue, void *y,

@@ -1,7 +1,7 @@
 // Ternary GEMM / implicit-GEMM convolution for outputs too small to fill the chip with big tiles
 // (a few hundred 64 x 64 tiles): the reduction is split over the wavefronts of a workgroup. Most such problems go on to
-// ring.hip (ring_ok says which and what both measure); what follows serves the longest reductions and results that are no
-// whole aligned quads.
+// ring.hip; what follows serves long reductions (mid_holds says which, and what both measure) and results that are no whole
+// aligned quads.
 //
 // A workgroup of WAVES wavefronts owns a (16 WM) x (16 WN) output tile; wavefront kg multiplies the
 // whole tile over the "pairs" (64 reduction indices each) kg, kg + WAVES, ... and the partial tiles
@@ -35,10 +35,12 @@ namespace tmq {
 
 // ring.hip: most of these problems, with everything a workgroup waits for asked for at once
 bool ring_ok(int64_t M, int64_t K, int64_t N, const float *scale, const float *bias, const void *residual, const void *y);
-int launch_ring_dense(const void *x, int64_t M, int64_t K, const void *native, int64_t N, const float *scale, const float *bias,
+int ring_tile(int64_t M, int64_t K, int64_t N, bool conv);
+RingTile ring_tile_shape(int tile);
+int launch_ring_dense(int tile, const void *x, int64_t M, int64_t K, const void *native, int64_t N, const float *scale, const float *bias,
                       const void *residual, int relu, void *y, int y_f16, const PairMap *pairs, void *stream);
-int launch_ring_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale, const float *bias,
-                     const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream);
+int launch_ring_conv(int tile, const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale,
+                     const float *bias, const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream);
 
 namespace {
 
@@ -997,12 +999,17 @@ int launch_stream32(const void *x, const void *native, int64_t M, int64_t K, int
     return check_launch();
 }
 
+// A problem's tile: fragments of 16 rows and of 16 columns, wavefronts, whole weight blocks per wavefront or single pairs.
+struct MidTile {
+    int wm, wn, waves;
+    bool blocks;
+    int64_t count(int64_t M, int64_t N) const { return ((M + 16 * wm - 1) / (16 * wm)) * ((N + 16 * wn - 1) / (16 * wn)); }
+};
+
 // Geometry: 64 x 128 tiles where they save a pass over the CUs (below); else the largest smaller tile
 // that keeps most CUs busy; then as many wavefronts per tile as it takes to put about ten on every CU,
 // each with at least two pairs to multiply.
-template <class Rows, class Ep>
-int dispatch(const Rows &rows, const void *native, int64_t M, int64_t K, int64_t N, const Ep &ep,
-             void *stream) {
+MidTile mid_tile(int64_t M, int64_t K, int64_t N, bool conv) {
     const int64_t npairs = (K + 63) / 64, tn = (N + 63) / 64;
     // Whole weight blocks per wavefront (one 16-byte load per lane and block instead of four dword loads) when the
     // blocks deal out evenly (or there are many); else pairs (K = 4608 over 4 wavefronts: 18 blocks would leave two
@@ -1022,20 +1029,9 @@ int dispatch(const Rows &rows, const void *native, int64_t M, int64_t K, int64_t
     // below, 256 -> 512 channels at stride 2 18.5 -> 16.7, 1024 -> 512 channels 47.8 -> 43.8 (whole weight blocks per
     // wavefront lose here: 61 us). Dense problems of these sizes stay as they are (M = 512 at K = N = 4096: 24.0 us on
     // 64 x 128 tiles, 27.6 this way), and so do convolutions with fewer tiles (98 tiles: 27 us on smaller tiles, 56 so).
-    constexpr bool kConv = Rows::kBuffer;
-    if (kConv && npairs >= 16 && ((M + 63) / 64) * tn >= 256 && ((M + 63) / 64) * tn <= 512)
-        return launch<4, 4, 4, Rows>(rows, native, M, K, N, ep, stream);
-    {
-        const int64_t tm = (M + 63) / 64, passes64 = (tm * tn + 255) / 256, passes128 = (tm * ((N + 127) / 128) + 255) / 256;
-        if (npairs >= 16 && passes64 >= 2 && 17 * passes128 < 10 * passes64)
-        {
-            if (by_blocks(4)) return launch<4, 8, 4, Rows, true>(rows, native, M, K, N, ep, stream);
-            // pairs two ahead (three LDS slots) once a wavefront has six or more: K = 4608 at M = 512, N = 4096
-            // 25.9 -> 24.7 us, the 512-channel convolutions of ResNet-18 29.5 -> 29.2 us
-            if (npairs >= 24) return launch<4, 8, 4, Rows, false, 3>(rows, native, M, K, N, ep, stream);
-            return launch<4, 8, 4, Rows>(rows, native, M, K, N, ep, stream);
-        }
-    }
+    if (conv && npairs >= 16 && ((M + 63) / 64) * tn >= 256 && ((M + 63) / 64) * tn <= 512) return {4, 4, 4, false};
+    const int64_t tm = (M + 63) / 64, passes64 = (tm * tn + 255) / 256, passes128 = (tm * ((N + 127) / 128) + 255) / 256;
+    if (npairs >= 16 && passes64 >= 2 && 17 * passes128 < 10 * passes64) return {4, 8, 4, by_blocks(4)};
     // Otherwise the largest of 64 x 64, 32 x 64, 32 x 32, 16 x 32 that still gives most CUs a tile (measured
     // at K = N = 4096: M = 64 10.0 -> 7.6 us with 32 x 32, M = 17 9.7 -> 6.4 us with 16 x 32, while
     // M = 96 .. 128 stay best on 32 x 64).
@@ -1046,30 +1042,84 @@ int dispatch(const Rows &rows, const void *native, int64_t M, int64_t K, int64_t
     else if (tiles(32, 32) >= 192) { bm = 32; bn = 32; }
     int waves = 1;
     while (waves < 8 && tiles(bm, bn) * waves < 2560 && npairs >= 4 * waves) waves *= 2;
+    return {bm / 16, bn / 16, waves, by_blocks(waves)};
+}
+
+template <class Rows, class Ep>
+int dispatch(const Rows &rows, const void *native, int64_t M, int64_t K, int64_t N, const Ep &ep,
+             void *stream) {
+    const MidTile tile = mid_tile(M, K, N, Rows::kBuffer);
+    if (tile.wn == 8) {
+        if (tile.blocks) return launch<4, 8, 4, Rows, true>(rows, native, M, K, N, ep, stream);
+        // pairs two ahead (three LDS slots) once a wavefront has six or more: K = 4608 at M = 512, N = 4096
+        // 25.9 -> 24.7 us, the 512-channel convolutions of ResNet-18 29.5 -> 29.2 us
+        if (K > 23 * 64) return launch<4, 8, 4, Rows, false, 3>(rows, native, M, K, N, ep, stream);
+        return launch<4, 8, 4, Rows>(rows, native, M, K, N, ep, stream);
+    }
     auto go = [&](auto wm_tag, auto wn_tag) {
         constexpr int WM = decltype(wm_tag)::value, WN = decltype(wn_tag)::value;
-        if (by_blocks(waves)) {
-            switch (waves) {
+        if (tile.blocks) {
+            switch (tile.waves) {
                 case 1: return launch<WM, WN, 1, Rows, true>(rows, native, M, K, N, ep, stream);
                 case 2: return launch<WM, WN, 2, Rows, true>(rows, native, M, K, N, ep, stream);
                 case 4: return launch<WM, WN, 4, Rows, true>(rows, native, M, K, N, ep, stream);
                 default: return launch<WM, WN, 8, Rows, true>(rows, native, M, K, N, ep, stream);
             }
         }
-        switch (waves) {
+        switch (tile.waves) {
             case 1: return launch<WM, WN, 1, Rows>(rows, native, M, K, N, ep, stream);
             case 2: return launch<WM, WN, 2, Rows>(rows, native, M, K, N, ep, stream);
             case 4: return launch<WM, WN, 4, Rows>(rows, native, M, K, N, ep, stream);
             default: return launch<WM, WN, 8, Rows>(rows, native, M, K, N, ep, stream);
         }
     };
-    if (bm == 64) return go(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
-    if (bn == 64) return go(std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{});
-    if (bm == 32) return go(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
+    if (tile.wm == 4) return go(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
+    if (tile.wn == 4) return go(std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{});
+    if (tile.wm == 2) return go(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
     return go(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{});
 }
 
+// Problems of ring.hip's that stay here: `ring` is the tile it would take. Its kernel starts sooner, this one runs faster once it
+// does (weights in registers, one 16-byte load for a whole block of them), so with the same tile and wavefronts a long reduction
+// is at home here. This kernel's time over ring.hip's (3700 shapes of rows, convolutions and fp32 row pairs):
+//   whole weight blocks, the same tile               rows 0.82 .. 0.98, convolutions 0.91 .. 0.98, pairs 0.93 .. 1.00
+//     32 x 32 tiles, another tile there              rows 0.91 .. 1.00, pairs from K = 4096 on 0.93 .. 0.96
+//     16 x 32 at K = 2048, another                   rows 0.94 .. 1.05 (0.99 on average)
+//     32 x 64 tiles in a convolution, another        0.93 .. 1.00 where they are filled (else to 1.4)
+//   single pairs, the same tile: 16 x 32, K >= 2048  rows 0.94 .. 1.04, convolutions 0.95 .. 1.01 (shorter: to 1.10)
+//     32 x 64, K >= 2560                             rows 0.95 .. 1.00, convolutions 0.94 .. 1.00 (shorter: to 1.08)
+//     64 x 64 in a convolution, K >= 2048            0.96 .. 1.00
+//   32 x 64 tiles of four wavefronts in two rounds, rows, K >= 704  0.91 .. 0.98 (shorter: 1.03 .. 1.11)
+// and everything else 0.95 to 1.6 (1.12 on average). 96 rows x 4096 -> 4096: 7.5 us here, 9.1 there.
+bool mid_holds(RingTile ring, int64_t M, int64_t K, int64_t N, bool conv, bool pairs) {
+    const MidTile t = mid_tile(M, K, N, conv);
+    if (t.wn == 8) return false;
+    const int64_t count = t.count(M, N);
+    const bool same = ring.wm == t.wm && ring.wn == t.wn && ring.waves == t.waves, filled = 5 * M * N >= 3 * count * 256 * t.wm * t.wn;
+    if (t.blocks && t.waves == 8) {
+        if (pairs) return t.wm == 2 && (t.wn == 4 ? same : K >= 4096);
+        return same || (t.wn == 2 ? !conv && (t.wm == 2 || K < 4096) : t.wm == 2 && conv && filled);
+    }
+    if (pairs) return false;
+    if (t.wm == 2 && t.wn == 4 && t.waves == 4) return !conv && K >= 704 && count > 256 && filled;
+    if (!same) return false;
+    return t.wm == 1 ? K >= 2048 : t.wm == 2 ? t.wn == 4 && K >= 2560 : conv && K >= 2048;
+}
+
+// The tile of ring.hip that takes a problem, or -1.
+int tile_of_ring(int64_t M, int64_t K, int64_t N, bool conv, bool pairs, const float *scale, const float *bias, const void *residual,
+                 const void *y) {
+    if (!ring_ok(M, K, N, scale, bias, residual, y)) return -1;
+    const int tile = ring_tile(M, K, N, conv);
+    return mid_holds(ring_tile_shape(tile), M, K, N, conv, pairs) ? -1 : tile;
+}
+
 }  // namespace
+
+// The same for 16-byte aligned operands.
+int split_reduction_tile(int64_t M, int64_t K, int64_t N, bool conv, bool pairs) {
+    return tile_of_ring(M, K, N, conv, pairs, nullptr, nullptr, nullptr, nullptr);
+}
 
 // True when the staged split-reduction kernel can take a dense fp16 problem.
 bool mid_dense_ok(const void *x, int64_t M, int64_t K) {
@@ -1078,8 +1128,8 @@ bool mid_dense_ok(const void *x, int64_t M, int64_t K) {
 
 int launch_mid_dense(const void *x, int64_t M, int64_t K, const void *native, int64_t N, const float *scale,
                      const float *bias, const void *residual, int relu, void *y, int y_f16, void *stream) {
-    if (ring_ok(M, K, N, scale, bias, residual, y))
-        return launch_ring_dense(x, M, K, native, N, scale, bias, residual, relu, y, y_f16, nullptr, stream);
+    const int tile = tile_of_ring(M, K, N, false, false, scale, bias, residual, y);
+    if (tile >= 0) return launch_ring_dense(tile, x, M, K, native, N, scale, bias, residual, relu, y, y_f16, nullptr, stream);
     MidEpilogue ep{scale, bias, residual, y, relu, y_f16};
     return dispatch(DenseRows{static_cast<const _Float16 *>(x), M, K}, native, M, K, N, ep, stream);
 }
@@ -1089,8 +1139,8 @@ int launch_mid_dense_pairs(const void *x16, int64_t M16, int64_t K, const void *
                            const float *bias, const void *residual, int relu, void *y, int y_f16, int64_t rows_out,
                            const float *group_scale, void *stream) {
     const PairMap map{rows_out, group_scale};
-    if (ring_ok(M16, K, N, scale, bias, residual, y))
-        return launch_ring_dense(x16, M16, K, native, N, scale, bias, residual, relu, y, y_f16, &map, stream);
+    const int tile = tile_of_ring(M16, K, N, false, true, scale, bias, residual, y);
+    if (tile >= 0) return launch_ring_dense(tile, x16, M16, K, native, N, scale, bias, residual, relu, y, y_f16, &map, stream);
     MidEpilogueT<PairMap> ep{scale, bias, residual, y, relu, y_f16, map};
     return dispatch(DenseRows{static_cast<const _Float16 *>(x16), M16, K}, native, M16, K, N, ep, stream);
 }
@@ -1164,8 +1214,8 @@ bool mid_conv_ok(const void *x, const tmq_conv_shape *s) {
 int launch_mid_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale,
                     const float *bias, const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream) {
     const int64_t M = (int64_t)s->B * ho * wo, K = (int64_t)s->C * s->ky * s->kx;
-    if (ring_ok(M, K, s->N, scale, bias, residual, y))
-        return launch_ring_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, map, stream);
+    const int tile = tile_of_ring(M, K, s->N, true, false, scale, bias, residual, y);
+    if (tile >= 0) return launch_ring_conv(tile, x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, map, stream);
     const ConvRows rows{static_cast<const _Float16 *>(x), M, K, s->B, s->C, s->H, s->W, ho, wo, s->ky, s->kx, s->sy,
                         s->sx, s->py, s->px, s->dy, s->dx, FastDiv((uint32_t)wo), FastDiv((uint32_t)ho),
                         FastDiv((uint32_t)s->C), FastDiv((uint32_t)s->kx)};

@@ -20,8 +20,6 @@
 
 namespace tmq {
 
-int ring_tile(int64_t M, int64_t K, int64_t N, bool conv);
-
 namespace {
 
 struct RingPlace {               // conv: geometry of the im2col view; dense: K alone
@@ -276,10 +274,7 @@ int launch(RingArgs<Map> a, void *stream) {
     return check_launch();
 }
 
-// The tiles on offer: fragments of 16 rows and of 16 columns, wavefronts, pairs in flight.
-struct RingTile {
-    int wm, wn, waves, depth;
-};
+// The tiles on offer.
 constexpr RingTile kRingTiles[] = {{1, 1, 4, 5}, {1, 1, 8, 4}, {1, 2, 4, 4}, {1, 2, 8, 4}, {2, 2, 4, 3}, {2, 2, 8, 2},
                                    {1, 4, 4, 4}, {2, 4, 8, 2}, {2, 4, 4, 3}, {4, 4, 4, 2}, {4, 4, 8, 2}};
 constexpr int kTiles = sizeof(kRingTiles) / sizeof(kRingTiles[0]);
@@ -316,8 +311,8 @@ int launch_tile(const RingArgs<Map> &a, void *stream) {
 }
 
 template <bool CONV, class Map>
-int by_cost(const RingArgs<Map> &a, void *stream) {
-    switch (ring_tile(a.M, a.K, a.N, CONV)) {
+int by_tile(const RingArgs<Map> &a, int tile, void *stream) {
+    switch (tile) {
         case 0: return launch_tile<CONV, 0>(a, stream);
         case 1: return launch_tile<CONV, 1>(a, stream);
         case 2: return launch_tile<CONV, 2>(a, stream);
@@ -358,9 +353,9 @@ RingArgs<Map> ring_args(const void *x, int64_t x_elements, int64_t M, int64_t K,
 
 }  // namespace
 
-// What of mid.hip's problems (K a multiple of 64, 16-byte aligned rows, fewer than 2^31 elements) comes here: results and
-// constants in whole quads, and reductions of up to 4608 indices -- with 192 64 x 64 tiles or more up to 3583, where mid.hip
-// fetches whole weight blocks. 1070 such shapes: 0.92 of mid.hip on average, 1.14 at most; beyond the lines 0.94, to 1.29.
+// What of mid.hip's problems (K a multiple of 64, 16-byte aligned rows, fewer than 2^31 elements) this kernel can take: results
+// and constants in whole quads, and reductions of up to 4608 indices -- with 192 64 x 64 tiles or more up to 3583, where mid.hip
+// fetches whole weight blocks (beyond these lines 0.94 of mid.hip on average, to 1.29). mid_holds (mid.hip) keeps the others.
 bool ring_ok(int64_t M, int64_t K, int64_t N, const float *scale, const float *bias, const void *residual, const void *y) {
     const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
     return K % 64 == 0 && K <= (tiles64 >= 192 ? 3583 : 4608) && N % 4 == 0 && N < (1 << 20) && M < (int64_t)0x7FFFFFFF && aligned16(y) &&
@@ -371,16 +366,17 @@ bool ring_ok(int64_t M, int64_t K, int64_t N, const float *scale, const float *b
 int ring_tile(int64_t M, int64_t K, int64_t N, bool conv) {
     return cheapest_tile(M, K / 64, N, conv, std::make_integer_sequence<int, kTiles>{});
 }
+RingTile ring_tile_shape(int tile) { return kRingTiles[tile]; }
 
-int launch_ring_dense(const void *x, int64_t M, int64_t K, const void *native, int64_t N, const float *scale, const float *bias,
+int launch_ring_dense(int tile, const void *x, int64_t M, int64_t K, const void *native, int64_t N, const float *scale, const float *bias,
                       const void *residual, int relu, void *y, int y_f16, const PairMap *pairs, void *stream) {
-    if (pairs) return by_cost<false>(ring_args(x, M * K, M, K, native, N, scale, bias, residual, relu, y, y_f16, *pairs), stream);
-    return by_cost<false>(ring_args(x, M * K, M, K, native, N, scale, bias, residual, relu, y, y_f16, NoMap{}), stream);
+    if (pairs) return by_tile<false>(ring_args(x, M * K, M, K, native, N, scale, bias, residual, relu, y, y_f16, *pairs), tile, stream);
+    return by_tile<false>(ring_args(x, M * K, M, K, native, N, scale, bias, residual, relu, y, y_f16, NoMap{}), tile, stream);
 }
 
 template <class Map>
-static int ring_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale, const float *bias,
-                     const void *residual, int relu, void *y, int y_f16, const Map &map, void *stream) {
+static int ring_conv(int tile, const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale,
+                     const float *bias, const void *residual, int relu, void *y, int y_f16, const Map &map, void *stream) {
     auto a = ring_args(x, (int64_t)s->B * s->H * s->W * s->C, (int64_t)s->B * ho * wo, (int64_t)s->C * s->ky * s->kx, native, s->N, scale, bias,
                        residual, relu, y, y_f16, map);
     a.at.H = s->H; a.at.W = s->W; a.at.C = s->C;
@@ -389,13 +385,13 @@ static int ring_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, con
     a.at.by_ho = FastDiv((uint32_t)ho);
     a.at.by_slabs = FastDiv((uint32_t)(s->C / 64));
     a.at.by_kx = FastDiv((uint32_t)s->kx);
-    return by_cost<true>(a, stream);
+    return by_tile<true>(a, tile, stream);
 }
 
-int launch_ring_conv(const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale, const float *bias,
-                     const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream) {
-    if (map) return ring_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, *map, stream);
-    return ring_conv(x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, NoMap{}, stream);
+int launch_ring_conv(int tile, const void *x, const tmq_conv_shape *s, int ho, int wo, const void *native, const float *scale,
+                     const float *bias, const void *residual, int relu, void *y, int y_f16, const RowMap *map, void *stream) {
+    if (map) return ring_conv(tile, x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, *map, stream);
+    return ring_conv(tile, x, s, ho, wo, native, scale, bias, residual, relu, y, y_f16, NoMap{}, stream);
 }
 
 }  // namespace tmq
