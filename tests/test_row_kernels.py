@@ -34,3 +34,12 @@ def test_long_reductions_on_the_same_tile_stay_with_mid():
     # fp32 row pairs: only whole weight blocks
     assert kernel(_capi.F32, 60, 3584, 4096) >= RING and kernel(_capi.F32, 64, 4096, 4096) == SPLIT
     assert kernel(_capi.F16, 16, 64, 64) < 0
+
+
+def test_16_x_64_tiles_of_medium_reductions_are_not_taken():
+    """(their cost is fitted too low there: 80 rows, 1792 -> 8192 9.5 us on them, 8.1 on 64 x 64)"""
+    from tmq_amd import _capi
+    kernel = _capi.load().tmq_ternary_rows_kernel
+    for K in (1280, 1536, 1792):
+        for M, N in ((80, 8192), (64, 11008), (256, 3072)):
+            assert kernel(_capi.F16, M, K, N) != 16 + 6
