@@ -43,3 +43,19 @@ def test_refuses_what_the_convolution_refuses():
     assert kernel_of(1, 64, 3, 3, 64, (5, 5), 0) == -1 and kernel_of(1, 64, 0, 3, 64, (1, 1), 0) == -1
     assert _capi.load().tmq_ternary_conv2d_kernel(None, _capi.F32) == -1
     assert kernel_of(0, 64, 8, 8, 64, (3, 3), 1) >= 0          # an empty batch is nothing to launch
+
+
+def test_fp32_opening_leaves_many_patches_to_the_conversion():
+    """Refused before anything is launched (the pointers here are no memory)."""
+    import torch
+    from tmq_amd import _capi
+    if torch.cuda.is_available():
+        pytest.skip("made-up pointers")
+    at = lambda n: ctypes.c_void_p(4096 * n)
+    def refused(planes, sy, B, size):
+        # a 7 x 7 opening of horizontal stride 2 over super-pixels
+        shape = _capi.ConvShape(B, 8, size, size // 2, 64, 7, 4, sy, 1, 3, 2, 1, 1, 3, 1)
+        return _capi.load().tmq_ternary_conv2d_relu_maxpool_planar_f32(at(1), planes, ctypes.byref(shape), at(2), at(3), at(4), at(5), at(6),
+                                                                       None) == _capi.ERR_UNSUPPORTED
+    # 224 x 224: 8 x 7 patches an image at vertical stride 2, 16 x 7 at 1
+    assert refused(1, 2, 110, 224) and refused(1, 1, 55, 224) and refused(2, 1, 55, 224) and refused(4, 1, 37, 224)

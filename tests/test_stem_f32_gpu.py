@@ -74,3 +74,25 @@ def test_fp32_opening_in_a_graph(cuda):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, call())
+
+
+# more patches than the fp32 form takes: converted first, the same bits
+@pytest.mark.parametrize("planes,stride,B", [(1, (2, 2), 80), (2, (1, 2), 40), (4, (1, 2), 27)])
+def test_many_patches_are_converted_first(cuda, planes, stride, B):
+    import tmq_amd as t
+    from tmq_amd import ops
+    torch.manual_seed(planes)
+    net = torch.nn.Sequential(torch.nn.Conv2d(planes, 8, 3, stride, 1, bias=False))
+    ctrl = t.QuantizationControl()
+    t.quantize_model(net, ctrl)
+    net.to(cuda).eval()
+    ctrl.quantize()
+    t.compressed_state_dict(net, strong=False)
+    x = torch.randn((B, planes, 256, 304), device=cuda) * 1e5
+    nw, kxs, pl, pr = net[0]._superpixel_plan(x)
+    form = ((stride[0], 1), ((1, 1), (pl, pr)), 1)
+    h, adjusted = ops.f32_to_f16_prescaled(x, None, 8)
+    want = ops.ternary_conv2d_relu_maxpool_planar(h, nw, *form, adjusted)
+    got = ops.ternary_conv2d_relu_maxpool_planar(x, nw, *form, prescale=True)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    assert torch.equal(net[0].compact_forward(x, pool=True).view(torch.int16), want.view(torch.int16))

@@ -353,6 +353,12 @@ int launch_opening(const void *x, const float *xf, int32_t planes, const tmq_con
     if (tiles == 0) return TMQ_OK;
     p.const_off = (int)(lds_window > tile_bytes ? lds_window : tile_bytes);
     const size_t lds = (size_t)p.const_off + 128 * 4;
+    // Many patches of fp32 planes, where a conversion in front is the faster one: a workgroup waits for its gathers, which the
+    // fp16 form has half of, and the more images follow each other the less a launch weighs. 64 channels, time of this form
+    // over the two launches (windows 3 x 2 to 7 x 4, 3000 to 40000 patches): vertical stride 2, one plane 0.89 .. 1.00 up to
+    // 8000 patches and 1.00 .. 1.08 beyond, two to four 0.88 .. 1.02; stride 1, one or two planes 0.91 .. 0.98 up to 5000 and
+    // 0.99 .. 1.14 from 7000 on, three 0.94 .. 1.03, four 0.94 .. 1.01 up to 3600 and 1.02 .. 1.16 from 4500 on.
+    if (xf && (s->sy > 1 ? planes == 1 : planes != 3) && tiles > (s->sy == 1 && planes == 4 ? 4096 : 6144)) return TMQ_ERR_UNSUPPORTED;
     if (xf) {
         p.xf = xf;
         p.partials = static_cast<const float *>(workspace);

@@ -956,8 +956,9 @@ def ternary_conv2d_relu_maxpool_planar(x: torch.Tensor, nw: NativeWeights, strid
             status = lib.tmq_ternary_conv2d_relu_maxpool_planar(ptr(x), C, ctypes.byref(shp), ptr(nw.buf), ep.scale, ep.bias,
                                                                 ptr(y), stream_of(x))
     if status == _capi.ERR_UNSUPPORTED:
-        if x.dtype == torch.float32:
+        if x.dtype == torch.float32:      # (for many patches of some numbers of planes that is the faster way)
             x, scale = f32_to_f16_prescaled(x, scale, nw.N)
+            return ternary_conv2d_relu_maxpool_planar(x, nw, stride, padding, dilation, scale, bias)
         return two_step()
     check(status, "ternary_conv2d_relu_maxpool_planar")
     return y
