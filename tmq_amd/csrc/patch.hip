@@ -15,7 +15,7 @@
 //   * Everybody fetches, multiplies and stores at the same time, so a second round would add both ends again: worth it for one
 //     round that fills the chip. Clock stamps for 256 -> 256 on 14 x 14, batch 64, us: patch in LDS at 3.3, products 11.0 (1.87
 //     GHz, MFMAs 80 % of the time), sums and stores 3.4.
-// Batch 64, 3 x 3, us: 256 -> 256 on 14 x 14 20.2 -> 17.7; 512 -> 512 on 7 x 7 25.0 -> 19.8.
+// Batch 64, 3 x 3, us: 256 -> 256 on 14 x 14 20.1 -> 17.8; 512 -> 512 on 7 x 7 23.1 -> 18.6 (25.0 -> 19.8 on another machine).
 #include "common.h"
 #include "mfma.h"
 #include "tile_epilogue.h"

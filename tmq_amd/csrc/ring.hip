@@ -11,9 +11,10 @@
 //   * Constants, residual and destinations are asked for between the first loads and the first wait, and the barriers of the
 //     sum wait for LDS only: stores and residuals are nobody's business there.
 // What bounds the longer reductions is the CU's vector-memory pipe (16 clocks an instruction, 2 WM + WN a pair): deeper rings
-// do not help (512 -> 512 on one 7 x 7 image: 5.8 us with four slots, 6.2 with eight), smaller tiles on more CUs do.
-// Against mid.hip, us: 64 -> 128, 1 x 1 / 2 on 56 x 56, batch 4 4.65 -> 3.5; 256 -> 512, 1 x 1 / 2 on 14 x 14, batch 16 5.6 -> 3.7;
-// 64 -> 64, 3 x 3 on one 56 x 56 image 4.5 -> 4.1; 128 rows x 400 -> 1024 5.2 -> 3.9; 333 fp32 rows, 2000 -> 1000 10.8 -> 9.7.
+// do not help (512 -> 512 on one 7 x 7 image: eight slots 7 % slower than four), smaller tiles on more CUs do.
+// Against mid.hip, through the public calls, us: 256 -> 512, 1 x 1 / 2 on 14 x 14, batch 16 5.5 -> 3.6; 128 -> 256, 1 x 1 / 2 on
+// 28 x 28, batch 4 4.7 -> 3.1; 64 -> 64, 3 x 3 on one 56 x 56 image 4.3 -> 3.7; 512 -> 512, 3 x 3 on one 7 x 7 5.8 -> 5.3; 128 rows,
+// 448 -> 1024 3.2 -> 2.8; 333 fp32 rows, 2000 -> 1000, with their split 15.2 -> 14.3.
 #include "common.h"
 #include "mfma.h"
 #include <utility>

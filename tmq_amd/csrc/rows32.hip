@@ -10,8 +10,8 @@
 //     position (j + c) % 16 of 256 bytes: both the writers, on neighbouring chunks, and the readers, on neighbouring
 //     columns, meet every bank.
 //   * Bound by the chain argument fetch -> rows -> maximum -> LDS -> product -> sum, about 2 us behind a launch's 1.6;
-//     neither memory nor the matrix pipe is busy. 5 rows, 1000 -> 3000: 6.3 us in two launches
-//     before, 4.0 so; 16 rows 9.7 in three, 5.1.
+//     neither memory nor the matrix pipe is busy. 5 rows, 1000 -> 3000: 6.1 us in two launches
+//     before, 3.7 so; 16 rows 9.6 in three, 4.8.
 #include "common.h"
 #include "mfma.h"
 #include "range.h"
@@ -263,9 +263,9 @@ int by_width(const Rows32 &a, void *stream) {
 
 // Which rows are split in the launch that multiplies them. The terms of the rows have to fit LDS (32 bytes an index, 64 from
 // nine rows on), and every workgroup prepares them again, which wide layers over long rows pay for: against the split in a
-// launch of its own, 600 shapes, 0.85 of its time at the median of 1 .. 8 rows and 0.5 of 9 .. 16 inside these lines (1.07 at
-// most), 1.08 .. 1.65 beyond (2304 x 25768, 6 rows 10.6 -> 14.0 us). 16 rows x 512 -> 512: 9.1 -> 3.9 us; 8 rows x 2048 -> 2048
-// 6.9 -> 5.0; 3 rows x 4096 -> 4096 7.5 -> 6.7. So do the widest layers over rows of any length, from the second round of
+// launch of its own, 600 shapes, 0.85 of its time at the median of 1 .. 8 rows and 0.5 of 9 .. 16 inside these lines (1.04 at
+// most), 1.08 .. 1.65 beyond (2304 x 25768, 6 rows 10.6 -> 14.0 us). 16 rows x 512 -> 512: 9.2 -> 3.5 us; 8 rows x 2048 -> 2048
+// 6.5 -> 4.6; 3 rows x 4096 -> 4096 7.2 -> 6.3. So do the widest layers over rows of any length, from the second round of
 // workgroups on (their sums leave room for one a CU; 360 shapes of 12000 columns and more): up to 32768 columns 0.42 .. 0.90 for
 // 9 .. 16 rows, beyond 0.81 .. 0.95 for up to 12 short ones to 65536 and 0.93 .. 1.36 for the others (16 rows x 40 -> 338116
 // 65.6 -> 84.4); 5 .. 8 rows 0.50 .. 0.99 to 131072 columns and to 32768 for more than 512 values, 0.79 .. 1.05 from there on;
