@@ -529,14 +529,15 @@ int tmq_ternary_conv2d_relu_maxpool(const void *x, const tmq_conv_shape *shape, 
 int tmq_ternary_conv2d_relu_maxpool_planar(const void *x, int32_t planes, const tmq_conv_shape *shape, const void *native,
                                            const float *scale, const float *bias, void *y, void *stream);
 
-/* ... and from an fp32 image: x is NCHW fp32 (8-byte aligned; TMQ_ERR_UNSUPPORTED otherwise, and for so many patches of 7 x 8
- * pooled positions that a conversion in front is faster: 6144 of one plane, with a vertical stride of 1 also of two planes and
- * 4096 of four). Same result bit for bit as
+/* ... and from an fp32 image: x is NCHW fp32 (8-byte aligned, else TMQ_ERR_UNSUPPORTED). Same result bit for bit as
  * tmq_f32_to_f16_prescaled on the whole input followed by that call with the adjusted scale, without the fp16 copy:
  * the scan for the largest |x| (partial maxima in `workspace`, tmq_f32_to_f16_prescaled_workspace_bytes of the input's
  * element count) and the opening, which scales and rounds what it reads.                              */
 int tmq_ternary_conv2d_relu_maxpool_planar_f32(const float *x, int32_t planes, const tmq_conv_shape *shape, const void *native,
                                                const float *scale, const float *bias, void *y, void *workspace, void *stream);
+/* 1 where that is the faster of the two ways (host only; 0: many patches of one plane, or of two or four at a vertical stride
+ * of 1, and shapes without an output). */
+int tmq_ternary_conv2d_relu_maxpool_planar_f32_pays(int32_t planes, const tmq_conv_shape *shape);
 
 /* Global average pool: x [B][HW][C] fp16 -> y [B][C] (TMQ_F16 or TMQ_F32), fp32 accumulation.    */
 int tmq_avgpool_global_nhwc(const void *x, int64_t B, int64_t HW, int64_t C, void *y, int y_dtype,

@@ -46,16 +46,15 @@ def test_refuses_what_the_convolution_refuses():
 
 
 def test_fp32_opening_leaves_many_patches_to_the_conversion():
-    """Refused before anything is launched (the pointers here are no memory)."""
-    import torch
     from tmq_amd import _capi
-    if torch.cuda.is_available():
-        pytest.skip("made-up pointers")
-    at = lambda n: ctypes.c_void_p(4096 * n)
-    def refused(planes, sy, B, size):
-        # a 7 x 7 opening of horizontal stride 2 over super-pixels
+
+    def pays(planes, sy, B, size=224):
+        # a 7 x 7 opening of horizontal stride 2 over super-pixels: 8 x 7 patches a 224 x 224 image at vertical stride 2, 16 x 7 at 1
         shape = _capi.ConvShape(B, 8, size, size // 2, 64, 7, 4, sy, 1, 3, 2, 1, 1, 3, 1)
-        return _capi.load().tmq_ternary_conv2d_relu_maxpool_planar_f32(at(1), planes, ctypes.byref(shape), at(2), at(3), at(4), at(5), at(6),
-                                                                       None) == _capi.ERR_UNSUPPORTED
-    # 224 x 224: 8 x 7 patches an image at vertical stride 2, 16 x 7 at 1
-    assert refused(1, 2, 110, 224) and refused(1, 1, 55, 224) and refused(2, 1, 55, 224) and refused(4, 1, 37, 224)
+        return _capi.load().tmq_ternary_conv2d_relu_maxpool_planar_f32_pays(planes, ctypes.byref(shape))
+    assert [pays(1, 2, B) for B in (109, 110)] == [1, 0]
+    for planes in (1, 2):
+        assert [pays(planes, 1, B) for B in (54, 55)] == [1, 0]
+    assert [pays(4, 1, B) for B in (36, 37)] == [1, 0]
+    assert pays(3, 1, 1000) == 1 and all(pays(planes, 2, 1000) for planes in (2, 3, 4))
+    assert pays(3, 2, 1, 0) == 0 and pays(5, 2, 1) == 0 and pays(0, 2, 1) == 0

@@ -76,7 +76,7 @@ def test_fp32_opening_in_a_graph(cuda):
         assert torch.equal(y, call())
 
 
-# more patches than the fp32 form takes: converted first, the same bits
+# more patches than the fp32 form is taken for: converted first, the same bits
 @pytest.mark.parametrize("planes,stride,B", [(1, (2, 2), 80), (2, (1, 2), 40), (4, (1, 2), 27)])
 def test_many_patches_are_converted_first(cuda, planes, stride, B):
     import tmq_amd as t

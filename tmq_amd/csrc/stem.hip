@@ -353,12 +353,6 @@ int launch_opening(const void *x, const float *xf, int32_t planes, const tmq_con
     if (tiles == 0) return TMQ_OK;
     p.const_off = (int)(lds_window > tile_bytes ? lds_window : tile_bytes);
     const size_t lds = (size_t)p.const_off + 128 * 4;
-    // Many patches of fp32 planes, where a conversion in front is the faster one: a workgroup waits for its gathers, which the
-    // fp16 form has half of, and the more images follow each other the less a launch weighs. 64 channels, time of this form
-    // over the two launches (windows 3 x 2 to 7 x 4, 3000 to 40000 patches): vertical stride 2, one plane 0.89 .. 1.00 up to
-    // 8000 patches and 1.00 .. 1.08 beyond, two to four 0.88 .. 1.02; stride 1, one or two planes 0.91 .. 0.98 up to 5000 and
-    // 0.99 .. 1.14 from 7000 on, three 0.94 .. 1.03, four 0.94 .. 1.01 up to 3600 and 1.02 .. 1.16 from 4500 on.
-    if (xf && (s->sy > 1 ? planes == 1 : planes != 3) && tiles > (s->sy == 1 && planes == 4 ? 4096 : 6144)) return TMQ_ERR_UNSUPPORTED;
     if (xf) {
         p.xf = xf;
         p.partials = static_cast<const float *>(workspace);
@@ -385,6 +379,19 @@ int tmq_ternary_conv2d_relu_maxpool(const void *x, const tmq_conv_shape *s, cons
 int tmq_ternary_conv2d_relu_maxpool_planar(const void *x, int32_t planes, const tmq_conv_shape *s, const void *native,
                                            const float *scale, const float *bias, void *y, void *stream) {
     return launch_opening(x, nullptr, planes, s, native, scale, bias, y, nullptr, stream);
+}
+
+// Many patches of fp32 planes, where a conversion in front is the faster one: a workgroup waits for its gathers, which the
+// fp16 form has half of, and the more images follow each other the less a launch weighs. 64 channels, time of this form
+// over the two launches (windows 3 x 2 to 7 x 4, 3000 to 40000 patches of 7 x 8 pooled positions): vertical stride 2, one plane
+// 0.89 .. 1.00 up to 8000 patches and 1.00 .. 1.08 beyond, two to four 0.88 .. 1.02; stride 1, one or two planes 0.91 .. 0.98 up
+// to 5000 and 0.99 .. 1.14 from 7000 on, three 0.94 .. 1.03, four 0.94 .. 1.01 up to 3600 and 1.02 .. 1.16 from 4500 on.
+int tmq_ternary_conv2d_relu_maxpool_planar_f32_pays(int32_t planes, const tmq_conv_shape *s) {
+    int32_t ho, wo;
+    if (!s || planes < 1 || planes > 4 || tmq_conv2d_out_hw(s, &ho, &wo) != TMQ_OK || ho <= 0 || wo <= 0) return 0;
+    if (s->sy > 1 ? planes > 1 : planes == 3) return 1;
+    const int64_t high = ((ho - 1) / 2 + 7) / 7, wide = ((wo - 1) / 2 + kPoolW) / kPoolW;      // 7 pooled rows a patch, 8 columns
+    return s->B * high * wide <= (s->sy == 1 && planes == 4 ? 4096 : 6144) ? 1 : 0;
 }
 
 int tmq_ternary_conv2d_relu_maxpool_planar_f32(const float *x, int32_t planes, const tmq_conv_shape *s, const void *native,

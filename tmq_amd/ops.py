@@ -942,6 +942,8 @@ def ternary_conv2d_relu_maxpool_planar(x: torch.Tensor, nw: NativeWeights, strid
     check(lib.tmq_conv2d_out_hw(ctypes.byref(shp), ctypes.byref(ho), ctypes.byref(wo)), "conv2d_out_hw")
     if ho.value <= 0 or wo.value <= 0:
         raise RuntimeError("ternary_conv2d_relu_maxpool_planar: empty output")
+    if x.dtype == torch.float32 and not lib.tmq_ternary_conv2d_relu_maxpool_planar_f32_pays(C, ctypes.byref(shp)):
+        x, scale = f32_to_f16_prescaled(x, scale, nw.N)
     y = torch.empty((B, nw.N, (ho.value - 1) // 2 + 1, (wo.value - 1) // 2 + 1), dtype=torch.float16, device=x.device,
                     memory_format=torch.channels_last)
     ep = _epilogue(nw, scale, bias, None, True, torch.float16, y)     # validates scale and bias
@@ -956,9 +958,8 @@ def ternary_conv2d_relu_maxpool_planar(x: torch.Tensor, nw: NativeWeights, strid
             status = lib.tmq_ternary_conv2d_relu_maxpool_planar(ptr(x), C, ctypes.byref(shp), ptr(nw.buf), ep.scale, ep.bias,
                                                                 ptr(y), stream_of(x))
     if status == _capi.ERR_UNSUPPORTED:
-        if x.dtype == torch.float32:      # (for many patches of some numbers of planes that is the faster way)
+        if x.dtype == torch.float32:
             x, scale = f32_to_f16_prescaled(x, scale, nw.N)
-            return ternary_conv2d_relu_maxpool_planar(x, nw, stride, padding, dilation, scale, bias)
         return two_step()
     check(status, "ternary_conv2d_relu_maxpool_planar")
     return y
