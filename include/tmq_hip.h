@@ -346,11 +346,12 @@ int tmq_fp32_rows_self_scaled(const void *x, int64_t M, int64_t K);
  * 6144 and N <= 6144 (each row scaled by its own power of two inside the one launch). */
 int tmq_fp32_rows_self_scaled_for(const void *x, int64_t M, int64_t K, int64_t N);
 /* 1 when tmq_ternary_linear(x, TMQ_F32, M, K, ...) takes these 16-byte aligned rows in one launch whatever their
- * magnitude: the rows of tmq_fp32_rows_self_scaled_for, and up to sixteen short ones (1 .. 8 rows of up to 2048 values
- * against up to 3 2^23 weights, of up to 4096 values against up to 4096 channels, from five rows on up to 131072 channels
- * (32768 for more than 512 values), from three on 16384 for more than 1024;
- * 9 .. 16 of up to 2048 against up to 2^25 weights and 32768 channels, up to 12 of up to 512 against 65536), each scaled by
- * its own power of two and split into two fp16 terms by the workgroups that multiply it. A workspace is not used. */
+ * magnitude and a workspace would not make it faster: the rows of tmq_fp32_rows_self_scaled_for, and up to sixteen short ones
+ * (1 .. 8 rows of up to 2048 values against up to 3 2^23 weights, of up to 4096 values against up to 4096 channels; 9 .. 16 of
+ * up to 2048 against up to 2^25 weights), each scaled by its own power of two and split into two fp16 terms by the workgroups
+ * that multiply it. 0, though tmq_ternary_linear takes them so, for the widest layers: from five rows on beyond 131072 channels
+ * (32768 for more than 512 values), from three beyond 16384 for more than 1024, from nine beyond 32768 (up to twelve of up to
+ * 512 values: 65536). */
 int tmq_fp32_rows_one_launch(const void *x, int64_t M, int64_t K, int64_t N);
 
 /* Which kernel multiplies 17 rows or more behind tmq_ternary_linear_ws, given its workspace and 16-byte aligned operands: for

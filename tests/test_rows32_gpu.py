@@ -85,3 +85,25 @@ def test_infinities_and_nan_stay_in_their_row(cuda, oracle, M):
     keep = [m for m in range(M) if m not in (1, 3)]
     assert torch.equal(y[keep], clean[keep])
     assert torch.isnan(y[1]).all() and not torch.isfinite(y[3]).any()
+
+
+@pytest.mark.parametrize("M,K,N", [(16, 40, 33000), (4, 1100, 17000)])
+def test_widest_layers_without_a_workspace_take_rows_of_any_magnitude(cuda, oracle, M, K, N):
+    """tmq_fp32_rows_one_launch prefers the workspace there; the call without one still scales the rows itself."""
+    from tmq_amd import ops, _capi
+    lib = _capi.load()
+    rng = np.random.default_rng(M)
+    W = rng.integers(-1, 2, size=(N, K)).astype(np.float32)
+    nw = ops.NativeWeights(torch.from_numpy(oracle.pack(W).view(np.int32)).to(cuda), N)
+    x = rng.standard_normal((M, K)).astype(np.float32) * np.float32(10.0) ** rng.integers(-30, 30, size=(M, 1)).astype(np.float32)
+    tx = torch.from_numpy(x).to(cuda)
+    assert lib.tmq_fp32_rows_one_launch(ops.ptr(tx), M, K, N) == 0
+    want = x.astype(np.float64) @ W.astype(np.float64).T
+    bound = np.abs(x.astype(np.float64)).sum(1, keepdims=True) * (2.0 ** -22 + (2 * -(-K // 512) + 8 + 2 + 33) * 2.0 ** -24)
+    y = torch.full((M, N), float("nan"), device=cuda)
+    assert lib.tmq_ternary_linear(ops.ptr(tx), _capi.F32, M, K, ops.ptr(nw.buf), N, None, ops.ptr(y), None) == 0
+    torch.cuda.synchronize()
+    assert np.all(np.abs(y.cpu().numpy() - want) <= bound + 1e-45)
+    # with the workspace: the rows' own powers of two as well, 22 bits a value, sums over up to K / 32 products
+    z = ops.ternary_linear(tx, nw)
+    assert np.all(np.abs(z.cpu().numpy() - want) <= 2 * bound + 1e-45)

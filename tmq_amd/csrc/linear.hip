@@ -42,6 +42,7 @@ int launch_gemv8_planes(const void *planes, int64_t M, int64_t K, const void *na
 int launch_gemv8_prepare(const void *x, int64_t M, int64_t K, void *planes, void *stream);
 // rows32.hip: up to sixteen short fp32 rows, split inside the launch
 bool rows32_ok(const void *x, int64_t M, int64_t K, int64_t N);
+bool rows32_pays(const void *x, int64_t M, int64_t K, int64_t N);
 int launch_rows32(const void *x, int64_t M, int64_t K, const void *native, int64_t N, const float *scale, const float *bias,
                   const void *residual, int relu, void *y, int y_f16, void *stream);
 bool gemv8_dense32_ok(const void *x, int64_t M, int64_t K, int64_t N);
@@ -1104,7 +1105,7 @@ int tmq_fp32_rows_self_scaled_for(const void *x, int64_t M, int64_t K, int64_t N
 }
 
 int tmq_fp32_rows_one_launch(const void *x, int64_t M, int64_t K, int64_t N) {
-    return gemv8_dense32_ok(x, M, K, N) || rows32_ok(x, M, K, N) ? 1 : 0;
+    return gemv8_dense32_ok(x, M, K, N) || rows32_pays(x, M, K, N) ? 1 : 0;
 }
 
 int tmq_fp32_rows_prefer_split(int64_t M, int64_t K, int64_t N) {
@@ -1175,7 +1176,8 @@ int tmq_ternary_linear(const void *x, int x_dtype, int64_t M, int64_t K, const v
     // ... and one fp32 row (the reference's GEMV convention) up to K = 16384, two over small layers: the same kernel on the rows' two fp16 halves
     if (x32 && gemv8_dense32_ok(x, M, K, N))
         return launch_gemv8_dense32(x, M, K, native, N, ep.scale, ep.bias, ep.residual, ep.relu, y, ep.y_dtype == TMQ_F16, stream);
-    // ... and up to sixteen short fp32 rows, scaled and split by the workgroups that multiply them (rows32.hip)
+    // ... and up to sixteen short fp32 rows, scaled and split by the workgroups that multiply them (rows32.hip; with a workspace
+    // the widest layers split them in a launch of its own, tmq_ternary_linear_ws)
     if (x32 && rows32_ok(x, M, K, N))
         return launch_rows32(x, M, K, native, N, ep.scale, ep.bias, ep.residual, ep.relu, y, ep.y_dtype == TMQ_F16, stream);
     // At most 16 fp16 rows against eight or more weight blocks per channel: the weight-stream kernel (mid.hip).

@@ -261,20 +261,27 @@ int by_width(const Rows32 &a, void *stream) {
 
 }  // namespace
 
-// Which rows are split in the launch that multiplies them. The terms of the rows have to fit LDS (32 bytes an index, 64 from
+// Which rows the launch that multiplies them can split. The terms of the rows have to fit LDS (32 bytes an index, 64 from
 // nine rows on), and every workgroup prepares them again, which wide layers over long rows pay for: against the split in a
-// launch of its own, 600 shapes, 0.85 of its time at the median of 1 .. 8 rows and 0.5 of 9 .. 16 inside these lines (1.04 at
-// most), 1.08 .. 1.65 beyond (2304 x 25768, 6 rows 10.6 -> 14.0 us). 16 rows x 512 -> 512: 9.2 -> 3.5 us; 8 rows x 2048 -> 2048
-// 6.5 -> 4.6; 3 rows x 4096 -> 4096 7.2 -> 6.3. So do the widest layers over rows of any length, from the second round of
-// workgroups on (their sums leave room for one a CU; 360 shapes of 12000 columns and more): up to 32768 columns 0.42 .. 0.90 for
-// 9 .. 16 rows, beyond 0.81 .. 0.95 for up to 12 short ones to 65536 and 0.93 .. 1.36 for the others (16 rows x 40 -> 338116
-// 65.6 -> 84.4); 5 .. 8 rows 0.50 .. 0.99 to 131072 columns and to 32768 for more than 512 values, 0.79 .. 1.05 from there on;
-// fewer rows 0.40 .. 0.85 at any width. More than 1024 values against more than 16384 columns 1.04 .. 1.12 from three rows on.
+// launch of its own, 600 shapes, 0.85 of its time at the median of 1 .. 8 rows and 0.5 of 9 .. 16 inside these lines, 1.08 .. 1.65
+// beyond (2304 x 25768, 6 rows 10.6 -> 14.0 us). 16 rows x 512 -> 512: 9.2 -> 3.5 us; 8 rows x 2048 -> 2048 6.5 -> 4.6; 3 rows x
+// 4096 -> 4096 7.2 -> 6.3.
 bool rows32_ok(const void *x, int64_t M, int64_t K, int64_t N) {
     if (M < 1 || M > 16 || K < 1 || N < 1 || !aligned16(x)) return false;
-    if (M > 8) return K <= 2048 && K * N <= (int64_t)1 << 25 && (N <= 32768 || (M <= 12 && N <= 65536 && K <= 512));
-    if ((M > 4 && N > (K > 512 ? 32768 : 131072)) || (M > 2 && K > 1024 && N > 16384)) return false;
+    if (M > 8) return K <= 2048 && K * N <= (int64_t)1 << 25;
     return K <= 2048 ? K * N <= (int64_t)3 << 23 : K <= 4096 && N <= 4096;
+}
+
+// Where that is also the faster way for a caller with a workspace. The widest layers pay for the repeated preparation with rows
+// of any length, from the second round of workgroups on (their sums leave room for one a CU). Against the split of its own, 360
+// shapes of 12000 columns and more: up to 32768 columns 0.42 .. 0.90 for 9 .. 16 rows, beyond 0.81 .. 0.95 for up to 12 short ones
+// to 65536 and 0.93 .. 1.36 for the others (16 rows x 40 -> 338116 65.6 -> 84.4 us); 5 .. 8 rows 0.50 .. 0.99 to 131072 columns and
+// to 32768 for more than 512 values, 0.79 .. 1.05 from there on; fewer rows 0.40 .. 0.85 at any width. More than 1024 values
+// against more than 16384 columns 1.04 .. 1.12 from three rows on. (Inside all lines 1.03 at most.)
+bool rows32_pays(const void *x, int64_t M, int64_t K, int64_t N) {
+    if (!rows32_ok(x, M, K, N)) return false;
+    if (M > 8) return N <= 32768 || (M <= 12 && N <= 65536 && K <= 512);
+    return !((M > 4 && N > (K > 512 ? 32768 : 131072)) || (M > 2 && K > 1024 && N > 16384));
 }
 
 int launch_rows32(const void *x, int64_t M, int64_t K, const void *native, int64_t N, const float *scale, const float *bias,
